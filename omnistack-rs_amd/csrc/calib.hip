@@ -11,48 +11,76 @@
 //          max_iters or when the largest fp32 move |c_new - c_old| < tol
 //          (the moved centroids are kept);
 //   result sorted ascending.
-// The sort is replaced by four radix-select passes (8 bits each, all 16
-// order statistics x_(r*bs - 1) at once) and one pass that sums the samples
-// below each of them: bin r's sum is F(r bs) - F((r-1) bs) with
-// F(m) = sum(x < v) + v (m - #(x < v)) for v the m-th smallest sample.
-// Sums are accumulated in fp64 per thread, then over threads and blocks in a
-// fixed order, so results are deterministic; means are rounded to fp32 once.
-// (The reference's fp32 `mean()` rounds along the way: its last bits can
-// differ, and so can a convergence decision taken at the tolerance.)
-// Samples must be finite.
+//
+// A Lloyd step needs no pass over the samples.  They are counted and stored
+// once by bins of their order-preserving key: a bin is one exponent (of one
+// sign) or a power-of-two part of it, as fine as its share of the samples
+// asks for (up to 512 a bin on average).  One exponent per bin makes the fp64 sum of up
+// to 2^29 of its samples exact in any order.  Under sorted centroids the
+// codes ascend with x, so cell k is a run of whole bins between two boundary
+// bins plus a part of each: per boundary the largest fp32 value that still
+// takes the lower code is found with the fp32 distances themselves, and only
+// that bin's samples are compared with it.  One block per group runs the
+// initial bins and every step in one launch, a wave per boundary; the bins'
+// places stay in LDS, the boundary bin's samples in registers, so a step
+// waits for memory once, and only where a boundary has moved to another bin.
+// 8 groups x 1.64 M fp32 samples, 300 steps (a pass over all samples and an
+// update launch per step before): 17.7 ms -> 1.2 ms (0.93 ms of it the steps).
+//
+// Results are deterministic: sums inside a bin are exact, sums over bins are
+// formed in fp64 in a fixed order, means are rounded to fp32 once.  (The
+// reference's fp32 `mean()` rounds along the way: its last bits can differ,
+// and so can a convergence decision taken at the tolerance.)  Where two
+// distances of one sample can round to a tie with a lower index (centroids
+// closer than 2^-22 of the distances compared) the step goes over the
+// samples one by one instead.  Samples must be finite.
 //
 // Layout: group g's samples are rows of `inner` contiguous elements:
 // element e of group g is x[(e / inner) * outer_stride + g * group_stride +
 // e % inner], e < outer * inner.  A flat vector is outer = 1; head h of a
 // (B, H, T, D) cache is outer = B, inner = T*D, outer_stride = H*T*D,
 // group_stride = T*D.
+#include <float.h>
 #include <math.h>
 
 #include "omni_common.h"
 
 namespace omni {
 
-constexpr int kLmK = 16;            // centroids
-constexpr int kLmThreads = 256;
-constexpr int kLmMaxBlocks = 240;   // blocks per group (grid-stride)
-constexpr int kLmIntervals = kLmK + 1;
+constexpr int kLmK = 16;                    // centroids
+constexpr int kLmThreads = 1024;
+constexpr int kLmPer = 32;                  // samples per thread of the counting and storing passes
+constexpr int kLmBlock = kLmThreads * kLmPer;
+constexpr int kLmOct = 512;                 // sign and exponent
+constexpr int kLmMaxBins = 32768;           // bins per group at most (their places fit LDS)
+// Samples per bin aimed at, where that keeps the bins within kLmMaxBins.
+// Finer bins cost the passes that fill them more than they save the steps:
+// count, store, bin sums and steps took 72 + 174 + 49 + 955 us at 64 samples,
+// 31 + 154 + 28 + 920 at 256 and 26 + 148 + 24 + 927 at 512 (8 x 1.64 M).
+constexpr int kLmFill = 512;
+constexpr int kLmCache = 32;                // samples per lane a boundary bin may hold in registers
+constexpr int kLmSlowSlots = 256;
 
 struct LmArgs {
     const void *x;
     int64_t outer, inner, outer_stride, group_stride, n, bs;
-    int blocks;
     int max_iters;
     float tol;
+    int nb, nch;            // bins (the last ones may be unused) and 64-bin chunks
+    int64_t fill;           // samples per bin aimed at
+    int mant;               // mantissa bits of the sample type
+    int vec, wide;          // 4-element loads; n >= 2^32: cursors relative to their bin
     // workspace (per group g)
-    uint32_t *hist;      // [g][16][256] radix histograms of the unique prefixes
-    uint32_t *prefix;    // [g][16] key prefix of each order statistic
-    int64_t *krank;      // [g][16] its rank among samples with that prefix
-    uint32_t *uprefix;   // [g][17]: [0] = number of unique prefixes, then the prefixes
-    double *psum;        // [g][blocks][17] block partial sums
-    uint64_t *pcnt;      // [g][blocks][17] block partial counts
-    float *cent;         // [g][16] current centroids
-    int *state;          // [g][2]: converged, iterations run
-    float *out;          // [g][16]
+    uint32_t *oct;          // [g][512] samples per sign and exponent
+    uint32_t *map;          // [g][512] first bin << 5 | key bits below the bin number
+    uint32_t *cnt;          // [g][nb]
+    uint32_t *cursor;       // [g][nb] next free place of each bin
+    uint64_t *start;        // [g][nb + 1] first place of each bin
+    double *bsum;           // [g][nb]
+    double *csum;           // [g][nch] sums of 64 bins
+    float *buf;             // [g][n] samples by bin
+    float *out;             // [g][16]
+    int32_t *iters;         // [g], nullable
 };
 
 __device__ __forceinline__ uint32_t lm_key(float f) {
@@ -64,428 +92,838 @@ __device__ __forceinline__ float lm_value(uint32_t k) {
 }
 
 template <int DT>
-__device__ __forceinline__ float lm_load(const LmArgs &a, int64_t o, int64_t i, int g) {
-    const int64_t idx = o * a.outer_stride + (int64_t)g * a.group_stride + i;
-    if constexpr (DT == OMNI_F32) return reinterpret_cast<const float *>(a.x)[idx];
-    const uint16_t h = reinterpret_cast<const uint16_t *>(a.x)[idx];
-    if constexpr (DT == OMNI_BF16) return bf16_to_f32(h);
-    return f16_to_f32(h);
+__device__ __forceinline__ float lm_widen(uint16_t h) {
+    return DT == OMNI_BF16 ? bf16_to_f32(h) : f16_to_f32(h);
 }
 
-// Visit this thread's elements of group g in a fixed order:
-// e = start, start + stride, ... (grid-stride over the flattened index,
-// the (row, column) pair advanced without division).
-// Eight loads are issued before the eight samples are used (the loop is
-// otherwise bound by one memory latency per sample).
-template <int DT, typename F>
-__device__ __forceinline__ void lm_for_each(const LmArgs &a, int g, F &&f) {
-    constexpr int U = 8;
-    const int64_t stride = (int64_t)a.blocks * kLmThreads;
-    const int64_t start = (int64_t)blockIdx.x * kLmThreads + threadIdx.x;
-    if (start >= a.n) return;
-    const int64_t so = stride / a.inner, si = stride % a.inner;
-    int64_t o = start / a.inner, i = start % a.inner;
-    for (int64_t e = start; e < a.n; e += U * stride) {
-        float xv[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            xv[u] = e + u * stride < a.n ? lm_load<DT>(a, o, i, g) : 0.0f;
-            o += so;
-            i += si;
-            if (i >= a.inner) {
-                i -= a.inner;
-                ++o;
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-            if (e + u * stride < a.n) f(xv[u]);
-    }
-}
-
-__global__ void lm_clear_kernel(LmArgs a) {
-    const int g = blockIdx.y;
-    uint32_t *h = a.hist + (size_t)g * kLmK * 256;
-    for (int s = threadIdx.x; s < kLmK * 256; s += blockDim.x) h[s] = 0u;
-    if (threadIdx.x < kLmK) {
-        a.prefix[g * kLmK + threadIdx.x] = 0u;
-        a.krank[g * kLmK + threadIdx.x] = (int64_t)(threadIdx.x + 1) * a.bs - 1;
-    }
-    if (threadIdx.x == 0) {
-        a.uprefix[g * (kLmK + 1)] = 1u;       // one unique (empty) prefix
-        a.uprefix[g * (kLmK + 1) + 1] = 0u;
-        a.state[2 * g] = 0;
-        a.state[2 * g + 1] = 0;
-    }
-}
-
-// Radix pass: histogram of key digit `pass` (bits 31-24 first) over the
-// samples whose higher digits equal one of the unique prefixes.
+// This thread's samples of the block's run of kLmBlock: bit s of the result
+// says that xv[s] is one.  The (row, column) pair advances without division.
 template <int DT>
-__global__ __launch_bounds__(kLmThreads) void lm_radix_kernel(LmArgs a, int pass) {
-    const int g = blockIdx.y;
-    __shared__ uint32_t lh[kLmK * 256];
-    __shared__ uint32_t up[kLmK];
-    const uint32_t nu = a.uprefix[g * (kLmK + 1)];
-    for (int s = threadIdx.x; s < kLmK * 256; s += kLmThreads) lh[s] = 0u;
-    if (threadIdx.x < kLmK) up[threadIdx.x] = a.uprefix[g * (kLmK + 1) + 1 + threadIdx.x];
-    __syncthreads();
-    const int shift = 24 - 8 * pass;
-    lm_for_each<DT>(a, g, [&](float x) {
-        const uint32_t key = lm_key(x);
-        const uint32_t hi = pass == 0 ? 0u : key >> (shift + 8);
-        const uint32_t dig = (key >> shift) & 0xffu;
-        for (uint32_t u = 0; u < nu; ++u)
-            if (up[u] == hi) {
-                atomicAdd(&lh[u * 256 + dig], 1u);
-                break;
+__device__ __forceinline__ uint32_t lm_load_run(const LmArgs &a, int g, float (&xv)[kLmPer]) {
+    const int w = a.vec ? 4 : 1;
+    const int64_t first = (int64_t)blockIdx.x * kLmBlock + (int64_t)threadIdx.x * w;
+    const int64_t stride = (int64_t)kLmThreads * w;
+    int64_t o = 0, i = first, so = 0, si = stride;
+    if (a.outer > 1) {
+        o = first / a.inner;
+        i = first - o * a.inner;
+        so = stride / a.inner;
+        si = stride - so * a.inner;
+    }
+    uint32_t valid = 0u;
+    const int64_t gbase = (int64_t)g * a.group_stride;
+    auto next = [&]() {
+        o += so;
+        i += si;
+        if (i >= a.inner) {
+            i -= a.inner;
+            ++o;
+        }
+    };
+    if (a.vec) {
+#pragma unroll
+        for (int j = 0; j < kLmPer / 4; ++j) {
+            const bool ok = first + j * stride < a.n;
+            const int64_t idx = ok ? o * a.outer_stride + gbase + i : gbase;
+            if constexpr (DT == OMNI_F32) {
+                const float4 t = *reinterpret_cast<const float4 *>(reinterpret_cast<const float *>(a.x) + idx);
+                xv[4 * j] = t.x; xv[4 * j + 1] = t.y; xv[4 * j + 2] = t.z; xv[4 * j + 3] = t.w;
+            } else {
+                const uint2 t = *reinterpret_cast<const uint2 *>(reinterpret_cast<const uint16_t *>(a.x) + idx);
+                xv[4 * j] = lm_widen<DT>((uint16_t)t.x); xv[4 * j + 1] = lm_widen<DT>((uint16_t)(t.x >> 16));
+                xv[4 * j + 2] = lm_widen<DT>((uint16_t)t.y); xv[4 * j + 3] = lm_widen<DT>((uint16_t)(t.y >> 16));
             }
-    });
-    __syncthreads();
-    uint32_t *h = a.hist + (size_t)g * kLmK * 256;
-    for (int s = threadIdx.x; s < (int)nu * 256; s += kLmThreads)
-        if (lh[s]) atomicAdd(&h[s], lh[s]);
+            valid |= ok ? 15u << (4 * j) : 0u;
+            next();
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < kLmPer; ++j) {
+            const bool ok = first + j * stride < a.n;
+            const int64_t idx = ok ? o * a.outer_stride + gbase + i : gbase;
+            if constexpr (DT == OMNI_F32) xv[j] = reinterpret_cast<const float *>(a.x)[idx];
+            else xv[j] = lm_widen<DT>(reinterpret_cast<const uint16_t *>(a.x)[idx]);
+            valid |= ok ? 1u << j : 0u;
+            next();
+        }
+    }
+    return valid;
 }
 
-// After a radix pass: each order statistic picks its digit (one wave per
-// statistic: a prefix sum of the 256 bin counts over the lanes, four bins
-// per lane), the unique prefixes for the next pass are listed, and the
-// histograms are cleared.
-__global__ __launch_bounds__(256) void lm_select_kernel(LmArgs a) {
+__device__ __forceinline__ uint32_t lm_bin(uint32_t map, uint32_t key) {
+    return (map >> 5) + ((key & 0x7fffffu) >> (map & 31u));
+}
+
+__global__ __launch_bounds__(256) void lm_clear_kernel(LmArgs a) {
+    const int b = blockIdx.x * 256 + threadIdx.x;
+    if (b < kLmOct) a.oct[(size_t)blockIdx.y * kLmOct + b] = 0u;
+    if (b >= a.nb) return;
+    const size_t at = (size_t)blockIdx.y * a.nb + b;
+    a.cnt[at] = 0u;
+    a.bsum[at] = 0.0;
+}
+
+// Samples per sign and exponent.  Most of them share a few: four copies of
+// the counters per block.
+template <int DT>
+__global__ __launch_bounds__(kLmThreads) void lm_oct_kernel(LmArgs a) {
+    __shared__ uint32_t lh[4][kLmOct];
     const int g = blockIdx.y;
-    uint32_t *h = a.hist + (size_t)g * kLmK * 256;
-    uint32_t *upg = a.uprefix + g * (kLmK + 1);
-    __shared__ uint32_t newp[kLmK];
-    const uint32_t nu = upg[0];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    for (int j = w; j < kLmK; j += 4) {
-        const uint32_t p = a.prefix[g * kLmK + j];
-        uint32_t u = 0;
-        while (u + 1 < nu && upg[1 + u] != p) ++u;
-        const int64_t k = a.krank[g * kLmK + j];
-        const uint4 c4 = reinterpret_cast<const uint4 *>(h + u * 256)[lane];
-        const uint64_t mine = (uint64_t)c4.x + c4.y + c4.z + c4.w;
-        uint64_t incl = mine;
+    float xv[kLmPer];
+    const uint32_t valid = lm_load_run<DT>(a, g, xv);
+    for (int w = threadIdx.x; w < 4 * kLmOct; w += kLmThreads) lh[0][w] = 0u;
+    __syncthreads();
+    uint32_t *mine = lh[threadIdx.x & 3];
 #pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const uint64_t y = __shfl_up(incl, off);
-            if (lane >= off) incl += y;
+    for (int s = 0; s < kLmPer; ++s)
+        if ((valid >> s) & 1u) atomicAdd(&mine[lm_key(xv[s]) >> 23], 1u);
+    __syncthreads();
+    for (int w = threadIdx.x; w < kLmOct; w += kLmThreads) {
+        const uint32_t v = lh[0][w] + lh[1][w] + lh[2][w] + lh[3][w];
+        if (v) atomicAdd(&a.oct[(size_t)g * kLmOct + w], v);
+    }
+}
+
+// Bins of each sign and exponent: 2^m with m the smallest that leaves `fill`
+// samples a bin or fewer on average (at most one per value of the sample
+// type), so 2 n / fill + 512 of them at most.
+__global__ __launch_bounds__(kLmOct) void lm_map_kernel(LmArgs a) {
+    __shared__ uint32_t wsum[kLmOct / 64];
+    const int g = blockIdx.x, t = threadIdx.x, lane = t & 63, w = t >> 6;
+    const uint64_t c = a.oct[(size_t)g * kLmOct + t];
+    int m = 0;
+    while (m < a.mant && ((uint64_t)a.fill << m) < c) ++m;
+    const uint32_t mine = 1u << m;
+    uint32_t incl = mine;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t y = __shfl_up(incl, off);
+        if (lane >= off) incl += y;
+    }
+    if (lane == 63) wsum[w] = incl;
+    __syncthreads();
+    uint32_t base = incl - mine;
+    for (int q = 0; q < w; ++q) base += wsum[q];
+    a.map[(size_t)g * kLmOct + t] = (base << 5) | (uint32_t)(23 - m);
+}
+
+// Samples per bin: 16-bit counters of a block's 32768 samples in LDS, then
+// one global addition per bin that the block met.
+template <int DT>
+__global__ __launch_bounds__(kLmThreads) void lm_count_kernel(LmArgs a) {
+    __shared__ uint32_t lh[kLmMaxBins / 2];
+    __shared__ uint32_t map[kLmOct];
+    const int g = blockIdx.y;
+    float xv[kLmPer];
+    const uint32_t valid = lm_load_run<DT>(a, g, xv);
+    const int words = a.nb / 2;
+    for (int w = threadIdx.x; w < words; w += kLmThreads) lh[w] = 0u;
+    if (threadIdx.x < kLmOct) map[threadIdx.x] = a.map[(size_t)g * kLmOct + threadIdx.x];
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < kLmPer; ++s)
+        if ((valid >> s) & 1u) {
+            const uint32_t k = lm_key(xv[s]), b = lm_bin(map[k >> 23], k);
+            atomicAdd(&lh[b >> 1], (b & 1u) ? 65536u : 1u);
         }
-        // the bin holding rank k lies in the first lane whose inclusive count exceeds k
-        const uint64_t over = __ballot(incl > (uint64_t)k);
-        const int L = over ? __ffsll((unsigned long long)over) - 1 : 63;
-        int64_t kk = k - (int64_t)__shfl(incl - mine, L);
-        const uint32_t b0 = __shfl(c4.x, L), b1 = __shfl(c4.y, L), b2 = __shfl(c4.z, L);
-        int d = 4 * L;
-        if (kk >= (int64_t)b0) {
-            kk -= b0;
-            ++d;
-            if (kk >= (int64_t)b1) {
-                kk -= b1;
-                ++d;
-                if (kk >= (int64_t)b2) {
-                    kk -= b2;
-                    ++d;
+    __syncthreads();
+    uint32_t *cnt = a.cnt + (size_t)g * a.nb;
+    for (int w = threadIdx.x; w < words; w += kLmThreads) {
+        const uint32_t v = lh[w];
+        if (v & 0xffffu) atomicAdd(&cnt[2 * w], v & 0xffffu);
+        if (v >> 16) atomicAdd(&cnt[2 * w + 1], v >> 16);
+    }
+}
+
+// First place of each bin: a block takes 4096 bins, four per thread, after
+// the sum of all bins before them.
+constexpr int kLmScan = 4 * kLmThreads;
+
+__global__ __launch_bounds__(kLmThreads) void lm_scan_kernel(LmArgs a) {
+    __shared__ uint64_t wsum[kLmThreads / 64], wpre[kLmThreads / 64];
+    const int g = blockIdx.y, t = threadIdx.x, lane = t & 63, w = t >> 6;
+    const uint4 *cnt = reinterpret_cast<const uint4 *>(a.cnt + (size_t)g * a.nb);
+    uint64_t pre = 0;
+    for (int k = t; k < (int)blockIdx.x * kLmThreads; k += kLmThreads) {
+        const uint4 v = cnt[k];
+        pre += (uint64_t)v.x + v.y + v.z + v.w;
+    }
+    const int b0 = (int)blockIdx.x * kLmScan + 4 * t;
+    const uint4 v = b0 < a.nb ? cnt[b0 >> 2] : make_uint4(0u, 0u, 0u, 0u);
+    const uint32_t cv[4] = {v.x, v.y, v.z, v.w};
+    const uint64_t mine = (uint64_t)v.x + v.y + v.z + v.w;
+    uint64_t incl = mine;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint64_t y = __shfl_up((unsigned long long)incl, off);
+        if (lane >= off) incl += y;
+        pre += __shfl_xor((unsigned long long)pre, off);
+    }
+    if (lane == 63) {
+        wsum[w] = incl;
+        wpre[w] = pre;
+    }
+    __syncthreads();
+    uint64_t at = incl - mine;
+    for (int q = 0; q < kLmThreads / 64; ++q) at += wpre[q] + (q < w ? wsum[q] : 0);
+    if (b0 >= a.nb) return;
+    uint64_t *start = a.start + (size_t)g * (a.nb + 1);
+    uint32_t *cursor = a.cursor + (size_t)g * a.nb;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const int b = b0 + k;
+        start[b] = at;
+        cursor[b] = a.wide ? 0u : (uint32_t)at;
+        at += cv[k];
+    }
+    if (b0 + 4 == a.nb) start[a.nb] = at;
+}
+
+// Samples to their bins: a block ranks its samples per bin in LDS, reserves a
+// run of every bin that it met with one global addition, and writes.  The
+// order inside a bin is not fixed and nothing below depends on it.
+template <int DT>
+__global__ __launch_bounds__(kLmThreads) void lm_store_kernel(LmArgs a) {
+    __shared__ uint32_t lh[kLmMaxBins];
+    __shared__ uint32_t map[kLmOct];
+    const int g = blockIdx.y;
+    float xv[kLmPer];
+    const uint32_t valid = lm_load_run<DT>(a, g, xv);
+    uint32_t *cursor = a.cursor + (size_t)g * a.nb;
+    float *buf = a.buf + (size_t)g * a.n;
+    for (int s = threadIdx.x; s < a.nb; s += kLmThreads) lh[s] = 0u;
+    if (threadIdx.x < kLmOct) map[threadIdx.x] = a.map[(size_t)g * kLmOct + threadIdx.x];
+    __syncthreads();
+    uint32_t at[kLmPer];                               // bin, rank among the block's samples in it << 15
+#pragma unroll
+    for (int s = 0; s < kLmPer; ++s) {
+        at[s] = 0u;
+        if ((valid >> s) & 1u) {
+            const uint32_t k = lm_key(xv[s]), b = lm_bin(map[k >> 23], k);
+            at[s] = b | (atomicAdd(&lh[b], 1u) << 15);
+        }
+    }
+    static_assert(kLmMaxBins <= 1 << 15 && kLmBlock <= 1 << 15, "bin and rank share 32 bits");
+    __syncthreads();
+    for (int s = threadIdx.x; s < a.nb; s += kLmThreads) {
+        const uint32_t c = lh[s];
+        if (c) lh[s] = atomicAdd(&cursor[s], c);
+    }
+    __syncthreads();
+    if (a.wide) {
+        const uint64_t *start = a.start + (size_t)g * (a.nb + 1);
+#pragma unroll
+        for (int s = 0; s < kLmPer; ++s)
+            if ((valid >> s) & 1u) buf[start[at[s] & 32767u] + lh[at[s] & 32767u] + (at[s] >> 15)] = xv[s];
+    } else {
+#pragma unroll
+        for (int s = 0; s < kLmPer; ++s)
+            if ((valid >> s) & 1u) buf[lh[at[s] & 32767u] + (at[s] >> 15)] = xv[s];
+    }
+}
+
+// Lane l's value as a scalar (l wave-uniform): the wave's own state stays in
+// scalar registers and its branches uniform.
+__device__ __forceinline__ float lm_lane(float v, int l) {
+    return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), l));
+}
+__device__ __forceinline__ double lm_lane(double v, int l) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    return __builtin_bit_cast(double, (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, l) |
+                                          ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), l) << 32));
+}
+
+// Wave sums by DPP row shifts (1, 2, 4, 8: each row's last lane holds its
+// sum) and row broadcasts (15 into rows 1 and 3, 31 into rows 2 and 3), no LDS
+// permutes; the result is a scalar.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint32_t lm_dpp(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xf, false);
+}
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double lm_dpp_add(double v) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint64_t t = (uint64_t)lm_dpp<CTRL, ROWS>((uint32_t)u) | ((uint64_t)lm_dpp<CTRL, ROWS>((uint32_t)(u >> 32)) << 32);
+    return v + __builtin_bit_cast(double, t);
+}
+__device__ __forceinline__ double lm_wave_sum(double v) {
+    v = lm_dpp_add<0x111, 0xf>(v);
+    v = lm_dpp_add<0x112, 0xf>(v);
+    v = lm_dpp_add<0x114, 0xf>(v);
+    v = lm_dpp_add<0x118, 0xf>(v);
+    v = lm_dpp_add<0x142, 0xa>(v);
+    v = lm_dpp_add<0x143, 0xc>(v);
+    return lm_lane(v, 63);
+}
+__device__ __forceinline__ uint32_t lm_wave_sum_u32(uint32_t v) {
+    v += lm_dpp<0x111, 0xf>(v);
+    v += lm_dpp<0x112, 0xf>(v);
+    v += lm_dpp<0x114, 0xf>(v);
+    v += lm_dpp<0x118, 0xf>(v);
+    v += lm_dpp<0x142, 0xa>(v);
+    v += lm_dpp<0x143, 0xc>(v);
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+
+// fp64 sum of each bin: a wave takes 1024 consecutive stored samples, mostly
+// one bin per 64, and adds once per bin.  Exact in any order (one exponent
+// per bin, up to 2^29 samples).
+__global__ __launch_bounds__(256) void lm_binsum_kernel(LmArgs a) {
+    constexpr int kVec = 16;
+    const int g = blockIdx.y, lane = threadIdx.x & 63;
+    const int64_t base = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * (64 * kVec);
+    if (base >= a.n) return;
+    const float *buf = a.buf + (size_t)g * a.n;
+    double *bsum = a.bsum + (size_t)g * a.nb;
+    const uint32_t *map = a.map + (size_t)g * kLmOct;
+    float v[kVec];
+    uint32_t bn[kVec];
+#pragma unroll
+    for (int k = 0; k < kVec; ++k) {
+        const int64_t e = base + 64 * k + lane;
+        v[k] = buf[e < a.n ? e : a.n - 1];
+    }
+#pragma unroll
+    for (int k = 0; k < kVec; ++k) {
+        const uint32_t key = lm_key(v[k]);
+        bn[k] = lm_bin(map[key >> 23], key);
+    }
+    double acc = 0.0;
+    uint32_t cur = 0u;
+    bool open = false;
+    auto flush = [&]() {
+        if (open) {
+            const double t = lm_wave_sum(acc);
+            if (lane == 0) unsafeAtomicAdd(&bsum[cur], t);
+        }
+        open = false;
+        acc = 0.0;
+    };
+#pragma unroll
+    for (int k = 0; k < kVec; ++k) {
+        const bool ok = base + 64 * k + lane < a.n;
+        const uint32_t b = bn[k];
+        const uint32_t b0 = __builtin_amdgcn_readfirstlane(b);
+        if (__builtin_amdgcn_ballot_w64(!ok || b != b0) == 0ull) {
+            if (open && b0 != cur) flush();
+            cur = b0;
+            open = true;
+            acc += (double)v[k];
+        } else {
+            // several bins: sums over each run of equal bins, added by its last lane
+            double t = ok ? (double)v[k] : 0.0;
+#pragma unroll
+            for (int d = 1; d < 64; d <<= 1) {
+                const double u = __shfl_up(t, d);
+                const uint32_t ub = __shfl_up(b, d);
+                if (lane >= d && ub == b) t += u;
+            }
+            const uint32_t nb1 = __shfl_down(b, 1);
+            const bool okn = __shfl_down(ok ? 1 : 0, 1) != 0;
+            if (ok && (lane == 63 || nb1 != b || !okn)) unsafeAtomicAdd(&bsum[b], t);
+        }
+    }
+    flush();
+}
+
+// Sums of 64 bins (a wave each).
+__global__ __launch_bounds__(kLmThreads) void lm_chunk_kernel(LmArgs a) {
+    const int g = blockIdx.y, lane = threadIdx.x & 63, c = blockIdx.x * (kLmThreads / 64) + (threadIdx.x >> 6);
+    if (c >= a.nch) return;
+    const double s = lm_wave_sum(a.bsum[(size_t)g * a.nb + 64 * c + lane]);
+    if (lane == 0) a.csum[(size_t)g * a.nch + c] = s;
+}
+
+// d_a <= d_b for a < b as the fp32 distances decide it, false from b on
+// (there the pairs further right decide); ascending x: true, then false.
+__device__ __forceinline__ bool lm_left(float x, float a, float b) {
+    return x < b && fabsf(x - a) <= fabsf(x - b);
+}
+
+// Key of the largest value that takes a's code rather than b's (wave).
+__device__ __forceinline__ uint32_t lm_threshold(float a, float b, int lane) {
+    uint32_t lo = lm_key(a), hi = lm_key(b);          // lm_left(lo), !lm_left(hi)
+    {
+        // 64 values around the midpoint: nearly always enough
+        const uint32_t mid = lm_key(0.5f * a + 0.5f * b);
+        const uint32_t k = mid - 32u + (uint32_t)lane;
+        const bool in = mid > lo + 32u && mid + 32u < hi;
+        const uint64_t t = __builtin_amdgcn_ballot_w64(in && lm_left(lm_value(k), a, b));
+        const int c = __popcll(t);
+        if (c > 0 && c < 64) return mid - 32u + (uint32_t)c - 1u;
+    }
+    while (hi - lo > 1u) {
+        const uint32_t step = (hi - lo + 63u) >> 6;
+        // offsets, not keys: lo + 64 step can pass 2^32
+        const uint64_t off = (uint64_t)step * (uint32_t)(lane + 1);
+        const uint64_t t = __builtin_amdgcn_ballot_w64(off < (uint64_t)(hi - lo) &&
+                                                       lm_left(lm_value(lo + (uint32_t)off), a, b));
+        const uint32_t c = (uint32_t)__popcll(t);
+        const uint64_t up = (uint64_t)step * (c + 1u);
+        if (up < (uint64_t)(hi - lo)) hi = lo + (uint32_t)up;
+        lo += step * c;
+    }
+    return lo;
+}
+
+// One boundary's bin, held by a wave: its samples as the low bits of their
+// ordered keys, kLmCache per lane (a larger bin is read from memory).
+struct LmBin {
+    int bin;                 // -1: none yet
+    int sh;                  // key bits below the bin number
+    uint32_t klo;            // the bin's first key
+    uint32_t cnt;
+    uint64_t at;             // its first place
+    double sum;
+    const float *src;
+    uint32_t low[kLmCache];
+};
+
+// fp64 sum of c samples of the bin whose ordered low bits sum to `low`
+// (exact: sign * (count * base + ulp * sum of magnitude bits)).
+__device__ __forceinline__ double lm_bin_value(const LmBin &B, uint64_t c, uint64_t low) {
+    const uint32_t mask = (1u << B.sh) - 1u;
+    const bool neg = (B.klo & 0x80000000u) == 0u;
+    const uint32_t u = neg ? ~B.klo & 0x7fffffffu : B.klo & 0x7fffffffu;   // magnitude bits of the first key
+    const uint32_t ex = (u >> 23) > 1u ? u >> 23 : 1u;
+    const double base = (double)__uint_as_float(u & ~mask);
+    const double ulp = __builtin_bit_cast(double, (uint64_t)(ex - 150u + 1023u) << 52);   // 2^(ex - 150)
+    const uint64_t mag = neg ? c * mask - low : low;
+    const double s = (double)c * base + ulp * (double)mag;
+    return neg ? -s : s;
+}
+
+// Samples of the bin with ordered low bits <= t: their number and the sum of
+// their low bits.
+__device__ __forceinline__ void lm_scan_bin(const LmArgs &a, const LmBin &B, uint32_t t, int lane, uint64_t &c_out,
+                                            uint64_t &s_out) {
+    const uint32_t mask = (1u << B.sh) - 1u;
+    if (B.sh <= 23 - a.mant) {
+        // one value of the sample type: its low bits are zeros (of a negative key: ones)
+        const uint32_t l = (B.klo & 0x80000000u) ? 0u : mask;
+        c_out = l <= t ? B.cnt : 0u;
+        s_out = (uint64_t)l * c_out;
+        return;
+    }
+    if (B.cnt <= 64u * kLmCache) {
+        uint32_t s = 0u, n = 0u;
+#pragma unroll
+        for (int q = 0; q < kLmCache / 4; ++q) {
+            if (256u * q < B.cnt) {                    // wave-uniform
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const uint32_t l = B.low[4 * q + k];
+                    const bool in = l <= t;
+                    n += in ? 1u : 0u;
+                    s += in ? l : 0u;
                 }
             }
         }
-        if (lane == 0) {
-            a.krank[g * kLmK + j] = kk;
-            newp[j] = (p << 8) | (uint32_t)d;
+        // two 32-bit wave sums: s < 2^28 in an 18-bit part and the rest,
+        // n <= 32 above the latter
+        static_assert(kLmCache <= 32, "s and n of a lane fit their parts");
+        const uint32_t p0 = lm_wave_sum_u32(s & 0x3ffffu), p1 = lm_wave_sum_u32((s >> 18) | (n << 18));
+        c_out = p1 >> 18;
+        s_out = ((uint64_t)(p1 & 0x3ffffu) << 18) + p0;
+        return;
+    }
+    uint64_t s = 0, c = 0;
+    for (uint32_t e = 0; e < B.cnt; e += 64u * 8u) {
+        uint32_t l[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const uint32_t i = e + 64u * k + (uint32_t)lane;
+            l[k] = i < B.cnt ? lm_key(B.src[i]) & mask : 0xffffffffu;
+        }
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const bool in = l[k] <= t;
+            c += (uint64_t)__popcll(__builtin_amdgcn_ballot_w64(in));
+            s += in ? l[k] : 0u;
         }
     }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        uint32_t n = 0;
-        for (int j = 0; j < kLmK; ++j) {
-            a.prefix[g * kLmK + j] = newp[j];
-            if (n == 0 || upg[n] != newp[j]) upg[1 + n++] = newp[j];   // prefixes ascend with j
-        }
-        upg[0] = n;
-    }
-    for (int t = threadIdx.x; t < kLmK * 256; t += blockDim.x) h[t] = 0u;
+    c_out = c;
+    s_out = (uint64_t)lm_wave_sum((double)s);          // < 2^53: exact
 }
 
-// Adds x to this thread's own LDS slot (fp64 sum, count).  Slots are
-// private to a thread, so the additions happen in its program order (the
-// same sums as register accumulators, without a 17-way select per sample).
-__device__ __forceinline__ void lm_slot_add(double *sum, uint32_t *cnt, float x) {
-    __hip_atomic_fetch_add(sum, (double)x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-
-// Block-wide fixed-order sum of nq (sum, count) pairs into the partials:
-// an xor tree inside each wave, then the four waves in order.
-__device__ __forceinline__ void lm_block_store(const LmArgs &a, int g, double (&s)[kLmIntervals],
-                                               uint64_t (&c)[kLmIntervals], int nq) {
-    constexpr int nwv = kLmThreads / 64;
-    __shared__ double ws[nwv][kLmIntervals];
-    __shared__ uint64_t wc[nwv][kLmIntervals];
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+// Requests the samples of bin `bin` (first key klo, sh key bits below its
+// number, cnt samples from place `at` on): raw until lm_settle_bin.
+__device__ __forceinline__ void lm_open_bin(const LmArgs &a, int g, LmBin &B, int bin, uint32_t klo, int sh,
+                                            uint64_t at, uint32_t cnt, int lane) {
+    B.bin = bin;
+    B.klo = klo;
+    B.sh = sh;
+    B.cnt = cnt;
+    B.at = at;
+    B.src = a.buf + (size_t)g * a.n + at;
+    if (cnt > 0u && cnt <= 64u * kLmCache && sh > 23 - a.mant) {
+        const uint32_t last = cnt - 1u;
 #pragma unroll
-    for (int m = 32; m >= 1; m >>= 1)
+        for (int q = 0; q < kLmCache / 4; ++q) {
+            if (256u * q < cnt) {
 #pragma unroll
-        for (int q = 0; q < kLmIntervals; ++q) {
-            s[q] += __shfl_xor(s[q], m);
-            c[q] += (uint64_t)__shfl_xor((unsigned long long)c[q], m);
-        }
-    if (lane == 0)
-#pragma unroll
-        for (int q = 0; q < kLmIntervals; ++q) {
-            ws[w][q] = s[q];
-            wc[w][q] = c[q];
-        }
-    __syncthreads();
-    if (t < nq) {
-        double ts = ws[0][t];
-        uint64_t tc = wc[0][t];
-#pragma unroll
-        for (int v = 1; v < nwv; ++v) {
-            ts += ws[v][t];
-            tc += wc[v][t];
-        }
-        const size_t o = ((size_t)g * a.blocks + blockIdx.x) * kLmIntervals + t;
-        a.psum[o] = ts;
-        a.pcnt[o] = tc;
-    }
-}
-
-// Sums and counts of the samples in each interval between the 16 order
-// statistics v_0 <= ... <= v_15: interval t holds #{j : v_j <= x} = t.
-template <int DT>
-__global__ __launch_bounds__(kLmThreads) void lm_interval_kernel(LmArgs a) {
-    const int g = blockIdx.y;
-    __shared__ double ls[kLmIntervals][kLmThreads];
-    __shared__ uint32_t lc[kLmIntervals][kLmThreads];
-    const int th = threadIdx.x;
-    float v[kLmK];
-#pragma unroll
-    for (int j = 0; j < kLmK; ++j) v[j] = lm_value(a.prefix[g * kLmK + j]);
-#pragma unroll
-    for (int q = 0; q < kLmIntervals; ++q) {
-        ls[q][th] = 0.0;
-        lc[q][th] = 0u;
-    }
-    lm_for_each<DT>(a, g, [&](float x) {
-        int t = 0;
-#pragma unroll
-        for (int j = 0; j < kLmK; ++j) t += v[j] <= x ? 1 : 0;
-        lm_slot_add(&ls[t][th], &lc[t][th], x);
-    });
-    double s[kLmIntervals];
-    uint64_t c[kLmIntervals];
-#pragma unroll
-    for (int q = 0; q < kLmIntervals; ++q) {
-        s[q] = ls[q][th];
-        c[q] = lc[q][th];
-    }
-    lm_block_store(a, g, s, c, kLmIntervals);
-}
-
-// Initial centroids from the order statistics and the interval sums
-// (thread t < 255 sums interval t / 15 over blocks t % 15, t % 15 + 15, ...;
-// the 15 partial sums of an interval are then added in order).
-__global__ __launch_bounds__(256) void lm_init_kernel(LmArgs a) {
-    const int g = blockIdx.y;
-    constexpr int kParts = 15;
-    __shared__ double ps[kLmIntervals][kParts];
-    __shared__ uint64_t pc[kLmIntervals][kParts];
-    const int t = threadIdx.x;
-    if (t < kLmIntervals * kParts) {
-        const int q = t / kParts, part = t % kParts;
-        double s = 0.0;
-        uint64_t n = 0;
-        for (int bl = part; bl < a.blocks; bl += kParts) {
-            const size_t o = ((size_t)g * a.blocks + bl) * kLmIntervals + q;
-            s += a.psum[o];
-            n += a.pcnt[o];
-        }
-        ps[q][part] = s;
-        pc[q][part] = n;
-    }
-    __syncthreads();
-    if (t != 0) return;
-    double isum[kLmIntervals];
-    uint64_t icnt[kLmIntervals];
-    for (int q = 0; q < kLmIntervals; ++q) {
-        isum[q] = 0.0;
-        icnt[q] = 0;
-        for (int part = 0; part < kParts; ++part) {
-            isum[q] += ps[q][part];
-            icnt[q] += pc[q][part];
-        }
-    }
-    double prev_f = 0.0, s_lt = 0.0;
-    uint64_t c_lt = 0;
-    for (int j = 0; j < kLmK; ++j) {
-        // samples below v_j: intervals 0..j
-        s_lt += isum[j];
-        c_lt += icnt[j];
-        const double vj = (double)lm_value(a.prefix[g * kLmK + j]);
-        const double m = (double)((j + 1) * a.bs);
-        const double f = s_lt + vj * (m - (double)c_lt);
-        a.cent[g * kLmK + j] = (float)((f - prev_f) / (double)a.bs);
-        prev_f = f;
-    }
-}
-
-// One Lloyd step, part 1: per-cell sums and counts under the current centroids.
-template <int DT>
-__global__ __launch_bounds__(kLmThreads) void lm_assign_kernel(LmArgs a) {
-    const int g = blockIdx.y;
-    if (a.state[2 * g]) return;                      // converged: uniform for the block
-    __shared__ double ls[kLmK][kLmThreads];
-    __shared__ uint32_t lc[kLmK][kLmThreads];
-    const int th = threadIdx.x;
-    float c[kLmK];
-#pragma unroll
-    for (int k = 0; k < kLmK; ++k) {
-        c[k] = a.cent[g * kLmK + k];
-        ls[k][th] = 0.0;
-        lc[k][th] = 0u;
-    }
-    lm_for_each<DT>(a, g, [&](float x) {
-        int best = 0;
-        float bd = fabsf(x - c[0]);
-#pragma unroll
-        for (int k = 1; k < kLmK; ++k) {
-            const float d = fabsf(x - c[k]);
-            if (d < bd) {
-                bd = d;
-                best = k;
+                for (int k = 0; k < 4; ++k) {
+                    const uint32_t i = 64u * (4 * q + k) + (uint32_t)lane;
+                    B.low[4 * q + k] = __float_as_uint(B.src[i < last ? i : last]);
+                }
             }
         }
-        lm_slot_add(&ls[best][th], &lc[best][th], x);
-    });
-    double s[kLmIntervals];
-    uint64_t n[kLmIntervals];
+    }
+}
+
+// Raw samples to ordered low bits, lanes past the last to all ones.
+__device__ __forceinline__ void lm_settle_bin(LmBin &B, int lane) {
+    const uint32_t flip = (B.klo & 0x80000000u) ? 0x80000000u : 0xffffffffu;   // key = u ^ flip (one sign)
 #pragma unroll
-    for (int k = 0; k < kLmK; ++k) {
-        s[k] = ls[k][th];
-        n[k] = lc[k][th];
+    for (int q = 0; q < kLmCache / 4; ++q) {
+        if (256u * q < B.cnt && B.cnt <= 64u * kLmCache) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const uint32_t i = 64u * (4 * q + k) + (uint32_t)lane;
+                const uint32_t l = (B.low[4 * q + k] ^ flip) - B.klo;
+                B.low[4 * q + k] = i < B.cnt ? l : 0xffffffffu;
+            }
+        }
     }
-    s[kLmK] = 0.0;
-    n[kLmK] = 0;
-    lm_block_store(a, g, s, n, kLmK);
 }
 
-// One Lloyd step, part 2: new centroids, the largest move, convergence.
-// 256 threads: thread t sums cell t % 16 over blocks t / 16, t / 16 + 16,
-// ...; the 16 partial sums of a cell are then added in order.
-__global__ __launch_bounds__(256) void lm_update_kernel(LmArgs a) {
-    const int g = blockIdx.y;
-    __shared__ float moved[kLmK];
-    __shared__ double ps[16][kLmK];
-    __shared__ uint64_t pc[16][kLmK];
-    const int t = threadIdx.x, k = t & (kLmK - 1), part = t >> 4;
-    if (a.state[2 * g]) return;
+// The whole calibration of a group: wave w finds order statistic w and then,
+// each step, boundary w and the mean of cell w.
+template <int DT>
+__global__ __launch_bounds__(kLmThreads) void lm_lloyd_kernel(LmArgs a) {
+    // places of the bins; a step that goes over the samples one by one uses
+    // the space for its sums and loads the places again
+    __shared__ __attribute__((aligned(16))) uint32_t place[kLmMaxBins + 4];
+    __shared__ double csum[kLmMaxBins / 64];
+    __shared__ uint32_t map[kLmOct];
+    __shared__ float cent2[2][kLmK], moved[kLmK];
+    __shared__ int bbin[kLmK];                         // boundary w: its bin (nb: none),
+    __shared__ uint64_t bcnt[kLmK];                    // the group's samples on its left,
+    __shared__ double bval[kLmK], bright[kLmK];        // the sums of its bin's samples on its left and right,
+    __shared__ double bhead[kLmK], btail[kLmK];        // and of the chunk's bins before and after that bin
+    __shared__ int slow;
+    double(*const ls)[kLmSlowSlots] = reinterpret_cast<double(*)[kLmSlowSlots]>(place);
+    uint32_t(*const lc)[kLmSlowSlots] = reinterpret_cast<uint32_t(*)[kLmSlowSlots]>(place + 2 * kLmK * kLmSlowSlots);
+    static_assert(3 * kLmK * kLmSlowSlots <= kLmMaxBins, "sums of the slow step fit the places' space");
+    const int g = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const double *bsum = a.bsum + (size_t)g * a.nb;
+    const uint64_t *start = a.start + (size_t)g * (a.nb + 1);
+    auto load_places = [&]() {
+        if (a.wide) return;                            // 64-bit places stay in memory
+        for (int b = tid; b <= a.nb; b += kLmThreads) place[b] = (uint32_t)start[b];
+    };
+    auto first_of = [&](int b) -> uint64_t { return a.wide ? start[b] : (uint64_t)place[b]; };
+    load_places();
+    for (int c = tid; c < a.nch; c += kLmThreads) csum[c] = a.csum[(size_t)g * a.nch + c];
+    if (tid < kLmOct) map[tid] = a.map[(size_t)g * kLmOct + tid];
+    __syncthreads();
+
+    LmBin B;
+    B.bin = -1;
+    B.cnt = 0u;
+    // Boundary w moves to the bin with first key klo: the one memory round
+    // trip of a step.  Its samples and its chunk's sums are requested together.
+    auto go_to = [&](int bin, uint32_t klo, int sh) {
+        if (bin == B.bin) return;
+        const uint64_t at = first_of(bin), end = first_of(bin + 1);
+        const uint32_t at_lo = __builtin_amdgcn_readfirstlane((uint32_t)at);
+        const uint32_t at_hi = __builtin_amdgcn_readfirstlane((uint32_t)(at >> 32));
+        const uint32_t n = __builtin_amdgcn_readfirstlane((uint32_t)(end - at));
+        const double mine = bsum[(bin & ~63) + lane];
+        lm_open_bin(a, g, B, bin, klo, sh, ((uint64_t)at_hi << 32) | at_lo, n, lane);
+        lm_settle_bin(B, lane);
+        B.sum = lm_lane(mine, bin & 63);
+        const double head = lm_wave_sum(lane < (bin & 63) ? mine : 0.0);
+        const double tail = lm_wave_sum(lane > (bin & 63) ? mine : 0.0);
+        if (lane == 0) {
+            bhead[w] = head;
+            btail[w] = tail;
+        }
+    };
+    // `c` of the bin's samples, `s` the sum of their low bits, lie on the left
+    auto set_left = [&](uint64_t c, uint64_t s) {
+        const double left = lm_bin_value(B, c, s);
+        if (lane == 0) {
+            bbin[w] = B.bin;
+            bcnt[w] = B.at + c;
+            bval[w] = left;
+            bright[w] = B.sum - left;                  // exact
+        }
+    };
+    // first key and shift of a bin
+    auto bin_key = [&](int bin, uint32_t &klo, int &sh) {
+        int o = 0;
+#pragma unroll
+        for (int q = 0; q < kLmOct / 64; ++q)
+            o += __popcll(__builtin_amdgcn_ballot_w64((int)(map[64 * q + lane] >> 5) <= bin));
+        o -= 1;
+        const uint32_t m = __builtin_amdgcn_readfirstlane(map[o]);
+        sh = (int)(m & 31u);
+        klo = ((uint32_t)o << 23) | ((uint32_t)(bin - (int)(m >> 5)) << sh);
+    };
+    // bin of the sample of rank k
+    auto bin_of_rank = [&](uint64_t k) {
+        int lo = 0, hi = a.nb;
+        while (hi - lo > 1) {
+            const int step = (hi - lo + 63) >> 6;
+            const int at = lo + step * (lane + 1);
+            const int c = __popcll(__builtin_amdgcn_ballot_w64(at < hi && first_of(at < hi ? at : hi) <= k));
+            const int up = lo + step * (c + 1);
+            hi = up < hi ? up : hi;
+            lo += step * c;
+        }
+        return lo;
+    };
+    uint32_t klo;
+    int sh;
+    bin_key(bin_of_rank((uint64_t)a.n - 1u), klo, sh);
+    const float xmax = lm_value(klo | ((1u << sh) - 1u));      // the data's largest value, or a little more
     {
-        double s = 0.0;
-        uint64_t n = 0;
-        for (int bl = part; bl < a.blocks; bl += 16) {
-            const size_t o = ((size_t)g * a.blocks + bl) * kLmIntervals + k;
-            s += a.psum[o];
-            n += a.pcnt[o];
+        const uint64_t k = (uint64_t)(w + 1) * (uint64_t)a.bs - 1u;
+        const int bin = bin_of_rank(k);
+        bin_key(bin, klo, sh);
+        go_to(bin, klo, sh);
+        const uint64_t kk = k - B.at;
+        // smallest low bits with more than kk samples at or below
+        uint32_t lo = 0u, hi = (1u << sh) - 1u;
+        uint64_t c, s;
+        while (lo < hi) {
+            const uint32_t mid = lo + ((hi - lo) >> 1);
+            lm_scan_bin(a, B, mid, lane, c, s);
+            if (c > kk) hi = mid;
+            else lo = mid + 1u;
         }
-        ps[part][k] = s;
-        pc[part][k] = n;
+        lm_scan_bin(a, B, lo, lane, c, s);
+        // of the samples equal to it, those up to rank k
+        set_left(kk + 1u, s - (c - (kk + 1u)) * lo);
     }
     __syncthreads();
-    if (t < kLmK) {
-        double s = 0.0;
-        uint64_t n = 0;
-        for (int p = 0; p < 16; ++p) {
-            s += ps[p][k];
-            n += pc[p][k];
+
+    // samples and sum of cell w: right part of the bin of boundary w - 1, the
+    // whole bins between, left part of the bin of boundary w
+    int kl = -2, kr = -2;
+    double kmid = 0.0;                                 // whole chunks between, kept with (kl, kr)
+    auto cell = [&](uint64_t &n, double &s) {
+        const int L = w > 0 ? __builtin_amdgcn_readfirstlane(bbin[w - 1]) : -1;
+        const int R = __builtin_amdgcn_readfirstlane(bbin[w]);
+        n = (R < a.nb ? bcnt[w] : (uint64_t)a.n) - (w > 0 ? bcnt[w - 1] : 0u);
+        if (L == R) {
+            s = bval[w] - bval[w - 1];
+            return;
         }
-        const float old = a.cent[g * kLmK + k];
-        const float nc = n > 0 ? (float)(s / (double)n) : old;
-        moved[k] = fabsf(nc - old);
-        a.cent[g * kLmK + k] = nc;
+        const int cl = L >= 0 ? L >> 6 : -1, cr = R >> 6;
+        if (L != kl || R != kr) {
+            kl = L;
+            kr = R;
+            double t = 0.0;
+            if (cl == cr) {                            // within one chunk
+                const int b = L + 1 + lane;
+                if (b < R) t = bsum[b];
+            } else {
+                for (int c = cl + 1 + lane; c < cr; c += 64) t += csum[c];
+            }
+            kmid = lm_wave_sum(t);
+        }
+        s = kmid;
+        if (cl != cr) {
+            if (L >= 0) s += btail[w - 1];
+            if (R < a.nb) s += bhead[w];
+        }
+        if (L >= 0) s += bright[w - 1];
+        if (R < a.nb) s += bval[w];
+    };
+    {
+        uint64_t n;
+        double s;
+        cell(n, s);
+        if (lane == 0) cent2[0][w] = (float)(s / (double)a.bs);
     }
     __syncthreads();
-    if (t == 0) {
-        float shift = 0.0f;
-        for (int j = 0; j < kLmK; ++j) shift = fmaxf(shift, moved[j]);
-        a.state[2 * g + 1] += 1;
-        if (shift < a.tol) a.state[2 * g] = 1;
-    }
-}
 
-// Sorted ascending (insertion sort of 16 values) into the output.
-__global__ void lm_final_kernel(LmArgs a) {
-    const int g = blockIdx.y;
-    if (threadIdx.x != 0) return;
-    float c[kLmK];
-    for (int k = 0; k < kLmK; ++k) c[k] = a.cent[g * kLmK + k];
-    for (int i = 1; i < kLmK; ++i) {
-        const float v = c[i];
-        int j = i - 1;
-        while (j >= 0 && c[j] > v) {
-            c[j + 1] = c[j];
-            --j;
+    float pa = NAN, pb = NAN;                          // the pair this wave's boundary was found for
+    int it = 0;
+    for (; it < a.max_iters; ++it) {
+        const float *cent = cent2[it & 1];
+        const float ck = cent[lane & (kLmK - 1)];
+        const float ca = lm_lane(ck, w);
+        const uint32_t rest = (uint32_t)__builtin_amdgcn_ballot_w64(lane < kLmK && lane > w && ck != ca);
+        const float cb = rest ? lm_lane(ck, __builtin_ctz(rest)) : ca;     // next distinct centroid
+        if (w < kLmK - 1 && !(ca == pa && cb == pb)) {
+            pa = ca;
+            pb = cb;
+            if (ca < cb) {
+                const uint32_t key = lm_threshold(ca, cb, lane);
+                const uint32_t m = __builtin_amdgcn_readfirstlane(map[key >> 23]);
+                const uint32_t mask = (1u << (m & 31u)) - 1u;
+                go_to((int)lm_bin(m, key), key & ~mask, (int)(m & 31u));
+                uint64_t c, s;
+                lm_scan_bin(a, B, key & mask, lane, c, s);
+                set_left(c, s);
+            } else if (lane == 0) {
+                bbin[w] = a.nb;
+            }
         }
-        c[j + 1] = v;
+        if (w == kLmK - 1) {
+            // Boundaries decide the codes if the centroids ascend and no
+            // distance to a lower centroid can round to a tie with the
+            // nearest one: gap >= 2 ulp of the largest distance compared.
+            bool bad = false;
+            const float up = __shfl_down(ck, 1);
+            if (lane < kLmK - 1) bad = !(ck <= up);
+            float lower = 0.0f;
+            bool have = false;
+            for (int j = 0; j < kLmK; ++j) {
+                const float c = lm_lane(ck, j);
+                if (lane < kLmK && j < lane && c != ck) { lower = c; have = true; }
+            }
+            float next = fmaxf(xmax, ck);
+            for (int j = kLmK - 1; j >= 0; --j) {
+                const float c = lm_lane(ck, j);
+                if (lane < kLmK && j > lane && c != ck) next = c;
+            }
+            if (lane < kLmK && have) bad = bad || !((ck - lower) >= (next - lower) * 2.384185791015625e-7f);
+            if (lane < kLmK) bad = bad || !(fabsf(ck) <= FLT_MAX) || !(fabsf(xmax - ck) <= FLT_MAX);
+            const bool any = __builtin_amdgcn_ballot_w64(bad) != 0ull;
+            if (lane == 0) {
+                slow = any ? 1 : 0;
+                bbin[w] = a.nb;
+            }
+        }
+        __syncthreads();
+        uint64_t n = 0;
+        double s = 0.0;
+        if (!__builtin_amdgcn_readfirstlane(slow)) {
+            // a centroid equal to the one before it gets no sample (first index)
+            if (w == 0 || lm_lane(ck, w > 0 ? w - 1 : 0) != ca) cell(n, s);
+        } else {
+            // sample by sample, in a fixed order (the places' readers of this
+            // step are past the barrier above)
+            if (tid < kLmSlowSlots) {
+                float c[kLmK];
+#pragma unroll
+                for (int k = 0; k < kLmK; ++k) {
+                    c[k] = cent[k];
+                    ls[k][tid] = 0.0;
+                    lc[k][tid] = 0u;
+                }
+                int64_t o = a.outer > 1 ? tid / a.inner : 0, i = tid - o * a.inner;
+                const int64_t so = a.outer > 1 ? kLmSlowSlots / a.inner : 0, si = kLmSlowSlots - so * a.inner;
+                for (int64_t e = tid; e < a.n; e += kLmSlowSlots) {
+                    const int64_t idx = o * a.outer_stride + (int64_t)g * a.group_stride + i;
+                    float x;
+                    if constexpr (DT == OMNI_F32) x = reinterpret_cast<const float *>(a.x)[idx];
+                    else x = lm_widen<DT>(reinterpret_cast<const uint16_t *>(a.x)[idx]);
+                    int best = 0;
+                    float bd = fabsf(x - c[0]);
+#pragma unroll
+                    for (int k = 1; k < kLmK; ++k) {
+                        const float d = fabsf(x - c[k]);
+                        if (d < bd) {
+                            bd = d;
+                            best = k;
+                        }
+                    }
+                    ls[best][tid] += (double)x;
+                    lc[best][tid] += 1u;
+                    o += so;
+                    i += si;
+                    if (i >= a.inner && a.outer > 1) {
+                        i -= a.inner;
+                        ++o;
+                    }
+                }
+            }
+            __syncthreads();
+            double m = 0.0;
+#pragma unroll
+            for (int q = 0; q < kLmSlowSlots / 64; ++q) {
+                s += ls[w][64 * q + lane];
+                m += (double)lc[w][64 * q + lane];
+            }
+            s = lm_wave_sum(s);
+            n = (uint64_t)lm_wave_sum(m);
+            __syncthreads();
+            load_places();                             // used after the next barrier
+        }
+        const float nc = n > 0 ? (float)(s / (double)n) : ca;
+        if (lane == 0) {
+            moved[w] = fabsf(nc - ca);
+            cent2[(it + 1) & 1][w] = nc;
+        }
+        __syncthreads();
+        const float mv = moved[lane & (kLmK - 1)];
+        if (__builtin_amdgcn_ballot_w64(!(mv < a.tol) && mv == mv) == 0ull) {
+            ++it;
+            break;
+        }
     }
-    for (int k = 0; k < kLmK; ++k) a.out[g * kLmK + k] = c[k];
-}
-
-static int lm_blocks(int64_t n) {
-    const int64_t b = (n + (int64_t)kLmThreads * 8 - 1) / ((int64_t)kLmThreads * 8);
-    return (int)(b < 1 ? 1 : (b > kLmMaxBlocks ? kLmMaxBlocks : b));
+    // sorted ascending
+    if (tid == 0) {
+        float c[kLmK];
+        for (int k = 0; k < kLmK; ++k) c[k] = cent2[it & 1][k];
+        for (int i = 1; i < kLmK; ++i) {
+            const float v = c[i];
+            int j = i - 1;
+            while (j >= 0 && c[j] > v) {
+                c[j + 1] = c[j];
+                --j;
+            }
+            c[j + 1] = v;
+        }
+        for (int k = 0; k < kLmK; ++k) a.out[g * kLmK + k] = c[k];
+        if (a.iters) a.iters[g] = it;
+    }
 }
 
 static size_t align256c(size_t x) { return (x + 255) & ~(size_t)255; }
 
+// Bins by the samples per group: kLmFill samples a bin, or as many as keep
+// 2 n / fill + 512 within kLmMaxBins.
+static void lm_shape(int x_dtype, int64_t n, LmArgs &a) {
+    const int64_t least = (n + (kLmMaxBins - kLmOct) / 2 - 1) / ((kLmMaxBins - kLmOct) / 2);
+    a.fill = least > kLmFill ? least : kLmFill;
+    const int64_t bins = 2 * (n / a.fill) + kLmOct;
+    a.nb = (int)(bins < kLmMaxBins ? (bins + 63) / 64 * 64 : kLmMaxBins);
+    a.nch = a.nb / 64;
+    a.mant = x_dtype == OMNI_F32 ? 23 : (x_dtype == OMNI_BF16 ? 7 : 10);
+    a.wide = n >= (int64_t(1) << 32) ? 1 : 0;
+}
+
 // Workspace carve-up; returns the total bytes (base may be null to size).
-static size_t lm_layout(int groups, int blocks, char *base, LmArgs *a) {
+static size_t lm_layout(int groups, int64_t n, char *base, LmArgs &a) {
     size_t off = 0;
     auto take = [&](size_t bytes) {
         char *p = base ? base + off : nullptr;
         off = align256c(off + bytes);
         return p;
     };
-    char *hist = take((size_t)groups * kLmK * 256 * 4);
-    char *prefix = take((size_t)groups * kLmK * 4);
-    char *krank = take((size_t)groups * kLmK * 8);
-    char *up = take((size_t)groups * (kLmK + 1) * 4);
-    char *psum = take((size_t)groups * blocks * kLmIntervals * 8);
-    char *pcnt = take((size_t)groups * blocks * kLmIntervals * 8);
-    char *cent = take((size_t)groups * kLmK * 4);
-    char *state = take((size_t)groups * 2 * 4);
-    if (a) {
-        a->hist = reinterpret_cast<uint32_t *>(hist);
-        a->prefix = reinterpret_cast<uint32_t *>(prefix);
-        a->krank = reinterpret_cast<int64_t *>(krank);
-        a->uprefix = reinterpret_cast<uint32_t *>(up);
-        a->psum = reinterpret_cast<double *>(psum);
-        a->pcnt = reinterpret_cast<uint64_t *>(pcnt);
-        a->cent = reinterpret_cast<float *>(cent);
-        a->state = reinterpret_cast<int *>(state);
-    }
+    const size_t gr = (size_t)groups;
+    a.oct = reinterpret_cast<uint32_t *>(take(gr * kLmOct * 4));
+    a.map = reinterpret_cast<uint32_t *>(take(gr * kLmOct * 4));
+    a.cnt = reinterpret_cast<uint32_t *>(take(gr * a.nb * 4));
+    a.cursor = reinterpret_cast<uint32_t *>(take(gr * a.nb * 4));
+    a.start = reinterpret_cast<uint64_t *>(take(gr * (a.nb + 1) * 8));
+    a.bsum = reinterpret_cast<double *>(take(gr * a.nb * 8));
+    a.csum = reinterpret_cast<double *>(take(gr * a.nch * 8));
+    a.buf = reinterpret_cast<float *>(take(gr * (size_t)n * 4));
     return off;
 }
 
 template <int DT>
 static void lm_launch(const LmArgs &a, int groups, hipStream_t st) {
-    const dim3 grid(a.blocks, groups), one(1, groups);
-    hipLaunchKernelGGL(lm_clear_kernel, one, dim3(256), 0, st, a);
-    for (int pass = 0; pass < 4; ++pass) {
-        hipLaunchKernelGGL((lm_radix_kernel<DT>), grid, dim3(kLmThreads), 0, st, a, pass);
-        hipLaunchKernelGGL(lm_select_kernel, one, dim3(256), 0, st, a);
-    }
-    hipLaunchKernelGGL((lm_interval_kernel<DT>), grid, dim3(kLmThreads), 0, st, a);
-    hipLaunchKernelGGL(lm_init_kernel, one, dim3(256), 0, st, a);
-    for (int it = 0; it < a.max_iters; ++it) {
-        hipLaunchKernelGGL((lm_assign_kernel<DT>), grid, dim3(kLmThreads), 0, st, a);
-        hipLaunchKernelGGL(lm_update_kernel, one, dim3(256), 0, st, a);
-    }
-    hipLaunchKernelGGL(lm_final_kernel, one, dim3(64), 0, st, a);
-}
-
-__global__ void lm_iters_kernel(const int *state, int groups, int32_t *iters) {
-    const int g = blockIdx.x * blockDim.x + threadIdx.x;
-    if (g < groups) iters[g] = state[2 * g + 1];
+    const unsigned gr = (unsigned)groups;
+    const dim3 grid((unsigned)((a.n + kLmBlock - 1) / kLmBlock), gr), block(kLmThreads);
+    const int clear = a.nb > kLmOct ? a.nb : kLmOct;
+    hipLaunchKernelGGL(lm_clear_kernel, dim3((unsigned)((clear + 255) / 256), gr), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((lm_oct_kernel<DT>), grid, block, 0, st, a);
+    hipLaunchKernelGGL(lm_map_kernel, dim3(gr), dim3(kLmOct), 0, st, a);
+    hipLaunchKernelGGL((lm_count_kernel<DT>), grid, block, 0, st, a);
+    hipLaunchKernelGGL(lm_scan_kernel, dim3((unsigned)((a.nb + kLmScan - 1) / kLmScan), gr), block, 0, st, a);
+    hipLaunchKernelGGL((lm_store_kernel<DT>), grid, block, 0, st, a);
+    hipLaunchKernelGGL(lm_binsum_kernel, dim3((unsigned)((a.n + 4095) / 4096), gr), dim3(256), 0, st, a);
+    hipLaunchKernelGGL(lm_chunk_kernel, dim3((unsigned)((a.nch + 15) / 16), gr), block, 0, st, a);
+    hipLaunchKernelGGL((lm_lloyd_kernel<DT>), dim3(gr), block, 0, st, a);
 }
 
 }  // namespace omni
@@ -493,8 +931,10 @@ __global__ void lm_iters_kernel(const int *state, int groups, int32_t *iters) {
 using namespace omni;
 
 extern "C" size_t omni_lloyd_max_workspace_size(int n_groups, int64_t outer, int64_t inner) {
-    if (n_groups <= 0 || outer <= 0 || inner <= 0) return 0;
-    return lm_layout(n_groups, lm_blocks(outer * inner), nullptr, nullptr);
+    if (n_groups <= 0 || outer <= 0 || inner <= 0 || outer > INT64_MAX / inner) return 0;
+    LmArgs a;
+    lm_shape(OMNI_F32, outer * inner, a);
+    return lm_layout(n_groups, outer * inner, nullptr, a);
 }
 
 extern "C" int omni_lloyd_max(const void *x, int x_dtype, int n_groups, int64_t outer, int64_t inner,
@@ -515,22 +955,24 @@ extern "C" int omni_lloyd_max(const void *x, int x_dtype, int n_groups, int64_t 
     a.outer = outer; a.inner = inner; a.outer_stride = outer_stride; a.group_stride = group_stride;
     a.n = n;
     a.bs = n / kLmK;
-    a.blocks = lm_blocks(n);
     a.max_iters = max_iters;
     a.tol = tol;
     a.out = codebooks;
-    const size_t need = lm_layout(n_groups, a.blocks, nullptr, nullptr);
+    a.iters = iters_out;
+    lm_shape(x_dtype, n, a);
+    // 4-element loads: every run of four lies in one row and is aligned
+    a.vec = (inner % 4 == 0 && outer_stride % 4 == 0 && group_stride % 4 == 0 &&
+             (uintptr_t)x % (4 * dtype_size(x_dtype)) == 0) ? 1 : 0;
+    const size_t need = omni_lloyd_max_workspace_size(n_groups, outer, inner);
     if (workspace == nullptr || workspace_bytes < need) {
         set_error("omni_lloyd_max: workspace of %zu bytes required, %zu given", need, workspace_bytes);
         return OMNI_EWORKSPACE;
     }
-    lm_layout(n_groups, a.blocks, reinterpret_cast<char *>(workspace), &a);
+    lm_layout(n_groups, n, reinterpret_cast<char *>(workspace), a);
     hipStream_t st = as_stream(stream);
     if (x_dtype == OMNI_F32) lm_launch<OMNI_F32>(a, n_groups, st);
     else if (x_dtype == OMNI_BF16) lm_launch<OMNI_BF16>(a, n_groups, st);
     else lm_launch<OMNI_F16>(a, n_groups, st);
-    if (iters_out) hipLaunchKernelGGL(lm_iters_kernel, dim3((n_groups + 63) / 64), dim3(64), 0, st, a.state, n_groups,
-                                      iters_out);
     OMNI_CHECK_LAUNCH("omni_lloyd_max");
     return OMNI_OK;
 }

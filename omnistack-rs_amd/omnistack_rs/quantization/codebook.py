@@ -8,8 +8,9 @@ assignment (first index on ties), per-cell mean update (empty cells keep
 their centroid), stop when the largest centroid move is below the tolerance;
 the result is sorted ascending.
 
-Samples on a HIP device run ``omni_lloyd_max`` (csrc/calib.hip: radix-select
-initialisation, one pass per Lloyd step, fp64 cell sums in a fixed order);
+Samples on a HIP device run ``omni_lloyd_max`` (csrc/calib.hip: samples
+stored by bins of their value once, every Lloyd step from the bins, fp64 cell
+sums in a fixed order);
 ``calibrate_heads`` calibrates every head of a (B, H, T, D) cache in one
 call without copying the per-head samples.  CPU samples run the same recipe
 with torch on the CPU, as the reference does.  Either way cell means are not

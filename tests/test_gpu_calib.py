@@ -135,3 +135,60 @@ def test_calibrate_heads_16bit_and_d32_bake(device, tmp_path):
     r_nib, _, _ = restate.quantize_heads(restate.wht(kv), cb, user_id=3)
     assert torch.equal(nib, r_nib)
     assert stats["seq_len"] == 30 and stats["n_kv_heads"] == 2
+
+
+def _step(x: torch.Tensor, c: torch.Tensor) -> torch.Tensor:
+    """One Lloyd step by its definition: first-index argmin of the fp32
+    distances, correctly rounded means (math.fsum), empty cells kept."""
+    out = c.clone()
+    code = torch.empty(x.numel(), dtype=torch.int64)
+    for s in range(0, x.numel(), 1 << 18):
+        code[s:s + (1 << 18)] = (x[s:s + (1 << 18), None] - c[None, :]).abs().argmin(dim=1)
+    for k in range(16):
+        m = x[code == k].double().numpy()
+        if m.size:
+            out[k] = float(np.float32(math.fsum(m) / m.size))
+    return out
+
+
+@pytest.mark.parametrize("kind", ["n16", "n17", "one_run", "run_plus_1", "odd_rows", "full_bins", "zeros", "outliers",
+                                  "close_levels", "tiny", "bf16_large", "f16"])
+def test_steps_match_their_definition(device, kind):
+    """Steps 1, 2 and 3 from the library's own initial centroids, at the edges
+    of the binned passes: the smallest groups, a block's run of 32768 samples
+    and one more, rows that are no multiple of four, bins with more samples
+    than a wave keeps in registers, values so far out or levels so close that
+    distances to several centroids round to a tie (samples one by one),
+    denormals, 16-bit types (one value per bin)."""
+    g = _data.gen(450)
+    n = {"n16": 16, "n17": 17, "one_run": 32768, "run_plus_1": 32769, "odd_rows": 3 * 4099}.get(kind, 50000)
+    x = torch.randn(n, generator=g)
+    if kind == "full_bins":
+        x[: 3 * n // 4] = 1.0 + torch.rand(3 * n // 4, generator=g) * 2.0 ** -14     # one narrow bump
+    elif kind == "zeros":
+        x[torch.rand(n, generator=g) < 0.7] = 0.0
+        x[5] = -0.0
+    elif kind == "outliers":
+        x[:4000] *= 1e30
+    elif kind == "close_levels":
+        x = 1.0 + torch.randint(0, 20, (n,), generator=g) * 2.0 ** -23
+    elif kind == "tiny":
+        x *= 1e-39
+    elif kind == "bf16_large":
+        x = torch.randn(200003, generator=g).to(torch.bfloat16)
+    elif kind == "f16":
+        x = x.to(torch.float16)
+    from omnistack_rs.quantization.codebook import _lloyd_max_hip
+    if kind == "odd_rows":                         # 3 rows of 4099 in a wider array, 2 groups
+        wide = torch.randn(3, 2, 4099 + 2, generator=g)
+        wide[:, 1, :4099] = x.reshape(3, 4099)
+        args = (wide.to(device), 2, 3, 4099, 2 * 4101, 4101)
+    else:
+        args = (x.to(device), 1, 1, x.numel(), 0, 0)
+    print(f"[calib] steps {kind} n={x.numel()}", flush=True)
+    c = _lloyd_max_hip(*args, 0, 1e-6)[0][-1].cpu()
+    for it in (1, 2, 3):
+        got, done = _lloyd_max_hip(*args, it, 0.0)
+        c = _step(x.float(), c)
+        assert int(done[-1]) == it
+        assert torch.equal(got[-1].cpu(), c.sort().values), f"{kind} step {it}"
