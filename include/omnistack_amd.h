@@ -114,7 +114,7 @@ size_t omni_encode_workspace_size(int64_t B, int H, int64_t T, int head_dim, int
  *     (same dtype and shape, same G and codebooks) into their own outputs.
  *     16-bit inputs at head_dim 128 with B * T >= 64 read the prebuilt
  *     `tables` (OMNI_EWORKSPACE when missing or short) in one launch; other
- *     inputs take the lane-per-row kernel (tables unused, may be NULL).
+ *     inputs need no tables (unused, may be NULL).
  */
 size_t omni_encode_tables_size(int H, int per_head_codebook);
 int omni_encode_build_tables(const float *codebooks, int per_head_codebook, int H, int x_dtype,

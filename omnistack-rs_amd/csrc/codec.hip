@@ -15,7 +15,6 @@
 namespace omni {
 
 constexpr int kRowsPerBlock = 256;
-constexpr int kProjGroup = 4;   // QJL projections accumulated together per pass
 
 // In-register normalized WHT of one row, reference butterfly order:
 // h = 1, 2, ..., D/2; (upper, lower) -> (upper + lower, upper - lower).
@@ -87,152 +86,6 @@ __global__ __launch_bounds__(kRowsPerBlock) void wht_kernel(const void *x, int d
     for (int d = 0; d < D; ++d) store_from_f32(out, dtype, row * D + d, v[d]);
 }
 
-// ── omni_encode ─────────────────────────────────────────────────────────
-//
-// One lane per row; a block covers up to 256 rows of one (b, h), so the
-// head's codebook and G are uniform across the block (scalar loads).
-
-// Exact sign of sum_j s_j e_j (s_j = +-1 from the G row bits) by fp64
-// Neumaier summation, for the rare projections whose fp32 sum is within its
-// rounding bound of zero.  Inlined and fully unrolled so the residual row
-// stays in registers (a call would force the whole row to scratch).
-template <int D>
-__device__ __forceinline__ bool exact_sign_nonneg(const float (&e)[D], const uint32_t *grow) {
-    double s = 0.0, c = 0.0;
-#pragma unroll
-    for (int w = 0; w < D / 32; ++w) {
-        const uint32_t gw = grow[w];
-#pragma unroll
-        for (int jj = 0; jj < 32; ++jj) {
-            double y = (double)e[32 * w + jj];
-            y = ((gw >> jj) & 1u) ? y : -y;
-            const double t = s + y;
-            c += (fabs(s) >= fabs(y)) ? ((s - t) + y) : ((y - t) + s);
-            s = t;
-        }
-    }
-    return (s + c) >= 0.0;
-}
-
-template <int D>
-__global__ __launch_bounds__(kRowsPerBlock) void encode_kernel(
-    const void *x, int dtype, int64_t T, int H, int rotate, const int8_t *sign_flip,
-    const float *codebooks, int per_head, const uint32_t *g_bits,
-    uint8_t *nibbles, uint8_t *qjl, float *norms, float scale) {
-    constexpr int QD = D / 2;       // QJL projections per row
-    constexpr int W = D / 32;       // G words per projection row
-    const int h = blockIdx.y;
-    const int64_t b = blockIdx.z;
-    const int64_t t = (int64_t)blockIdx.x * kRowsPerBlock + threadIdx.x;
-    if (t >= T) return;
-    const int64_t row = (b * H + h) * T + t;
-
-    float v[D];
-    load_row<D>(x, dtype, row, v);
-    if (rotate) rotate_row<D>(v, dtype, sign_flip, scale);
-
-    const float *cbp = codebooks + (per_head ? h * 16 : 0);
-    float cb[16];
-    bool cb_nan = false;
-#pragma unroll
-    for (int k = 0; k < 16; ++k) { cb[k] = cbp[k]; cb_nan |= (cb[k] != cb[k]); }
-
-    // Nearest centroid: fp32 |x - c_k|, strictly smaller wins (first index
-    // on ties).  A NaN distance is the minimum (torch.argmin); that only
-    // matters when the codebook itself holds a NaN: a NaN x gives NaN for
-    // every k and keeps code 0 either way.
-    uint32_t packed[D / 8];
-#pragma unroll
-    for (int w = 0; w < D / 8; ++w) packed[w] = 0u;
-#pragma unroll
-    for (int d = 0; d < D; ++d) {
-        float best = fabsf(v[d] - cb[0]);
-        int code = 0;
-        float cval = cb[0];
-#pragma unroll
-        for (int k = 1; k < 16; ++k) {
-            float dk = fabsf(v[d] - cb[k]);
-            bool take = dk < best;
-            if (cb_nan) take = take || ((dk != dk) && (best == best));
-            best = take ? dk : best;
-            code = take ? k : code;
-            cval = take ? cb[k] : cval;
-        }
-        packed[d >> 3] |= (uint32_t)code << (4 * (d & 7));
-        v[d] = v[d] - cval;  // residual e_d (fp32), quantize.py:580
-    }
-
-    // ||e||_2: the exact squares (fp32 x fp32 fits fp64) summed in fp64 and
-    // rounded once; a sum beyond the fp32 range is +inf, where the
-    // reference's fp32 accumulation overflows.
-    double ss = 0.0;
-    float abs_sum = 0.0f;
-#pragma unroll
-    for (int d = 0; d < D; ++d) {
-        const double ed = (double)v[d];
-        ss = __builtin_fma(ed, ed, ss);
-        abs_sum += fabsf(v[d]);
-    }
-    const float nrm = ss > 3.4028234663852886e38 ? INFINITY : (float)sqrt(ss);
-
-    // QJL signs.  fp32 sequential sums carry |err| <= (D-1) u sum|e_j|; a
-    // result farther than D * 2^-24 * abs_sum from zero has a certain sign,
-    // anything closer is recomputed exactly.  Non-finite rows take the fp32
-    // result's (deterministic) sign like the reference's BLAS does.
-    const float bound = abs_sum * ((float)D * 5.9604644775390625e-8f);
-    const bool finite_row = isfinite(abs_sum);
-    const uint32_t *gh = g_bits + (int64_t)h * QD * W;
-    uint32_t sbits[QD / 32 > 0 ? QD / 32 : 1];
-#pragma unroll
-    for (int k = 0; k < (QD / 32 > 0 ? QD / 32 : 1); ++k) sbits[k] = 0u;
-#pragma unroll 1
-    for (int i0 = 0; i0 < QD; i0 += kProjGroup) {
-        float acc[kProjGroup];
-#pragma unroll
-        for (int ii = 0; ii < kProjGroup; ++ii) acc[ii] = 0.0f;
-#pragma unroll
-        for (int w = 0; w < W; ++w) {
-            uint32_t gw[kProjGroup];
-#pragma unroll
-            for (int ii = 0; ii < kProjGroup; ++ii) gw[ii] = gh[(i0 + ii) * W + w];
-#pragma unroll
-            for (int jj = 0; jj < 32; ++jj) {
-#pragma unroll
-                for (int ii = 0; ii < kProjGroup; ++ii) {
-                    float s = ((gw[ii] >> jj) & 1u) ? 1.0f : -1.0f;
-                    acc[ii] = __builtin_fmaf(s, v[32 * w + jj], acc[ii]);
-                }
-            }
-        }
-        uint32_t unc = 0u;
-#pragma unroll
-        for (int ii = 0; ii < kProjGroup; ++ii) {
-            const int i = i0 + ii;
-            if (finite_row && !(fabsf(acc[ii]) > bound)) unc |= 1u << ii;
-            sbits[i >> 5] |= (uint32_t)(acc[ii] >= 0.0f) << (i & 31);
-        }
-        while (unc) {
-            const int ii = __builtin_ctz(unc);
-            unc &= unc - 1u;
-            const int i = i0 + ii;
-            const bool bit = exact_sign_nonneg<D>(v, gh + i * W);
-            sbits[i >> 5] = (sbits[i >> 5] & ~(1u << (i & 31))) | ((uint32_t)bit << (i & 31));
-        }
-    }
-
-    // Stores: nibbles (D/2 B), signs (D/16 B), norm.
-    if constexpr (D == 128) {
-        uint4 *np = reinterpret_cast<uint4 *>(nibbles + row * (D / 2));
-#pragma unroll
-        for (int k = 0; k < 4; ++k) np[k] = make_uint4(packed[4 * k], packed[4 * k + 1], packed[4 * k + 2], packed[4 * k + 3]);
-        reinterpret_cast<uint2 *>(qjl + row * (D / 16))[0] = make_uint2(sbits[0], sbits[1]);
-    } else {
-        reinterpret_cast<uint4 *>(nibbles + row * (D / 2))[0] = make_uint4(packed[0], packed[1], packed[2], packed[3]);
-        reinterpret_cast<uint16_t *>(qjl + row * (D / 16))[0] = (uint16_t)(sbits[0] & 0xffffu);
-    }
-    norms[row] = nrm;
-}
-
 typedef float float4_t __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ uint32_t cvt_pk_f16(float x, float y) {
@@ -241,9 +94,17 @@ __device__ __forceinline__ uint32_t cvt_pk_f16(float x, float y) {
     return __builtin_bit_cast(uint32_t, __builtin_convertvector((f2_t){x, y}, h2_t));
 }
 
-// ── fast encoder: 16-bit input, D = 128 ─────────────────────────────────
+// ── omni_encode ─────────────────────────────────────────────────────────
 //
-// Same contract as encode_kernel, organised for gfx950:
+// Two wave kernels: encode128_kernel (16-bit input, D = 128: codes from a
+// table of all values) and encode_grid_kernel (the rest).  For each row
+//   code_d = argmin_k fp32 |x_d - c_k|, first index on ties; a NaN distance
+//            is the minimum (torch.argmin), which only matters when the
+//            codebook itself holds a NaN
+//   e = x - c[code] (fp32), norm = ||e||_2, bit_i = [G_i . e >= 0]
+//
+// ── 16-bit input, D = 128 ───────────────────────────────────────────────
+//
 //   * 16 rows per wave-iteration; lane (n, g) holds elements 32 s + 8 g + i
 //     (s < 4, i < 8) of row n.  The WHT runs in registers (h = 1, 2, 4, 32,
 //     64) and by paired v_permlane16/32_swap butterflies (h = 8, 16), in the
@@ -295,6 +156,8 @@ struct EncArgs {
     const int32_t *page_table, *positions;
     int64_t max_pages, n_pages;
     int page_shift;
+    // encode_grid_kernel: rows between a wave's groups as (batch entries, tokens)
+    int64_t step_b, step_t;
 };
 
 template <int XDT>
@@ -806,6 +669,511 @@ __global__ __launch_bounds__(64 * kEncWaves) void encode128_kernel(EncArgs a) {
     }
 }
 
+// ── wave encoder without a value table: f32 input, D = 32 ───────────────
+//
+// The contract and the matrix-core projections of encode128_kernel for the
+// inputs whose codes no table of all values can give (f32) or that are too
+// short for one (D = 32).  Lane (n, g) holds 32 values as x[s][i]: elements
+// 32 s + 8 g + i of row n (D = 128, 16 rows per wave iteration), or elements
+// 8 g + i of row 16 s + n (D = 32, 64 rows).
+//   * Codes: the values from c_0 - r to c_15 + 7 r (r = c_15 - c_0) fall into
+//     1023 equal cells, and a byte table in LDS, built by each block, names
+//     the lower of the two adjacent codes that a cell's values can take (the
+//     codes at its edges, one percent of a cell further out, differ by at most
+//     one, and codes ascend with the value).  Both fp32 distances then decide,
+//     first index on ties.  Cells with more boundaries, values beyond the last
+//     cell, and codebooks that do not ascend by more than a rounding error of
+//     the distances compared point at a NaN centroid: such a group of rows is
+//     coded again over all 16 centroids.
+//   * Bound by VALU issue, as encode128_kernel.  K and V of 16 x 4096 tokens,
+//     8 heads, with a lane per row and 16 distances per value before: f32 at
+//     D = 128 3851 -> 176 us (3.5 TB/s), bf16 at D = 32 595 -> 86 us; one
+//     token of one sequence 385 -> 10 us.  On 16-bit rows at D = 128 the value
+//     table is the better of the two where it is built already (146 against
+//     197 us; equal below 1000 rows per head).
+
+constexpr int kEgWaves = 4;
+constexpr int kEgCells = 1024;                        // the last one: values past the grid
+constexpr float kEgBelow = 1.0f, kEgAbove = 7.0f;     // the grid's reach past the centroids, in r
+
+template <int D>
+struct EgLds {
+    static constexpr int S = D == 128 ? 4 : 1;        // chunks of a row
+    static constexpr int CB = D == 128 ? 4 : 1;       // blocks of 16 projections
+    uint8_t cell[kEgCells];                           // 4 * lower code (64: none)
+    float cent[20];                                   // 16..19: NaN
+    uint4 gimg[CB * S * 64];                          // [cb][s][lane]: 8 bf16 +-1 of G
+    uint32_t gbits[(D / 2) * (D / 32)];
+    uint32_t flip[D];                                 // sign-bit xor of each element
+    float stage[kEgWaves][D];                         // one residual row (rare paths)
+};
+
+// sum_j s_j e_j over one staged residual row of D floats (wave_row_dot for
+// any D).
+template <int D>
+__device__ __forceinline__ double eg_row_dot(const float *st, const uint32_t *grow, int lane, uint32_t &fl) {
+    if constexpr (D == 128) {
+        return wave_row_dot(st, grow, lane, fl);
+    } else {
+        float f = 0.0f;
+        if (lane < 32) f = ((grow[0] >> lane) & 1u) ? st[lane] : -st[lane];
+        const uint32_t cls = (f != f) ? 1u : (f == INFINITY ? 2u : (f == -INFINITY ? 4u : 0u));
+        fl = (__builtin_amdgcn_ballot_w64((cls & 1u) != 0u) ? 1u : 0u) | (__builtin_amdgcn_ballot_w64((cls & 2u) != 0u) ? 2u : 0u) |
+             (__builtin_amdgcn_ballot_w64((cls & 4u) != 0u) ? 4u : 0u);
+        double s = (double)f, c = 0.0;
+#pragma unroll
+        for (int m = 32; m >= 1; m >>= 1) {
+            const double so = __shfl_xor(s, m), co = __shfl_xor(c, m);
+            const double t = s + so;
+            const double bp = t - s;
+            const double err = (s - (t - bp)) + (so - bp);
+            s = t;
+            c = (c + co) + err;
+        }
+        return s + c;
+    }
+}
+
+// First-index argmin of the fp32 distances (no NaN).
+__device__ __forceinline__ int eg_code(float x, const float (&cb)[16]) {
+    float best = fabsf(x - cb[0]);
+    int code = 0;
+#pragma unroll
+    for (int k = 1; k < 16; ++k) {
+        const float d = fabsf(x - cb[k]);
+        code = d < best ? k : code;
+        best = fminf(best, d);
+    }
+    return code;
+}
+
+template <int XDT, int D, bool ROT>
+__global__ __launch_bounds__(64 * kEgWaves, D == 128 ? 3 : 2) void encode_grid_kernel(EncArgs a) {
+    using L = EgLds<D>;
+    constexpr int S = L::S, CB = L::CB;
+    constexpr int kGroup = D == 128 ? 16 : 64;        // rows per wave iteration
+    constexpr int QD = D / 2, W = D / 32;
+    __shared__ __attribute__((aligned(16))) L sm;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n = lane & 15, g = lane >> 4;
+    const int h = blockIdx.y, zb = blockIdx.z;
+    const int64_t rpb = a.rows_per_block[zb];
+    const int64_t v_begin = (int64_t)blockIdx.x * rpb;
+    if (v_begin >= a.nrows_head) return;               // block-uniform, before any barrier
+    const int64_t v_end = v_begin + rpb < a.nrows_head ? v_begin + rpb : a.nrows_head;
+    const void *const xz = a.x[zb];
+    uint8_t *const nibz = a.nibbles[zb];
+    uint8_t *const qjlz = a.qjl[zb];
+    float *const nrmz = a.norms[zb];
+
+    // ── prologue: centroids, cells, G images, sign flips ─────────────
+    const float *cbp = a.codebooks + (a.per_head ? h * 16 : 0);
+    const uint32_t *gh = a.g_bits + (int64_t)h * QD * W;
+    if (tid < 20) sm.cent[tid] = tid < 16 ? cbp[tid] : __builtin_nanf("");
+    for (int k = tid; k < QD * W; k += 64 * kEgWaves) sm.gbits[k] = gh[k];
+    for (int d = tid; d < D; d += 64 * kEgWaves) sm.flip[d] = (ROT && a.sign_flip && a.sign_flip[d] < 0) ? 0x80000000u : 0u;
+    for (int m = tid; m < CB * S * 64; m += 64 * kEgWaves) {
+        const int cb = m / (S * 64), s = (m / 64) % S, l = m & 63;
+        const uint32_t byte = (gh[(16 * cb + (l & 15)) * W + s] >> (8 * (l >> 4))) & 0xffu;
+        uint32_t w[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            w[k] = (((byte >> (2 * k)) & 1u) ? 0x3F80u : 0xBF80u) | ((((byte >> (2 * k + 1)) & 1u) ? 0x3F80u : 0xBF80u) << 16);
+        sm.gimg[m] = make_uint4(w[0], w[1], w[2], w[3]);
+    }
+    __syncthreads();
+    const float c0 = sm.cent[0], r = sm.cent[15] - c0;
+    const float g_lo = c0 - kEgBelow * r, g_hi = sm.cent[15] + kEgAbove * r;
+    const float inv = (float)(kEgCells - 1) / (g_hi - g_lo), off = -g_lo * inv;
+    float cb[16];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) cb[k] = sm.cent[k];
+    // ascending, and no distance to a lower centroid can round to a tie with
+    // the nearest one anywhere on the grid: gap >= 2 ulp of it (lane k: the
+    // gap of centroids k and k + 1)
+    const float lo = sm.cent[n < 15 ? n : 14], hi = sm.cent[n < 15 ? n + 1 : 15];
+    float next = g_hi;
+#pragma unroll
+    for (int j = 15; j > 0; --j) next = cb[j] > hi ? cb[j] : next;
+    const bool good = lo == hi || (lo < hi && hi - lo >= (next - lo) * 2.384185791015625e-7f);
+    const bool grid_ok = __builtin_amdgcn_ballot_w64(!good) == 0ull && r > 0.0f && inv > 1e-30f && inv < 1e30f &&
+                         fabsf(g_lo) < 1e30f && fabsf(g_hi) < 1e30f;
+    const double width = 1.0 / (double)inv;
+    for (int c = tid; c < kEgCells; c += 64 * kEgWaves) {
+        int code = 16;
+        if (grid_ok && c < kEgCells - 1) {
+            const float x0 = (float)(((double)c - 0.01 - (double)off) * width);
+            const float x1 = (float)(((double)c + 1.01 - (double)off) * width);
+            const int k0 = c == 0 ? 0 : eg_code(x0, cb), k1 = eg_code(x1, cb);
+            if (k1 >= k0 && k1 - k0 <= 1) code = k0 < 14 ? k0 : 14;
+        }
+        sm.cell[c] = (uint8_t)(4 * code);
+    }
+    __syncthreads();
+    const char *cent_b = reinterpret_cast<const char *>(sm.cent);
+
+    // (vb, vt): batch entry and token of the first row of the wave's group;
+    // groups of a wave lie kEgWaves * kGroup rows apart = (step_b, step_t)
+    int64_t vcur = v_begin + kGroup * wave;
+    if (vcur >= v_end) return;                         // no barrier follows
+    int64_t vb = vcur / a.T, vt = vcur - vb * a.T;
+    constexpr int kSets = D == 128 ? 1 : 4;            // 16-row sets of a group
+    auto rows_of = [&](int64_t (&row)[kSets], int64_t v, int64_t b0, int64_t t0) {
+#pragma unroll
+        for (int q = 0; q < kSets; ++q) {
+            const int64_t left = v_end - 1 - v;
+            int64_t b = b0, t = t0 + (16 * q + n < left ? (int64_t)(16 * q + n) : left);
+            while (t >= a.T) {
+                t -= a.T;
+                ++b;
+            }
+            row[q] = (b * a.H + h) * a.T + t;
+        }
+    };
+    constexpr int kRaw = XDT == OMNI_F32 ? 2 : 1;      // 16-byte loads of a chunk
+    auto load = [&](uint4 (&raw)[4][kRaw], const int64_t (&row)[kSets]) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const int64_t e = row[D == 128 ? 0 : s] * D + (D == 128 ? 32 * s : 0) + 8 * g;
+            if constexpr (XDT == OMNI_F32) {
+                const uint4 *p = reinterpret_cast<const uint4 *>(reinterpret_cast<const float *>(xz) + e);
+                raw[s][0] = p[0];
+                raw[s][1] = p[1];
+            } else {
+                raw[s][0] = *reinterpret_cast<const uint4 *>(reinterpret_cast<const uint16_t *>(xz) + e);
+            }
+        }
+    };
+    auto encode = [&](float (&x)[4][8], const int64_t (&row)[kSets], const int64_t v0) {
+        if (ROT) {
+#pragma unroll
+            for (int hh = 1; hh < 8; hh <<= 1)
+#pragma unroll
+                for (int s = 0; s < 4; ++s)
+#pragma unroll
+                    for (int i = 0; i < 8; ++i)
+                        if (!(i & hh)) {
+                            const float u = x[s][i], l = x[s][i + hh];
+                            x[s][i] = u + l;
+                            x[s][i + hh] = u - l;
+                        }
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+#pragma unroll
+                for (int i = 0; i < 8; i += 2) xlane_pair_butterfly<16>(x[s][i], x[s][i + 1]);
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+#pragma unroll
+                for (int i = 0; i < 8; i += 2) xlane_pair_butterfly<32>(x[s][i], x[s][i + 1]);
+            if constexpr (D == 128) {
+#pragma unroll
+                for (int hs = 1; hs < 4; hs <<= 1)
+#pragma unroll
+                    for (int s = 0; s < 4; ++s)
+                        if (!(s & hs))
+#pragma unroll
+                            for (int i = 0; i < 8; ++i) {
+                                const float u = x[s][i], l = x[s + hs][i];
+                                x[s][i] = u + l;
+                                x[s + hs][i] = u - l;
+                            }
+            }
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    float p = x[s][i] * a.scale;
+                    // the product is rounded to fp32 before it is rounded to
+                    // f16 (v_fma_mixlo_f16 would round once)
+                    if (XDT == OMNI_F16) asm volatile("" : "+v"(p));
+                    x[s][i] = round_to_dtype(p, XDT);
+                }
+        }
+        // codes and residuals: the cell's two candidates
+        float e[4][8];
+        uint32_t nib[4];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            uint32_t cell[8], wn = 0u;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const float t = __builtin_amdgcn_fmed3f(__builtin_fmaf(x[s][i], inv, off), 0.0f, (float)(kEgCells - 1));
+                cell[i] = sm.cell[(uint32_t)t];
+            }
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const float *c = reinterpret_cast<const float *>(cent_b + cell[i]);
+                const float e0 = x[s][i] - c[0], e1 = x[s][i] - c[1];
+                const bool up = fabsf(e1) < fabsf(e0);
+                e[s][i] = up ? e1 : e0;
+                wn += ((cell[i] >> 2) + (up ? 1u : 0u)) << (4 * i);
+            }
+            nib[s] = wn;
+        }
+        // per chunk: sum |e| over the row's four lanes (and chunks, D = 128);
+        // not finite where a value's cell names no code, or by itself
+        float as[kSets];
+        auto abs_sums = [&]() {
+            float p[4];
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                p[s] = 0.0f;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) p[s] += fabsf(e[s][i]);
+            }
+            if constexpr (D == 128) {
+                as[0] = xlane_sum_f32((p[0] + p[1]) + (p[2] + p[3]));
+            } else {
+#pragma unroll
+                for (int s = 0; s < 4; ++s) as[s] = xlane_sum_f32(p[s]);
+            }
+        };
+        abs_sums();
+        bool odd = false;
+#pragma unroll
+        for (int q = 0; q < kSets; ++q) odd = odd || !(as[q] < 0x1p127f);
+        if (__builtin_amdgcn_ballot_w64(odd)) {
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                nib[s] = 0u;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) e[s][i] = x[s][i] - sm.cent[0];
+            }
+#pragma unroll 1
+            for (int k = 1; k < 16; ++k) {
+                const float c = sm.cent[k];
+#pragma unroll
+                for (int s = 0; s < 4; ++s)
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) {
+                        const float d = x[s][i] - c;
+                        const bool take = fabsf(d) < fabsf(e[s][i]) || (d != d && e[s][i] == e[s][i]);
+                        e[s][i] = take ? d : e[s][i];
+                        nib[s] = take ? ((nib[s] & ~(15u << (4 * i))) | ((uint32_t)k << (4 * i))) : nib[s];
+                    }
+            }
+            abs_sums();
+        }
+        // norms: fp64 sums of the exact squares
+        double ss[kSets];
+        {
+            double p[4];
+#pragma unroll
+            for (int s = 0; s < 4; ++s) p[s] = 0.0;
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+#pragma unroll
+                for (int s = 0; s < 4; ++s) {
+                    const double ed = (double)e[s][i];
+                    p[s] = __builtin_fma(ed, ed, p[s]);
+                }
+            if constexpr (D == 128) {
+                ss[0] = xlane_sum_f64<32>(xlane_sum_f64<16>((p[0] + p[1]) + (p[2] + p[3])));
+            } else {
+#pragma unroll
+                for (int s = 0; s < 4; ++s) ss[s] = xlane_sum_f64<32>(xlane_sum_f64<16>(p[s]));
+            }
+        }
+        // projections as in encode128_kernel: two bf16 parts of each residual,
+        // G exact; D = 128: acc[cb] over the chunks, D = 32: acc[s] per set
+        float4_t acc[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) acc[q] = float4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            uint32_t ph[4], pm[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                typedef __bf16 bf2_t __attribute__((ext_vector_type(2)));
+                typedef float f2_t __attribute__((ext_vector_type(2)));
+                const float e0 = e[s][2 * j], e1 = e[s][2 * j + 1];
+                const uint32_t hp = __builtin_bit_cast(uint32_t, __builtin_convertvector((f2_t){e0, e1}, bf2_t));
+                const float r0 = e0 - __uint_as_float(hp << 16);
+                const float r1 = e1 - __uint_as_float(hp & 0xffff0000u);
+                ph[j] = hp;
+                pm[j] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f2_t){r0, r1}, bf2_t));
+            }
+            const bf16x8_t bh = __builtin_bit_cast(bf16x8_t, make_uint4(ph[0], ph[1], ph[2], ph[3]));
+            const bf16x8_t bm = __builtin_bit_cast(bf16x8_t, make_uint4(pm[0], pm[1], pm[2], pm[3]));
+#pragma unroll
+            for (int cb = 0; cb < CB; ++cb) {
+                const bf16x8_t ga = __builtin_bit_cast(bf16x8_t, sm.gimg[(cb * S + (D == 128 ? s : 0)) * 64 + lane]);
+                float4_t &t = acc[D == 128 ? cb : s];
+                t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ga, bh, t, 0, 0, 0);
+                t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ga, bm, t, 0, 0, 0);
+            }
+        }
+        // signs: bits q of `sg` is acc[q / 4][q % 4] >= 0 (lane (n, g): D = 128
+        // projection 16 (q / 4) + 4 g + q % 4 of row n, D = 32 projection
+        // 4 g + q % 4 of row 16 (q / 4) + n)
+        uint32_t sg = 0u, unc = 0u, nf = 0u;
+        float amin[kSets];
+#pragma unroll
+        for (int q = 0; q < kSets; ++q) amin[q] = INFINITY;
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                sg |= acc[q][i] >= 0.0f ? 1u << (4 * q + i) : 0u;
+                float &m = amin[D == 128 ? 0 : q];
+                m = fminf(m, fabsf(acc[q][i]));
+            }
+        // Uncertain signs of finite rows and rows whose residual is not finite
+        // (or whose |e| sum reaches 2^127): encode128_kernel's bound, which was
+        // derived for 128 elements and holds for 32
+        bool rare = false;
+        float bound[kSets];
+#pragma unroll
+        for (int q = 0; q < kSets; ++q) {
+            bound[q] = as[q] * 7.82012939453125e-05f + 7.888609052210118e-31f;
+            const bool fin = as[q] < 0x1p127f, in = v0 + 16 * q + n < v_end;
+            nf |= (!fin && in) ? 1u << q : 0u;
+            rare = rare || (fin && !(amin[q] > bound[q])) || (!fin && in);
+        }
+        if (__builtin_amdgcn_ballot_w64(rare)) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int z = D == 128 ? 0 : q;
+                    if (as[z] < 0x1p127f && !(fabsf(acc[q][i]) > bound[z])) unc |= 1u << (4 * q + i);
+                }
+            float *st = sm.stage[wave];
+            int staged = -1;
+            auto stage = [&](int rr) {                 // row rr of the group
+                if (rr == staged) return;
+                if (n == (rr & 15)) {
+#pragma unroll
+                    for (int s = 0; s < 4; ++s)
+                        if (D == 128 || s == (rr >> 4))
+#pragma unroll
+                            for (int i = 0; i < 8; ++i) st[(D == 128 ? 32 * s : 0) + 8 * g + i] = e[s][i];
+                }
+                staged = rr;
+            };
+            uint64_t pend = __builtin_amdgcn_ballot_w64(unc != 0u);
+            while (pend) {
+                const int Lq = __builtin_ctzll(pend);
+                const uint32_t uL = __builtin_amdgcn_readlane(unc, Lq);
+                const int item = __builtin_ctz(uL);
+                const int o = (D == 128 ? 16 * (item >> 2) : 0) + 4 * (Lq >> 4) + (item & 3);
+                stage((Lq & 15) + (D == 128 ? 0 : 16 * (item >> 2)));
+                uint32_t fl;
+                const double tot = eg_row_dot<D>(st, sm.gbits + o * W, lane, fl);
+                if (lane == Lq) {
+                    unc &= ~(1u << item);
+                    sg = (sg & ~(1u << item)) | ((tot >= 0.0 ? 1u : 0u) << item);
+                }
+                pend = __builtin_amdgcn_ballot_w64(unc != 0u);
+            }
+#pragma unroll 1
+            for (int q = 0; q < kSets; ++q) {
+                uint64_t nfm = __builtin_amdgcn_ballot_w64(((nf >> q) & 1u) && g == 0);
+                while (nfm) {
+                    const int rr = __builtin_ctzll(nfm);
+                    nfm &= nfm - 1;
+                    stage(16 * q + rr);
+#pragma unroll 1
+                    for (int o = 0; o < QD; ++o) {
+                        // order-free sign of the fp32 sum (see encode128_kernel)
+                        uint32_t fl;
+                        const double tot = eg_row_dot<D>(st, sm.gbits + o * W, lane, fl);
+                        uint32_t bit;
+                        if ((fl & 1u) || (fl & 6u) == 6u) bit = 0u;
+                        else if (fl & 2u) bit = 1u;
+                        else if (fl & 4u) bit = 0u;
+                        else bit = tot >= 0.0 ? 1u : 0u;
+                        const int item = (D == 128 ? 4 * (o >> 4) : 4 * q) + (o & 3);
+                        if (n == rr && g == ((o & 15) >> 2)) sg = (sg & ~(1u << item)) | (bit << item);
+                    }
+                }
+            }
+        }
+        // stores
+        auto norm = [](double t) { return t > 3.4028234663852886e38 ? INFINITY : (float)sqrt(t); };
+        if constexpr (D == 128) {
+            uint32_t slo = ((sg & 15u) << (4 * g)) | (((sg >> 4) & 15u) << (16 + 4 * g));
+            uint32_t shi = (((sg >> 8) & 15u) << (4 * g)) | ((sg >> 12) << (16 + 4 * g));
+            slo |= xlane_u32<16>(slo);
+            slo |= xlane_u32<32>(slo);
+            shi |= xlane_u32<16>(shi);
+            shi |= xlane_u32<32>(shi);
+            if (v0 + n < v_end) {
+                uint32_t *np = reinterpret_cast<uint32_t *>(nibz + row[0] * 64);
+#pragma unroll
+                for (int s = 0; s < 4; ++s) np[4 * s + g] = nib[s];
+                if (g == 0) {
+                    reinterpret_cast<uint2 *>(qjlz + row[0] * 8)[0] = make_uint2(slo, shi);
+                    nrmz[row[0]] = norm(ss[0]);
+                }
+            }
+        } else {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                uint32_t sw = ((sg >> (4 * q)) & 15u) << (4 * g);
+                sw |= xlane_u32<16>(sw);
+                sw |= xlane_u32<32>(sw);
+                if (v0 + 16 * q + n < v_end) {
+                    reinterpret_cast<uint32_t *>(nibz + row[q] * 16)[g] = nib[q];
+                    if (g == 0) {
+                        reinterpret_cast<uint16_t *>(qjlz + row[q] * 2)[0] = (uint16_t)sw;
+                        nrmz[row[q]] = norm(ss[q]);
+                    }
+                }
+            }
+        }
+    };
+
+    // The next group's rows are requested as soon as the current ones are
+    // widened (past the last group: the current rows again).
+    uint4 raw[4][kRaw];
+    int64_t row[kSets];
+    rows_of(row, vcur, vb, vt);
+    load(raw, row);
+    for (;;) {
+        float x[4][8];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const uint4 *fl = reinterpret_cast<const uint4 *>(sm.flip + (D == 128 ? 32 * s : 0) + 8 * g);
+            const uint4 f0 = ROT ? fl[0] : make_uint4(0u, 0u, 0u, 0u), f1 = ROT ? fl[1] : f0;
+            const uint32_t f[8] = {f0.x, f0.y, f0.z, f0.w, f1.x, f1.y, f1.z, f1.w};
+            if constexpr (XDT == OMNI_F32) {
+                const uint32_t w[8] = {raw[s][0].x, raw[s][0].y, raw[s][0].z, raw[s][0].w,
+                                       raw[s][1].x, raw[s][1].y, raw[s][1].z, raw[s][1].w};
+#pragma unroll
+                for (int i = 0; i < 8; ++i) x[s][i] = __uint_as_float(w[i] ^ f[i]);
+            } else {
+                const uint32_t w[4] = {raw[s][0].x, raw[s][0].y, raw[s][0].z, raw[s][0].w};
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const uint32_t u = (i & 1) ? (w[i >> 1] >> 16) : (w[i >> 1] & 0xffffu);
+                    const float v = XDT == OMNI_BF16 ? __uint_as_float(u << 16) : f16_to_f32((uint16_t)u);
+                    x[s][i] = __uint_as_float(__float_as_uint(v) ^ f[i]);
+                }
+            }
+        }
+        const int64_t v0 = vcur;
+        int64_t cur[kSets];
+#pragma unroll
+        for (int q = 0; q < kSets; ++q) cur[q] = row[q];
+        vcur += kEgWaves * kGroup;
+        const bool more = vcur < v_end;
+        if (more) {
+            vb += a.step_b;
+            vt += a.step_t;
+            if (vt >= a.T) {
+                vt -= a.T;
+                ++vb;
+            }
+            rows_of(row, vcur, vb, vt);
+        }
+        load(raw, row);
+        encode(x, cur, v0);
+        if (!more) break;
+    }
+}
+
 // ── omni_dequantize ─────────────────────────────────────────────────────
 //
 // k_hat_d = fl(cb[code_d] + fl(s_d * fl(norm * c))), c = fp32(sqrt(2/pi)/D),
@@ -890,7 +1258,7 @@ extern "C" int omni_wht_rotate(const void *x, int dtype, int64_t rows, int head_
 
 // The table-driven wave kernel serves 16-bit inputs at D = 128 when each head
 // has enough rows to amortise its 64 KB table; the rest (f32 inputs, D = 32,
-// one-row "heads" of the row-seeded API) take the lane-per-row kernel.
+// few rows per head) goes to launch_encode_rows.
 static bool enc_fast(int64_t B, int64_t T, int head_dim, int x_dtype) {
     return head_dim == 128 && (x_dtype == OMNI_BF16 || x_dtype == OMNI_F16) && B * T >= 64;
 }
@@ -981,18 +1349,48 @@ static int launch_encode128(const void *const xs[2], int nz, int x_dtype, int64_
     return OMNI_OK;
 }
 
-// The lane-per-row kernel (f32 inputs, D = 32, few rows per head).
-static int launch_encode_rows(const void *x, int x_dtype, int64_t B, int H, int64_t T, int head_dim, int rotate,
-                              const int8_t *sign_flip, const float *codebooks, int per_head_codebook,
-                              const uint32_t *g_bits, uint8_t *nibbles, uint8_t *qjl, float *norms, hipStream_t st) {
+// encode_grid_kernel over nz (1 or 2) tensors of one shape.
+template <int XDT, int D>
+static void launch_encode_grid(const EncArgs &a, dim3 grid, hipStream_t st) {
+    if (a.rotate) hipLaunchKernelGGL((encode_grid_kernel<XDT, D, true>), grid, dim3(64 * kEgWaves), 0, st, a);
+    else hipLaunchKernelGGL((encode_grid_kernel<XDT, D, false>), grid, dim3(64 * kEgWaves), 0, st, a);
+}
+
+// Inputs without a value table (f32, D = 32, few rows per head).
+static int launch_encode_rows(const void *const xs[2], int nz, int x_dtype, int64_t B, int H, int64_t T, int head_dim,
+                              int rotate, const int8_t *sign_flip, const float *codebooks, int per_head_codebook,
+                              const uint32_t *g_bits, uint8_t *const nib[2], uint8_t *const qjl[2],
+                              float *const nrm[2], hipStream_t st) {
     const float s = inv_sqrt_dim_f32(head_dim);
-    dim3 grid((unsigned)((T + kRowsPerBlock - 1) / kRowsPerBlock), (unsigned)H, (unsigned)B);
-    if (head_dim == 128)
-        hipLaunchKernelGGL(encode_kernel<128>, grid, dim3(kRowsPerBlock), 0, st, x, x_dtype, T, H,
-                           rotate, sign_flip, codebooks, per_head_codebook, g_bits, nibbles, qjl, norms, s);
-    else
-        hipLaunchKernelGGL(encode_kernel<32>, grid, dim3(kRowsPerBlock), 0, st, x, x_dtype, T, H,
-                           rotate, sign_flip, codebooks, per_head_codebook, g_bits, nibbles, qjl, norms, s);
+    EncArgs a{};
+    for (int z = 0; z < 2; ++z) {
+        const int zz = z < nz ? z : 0;
+        a.x[z] = xs[zz]; a.nibbles[z] = nib[zz]; a.qjl[z] = qjl[zz]; a.norms[z] = nrm[zz];
+    }
+    a.codebooks = codebooks; a.g_bits = g_bits; a.sign_flip = sign_flip;
+    a.T = T; a.nrows_head = B * T; a.H = H; a.per_head = per_head_codebook; a.rotate = rotate;
+    a.scale = s;
+    // three blocks of four waves per CU across the tensors and heads, each
+    // a run of rows of one head of one tensor
+    const int64_t grp = (head_dim == 128 ? 16 : 64) * kEgWaves;
+    const int64_t want = ((int64_t)3 * device_cus() + (int64_t)H * nz - 1) / ((int64_t)H * nz);
+    int64_t rpb = (a.nrows_head + want - 1) / want;
+    rpb = (rpb + grp - 1) / grp * grp;
+    a.rows_per_block[0] = a.rows_per_block[1] = rpb;
+    a.step_b = grp / T;
+    a.step_t = grp % T;
+    const int64_t nx = (a.nrows_head + rpb - 1) / rpb;
+    OMNI_CHECK_ARG(nx <= 2147483647LL, "omni_encode: grid too large");
+    const dim3 eg((unsigned)nx, (unsigned)H, (unsigned)nz);
+    if (head_dim == 128) {
+        if (x_dtype == OMNI_F32) launch_encode_grid<OMNI_F32, 128>(a, eg, st);
+        else if (x_dtype == OMNI_BF16) launch_encode_grid<OMNI_BF16, 128>(a, eg, st);
+        else launch_encode_grid<OMNI_F16, 128>(a, eg, st);
+    } else {
+        if (x_dtype == OMNI_F32) launch_encode_grid<OMNI_F32, 32>(a, eg, st);
+        else if (x_dtype == OMNI_BF16) launch_encode_grid<OMNI_BF16, 32>(a, eg, st);
+        else launch_encode_grid<OMNI_F16, 32>(a, eg, st);
+    }
     OMNI_CHECK_LAUNCH("omni_encode");
     return OMNI_OK;
 }
@@ -1009,6 +1407,9 @@ extern "C" int omni_encode(const void *x, int x_dtype, int64_t B, int H, int64_t
     OMNI_CHECK_ARG(x && codebooks && g_bits && nibbles && qjl && norms, "omni_encode: NULL pointer");
     OMNI_CHECK_ARG(B <= 65535 && H <= 65535, "omni_encode: B and H must be <= 65535");
     hipStream_t st = as_stream(stream);
+    const void *xs[2] = {x, x};
+    uint8_t *nib[2] = {nibbles, nibbles}, *qj[2] = {qjl, qjl};
+    float *nr[2] = {norms, norms};
     if (enc_fast(B, T, head_dim, x_dtype)) {
         const size_t need = omni_encode_workspace_size(B, H, T, head_dim, x_dtype, per_head_codebook);
         if (workspace == nullptr || workspace_bytes < need) {
@@ -1018,14 +1419,11 @@ extern "C" int omni_encode(const void *x, int x_dtype, int64_t B, int H, int64_t
         uint8_t *table = reinterpret_cast<uint8_t *>(workspace);
         launch_code_tables(codebooks, per_head_codebook, H, x_dtype, table, st);
         OMNI_CHECK_LAUNCH("omni_encode (code table)");
-        const void *xs[2] = {x, x};
-        uint8_t *nib[2] = {nibbles, nibbles}, *qj[2] = {qjl, qjl};
-        float *nr[2] = {norms, norms};
         return launch_encode128(xs, 1, x_dtype, B, H, T, rotate, sign_flip, codebooks, per_head_codebook, g_bits,
                                 table, nib, qj, nr, st);
     }
-    return launch_encode_rows(x, x_dtype, B, H, T, head_dim, rotate, sign_flip, codebooks, per_head_codebook, g_bits,
-                              nibbles, qjl, norms, st);
+    return launch_encode_rows(xs, 1, x_dtype, B, H, T, head_dim, rotate, sign_flip, codebooks, per_head_codebook,
+                              g_bits, nib, qj, nr, st);
 }
 
 extern "C" size_t omni_encode_tables_size(int H, int per_head_codebook) {
@@ -1063,24 +1461,20 @@ extern "C" int omni_encode_pair(const void *x0, const void *x1, int x_dtype, int
     OMNI_CHECK_ARG(nz == 1 || (nibbles1 && qjl1 && norms1), "omni_encode_pair: NULL output for the second tensor");
     OMNI_CHECK_ARG(B <= 65535 && H <= 65535, "omni_encode_pair: B and H must be <= 65535");
     hipStream_t st = as_stream(stream);
+    const void *xs[2] = {x0, x1 ? x1 : x0};
+    uint8_t *nib[2] = {nibbles0, nz > 1 ? nibbles1 : nibbles0}, *qj[2] = {qjl0, nz > 1 ? qjl1 : qjl0};
+    float *nr[2] = {norms0, nz > 1 ? norms1 : norms0};
     if (enc_fast(B, T, head_dim, x_dtype)) {
         const size_t need = omni_encode_tables_size(H, per_head_codebook);
         if (tables == nullptr || tables_bytes < need) {
             set_error("omni_encode_pair: %zu bytes of code tables required, %zu given", need, tables_bytes);
             return OMNI_EWORKSPACE;
         }
-        const void *xs[2] = {x0, x1 ? x1 : x0};
-        uint8_t *nib[2] = {nibbles0, nz > 1 ? nibbles1 : nibbles0}, *qj[2] = {qjl0, nz > 1 ? qjl1 : qjl0};
-        float *nr[2] = {norms0, nz > 1 ? norms1 : norms0};
         return launch_encode128(xs, nz, x_dtype, B, H, T, rotate, sign_flip, codebooks, per_head_codebook, g_bits,
                                 tables, nib, qj, nr, st);
     }
-    int rc = launch_encode_rows(x0, x_dtype, B, H, T, head_dim, rotate, sign_flip, codebooks, per_head_codebook,
-                                g_bits, nibbles0, qjl0, norms0, st);
-    if (rc == OMNI_OK && nz > 1)
-        rc = launch_encode_rows(x1, x_dtype, B, H, T, head_dim, rotate, sign_flip, codebooks, per_head_codebook,
-                                g_bits, nibbles1, qjl1, norms1, st);
-    return rc;
+    return launch_encode_rows(xs, nz, x_dtype, B, H, T, head_dim, rotate, sign_flip, codebooks, per_head_codebook,
+                              g_bits, nib, qj, nr, st);
 }
 
 extern "C" int omni_encode_paged(const void *k, const void *v, int x_dtype, int64_t B, int H, int64_t T,

@@ -281,6 +281,68 @@ def test_known_answers_through_the_kernels(device):
         assert torch.equal(out[0, 0, 0, :n], want)
 
 
+# ── the wave encoder without a value table (f32 input, D = 32, few rows) ──
+
+_GRID_ROWS = [(1, 1), (15, 1), (1, 17), (5, 3), (1, 64), (3, 65), (7, 37)]
+
+
+@pytest.mark.parametrize("D,dtype", [(128, torch.float32), (32, torch.float32), (32, torch.bfloat16),
+                                     (32, torch.float16), (128, torch.bfloat16)])
+@pytest.mark.parametrize("B,T", _GRID_ROWS)
+def test_grid_encoder_row_counts(device, B, T, D, dtype):
+    """Rows per head around the 16- and 64-row groups, groups that span
+    several sequences, rotation and sign flip in the kernel, K and V."""
+    from omnistack_rs.kernels.quantize import PackedKVEncoder
+    if D == 128 and dtype == torch.bfloat16 and B * T >= 64:
+        pytest.skip("the value-table kernel's range")
+    H = 3
+    x = [_data.kv((B, H, T, D), seed=60 + z, dtype=dtype) for z in range(2)]
+    s = _data.sign_flip(D)
+    cb = _data.gaussian_codebook(H) * torch.linspace(0.8, 1.4, H).reshape(H, 1)
+    print(f"[encode] grid B{B} T{T} D{D} {dtype}", flush=True)
+    enc = PackedKVEncoder(cb.to(device), H, user_id=9, sign_flip=s.to(device), dtype=dtype, head_dim=D)
+    for xi, out in zip(x, enc.encode(x[0].to(device), x[1].to(device))):
+        _check_encode(restate.rotate(xi, s), cb, 9, *out, tag=f"grid B{B} T{T} D{D} {dtype}")
+
+
+@pytest.mark.parametrize("D", [128, 32])
+@pytest.mark.parametrize("kind", ["plain", "duplicates", "close", "unsorted", "wide", "one_value", "nan"])
+def test_grid_encoder_codebooks(device, kind, D):
+    """Codes at centroids, midpoints and one ulp to either side, across the
+    grid's ends and far past them, for codebooks the cells can serve and ones
+    that send every value through all 16 distances."""
+    from omnistack_rs.kernels.quantize import quantize_heads
+    cb = _data.gaussian_codebook(1)[0].clone()
+    if kind == "duplicates":
+        cb[7] = cb[8]
+        cb[15] = cb[14]
+    elif kind == "close":
+        cb[5] = torch.nextafter(cb[4], torch.tensor(10.0))
+    elif kind == "unsorted":
+        cb = cb[torch.randperm(16, generator=_data.gen(61))]
+    elif kind == "wide":
+        cb[15], cb[0] = 1e30, -1e30
+    elif kind == "one_value":
+        cb[:] = 0.25
+    elif kind == "nan":
+        cb[3] = float("nan")
+    inf = torch.tensor(float("inf"))
+    mid = (cb[:-1] + cb[1:]) / 2
+    pts = torch.cat([cb, mid, torch.nextafter(mid, inf), torch.nextafter(mid, -inf), 8 * cb, 7.9 * cb, 1e6 * cb, 1e30 * cb,
+                     torch.tensor([0.0, -0.0, 1e-40, -1e-40, 3e38, -3e38])])
+    x = torch.randn(1, 1, 40, D, generator=_data.gen(62))
+    pts = pts[torch.isfinite(pts)]
+    x.view(-1)[: pts.numel()] = pts
+    print(f"[encode] grid codebook {kind} D{D}", flush=True)
+    nib, qjl, nrm = quantize_heads(x.to(device), cb.to(device), user_id=4)
+    if kind == "nan":                                    # residuals are NaN where the NaN centroid wins
+        r_nib, r_qjl, _ = restate.quantize_heads(x, cb, user_id=4)
+        assert torch.equal(nib.cpu(), r_nib)
+        assert torch.equal(qjl.cpu(), r_qjl)
+        return
+    _check_encode(x, cb, 4, nib, qjl, nrm, tag=f"grid codebook {kind} D{D}")
+
+
 # ── the table-driven wave encoder (16-bit input, D = 128, >= 64 rows/head) ──
 
 def test_fast_encoder_edge_rows_bf16(device):
