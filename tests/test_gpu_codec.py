@@ -281,6 +281,42 @@ def test_known_answers_through_the_kernels(device):
         assert torch.equal(out[0, 0, 0, :n], want)
 
 
+@pytest.mark.parametrize("rows", [1, 15, 17, 63, 64, 65, 257])
+@pytest.mark.parametrize("D", [128, 32])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_wht_row_counts(device, rows, D, dtype):
+    """Rows around a wave's 16 (64 at head_dim 32) and a block's four waves,
+    out of place and in place."""
+    from omnistack_rs import _lib
+    from omnistack_rs.kernels.hadamard import rotate
+    x = _data.kv((1, 1, rows, D), seed=70 + rows, dtype=dtype)[0, 0]
+    x[rows // 2, 3] = 3e4
+    s = _data.sign_flip(D)
+    want = restate.rotate(x, s)
+    xd = x.to(device)
+    assert torch.equal(rotate(xd, s.to(device)).cpu(), want) and torch.equal(xd.cpu(), x)
+    sd = s.to(device)
+    _lib.check(_lib.lib().omni_wht_rotate(xd.data_ptr(), _lib.dtype_code(dtype), rows, D, sd.data_ptr(), xd.data_ptr(),
+                                          _lib.stream_of(xd.device)))
+    assert torch.equal(xd.cpu(), want)
+
+
+@pytest.mark.parametrize("B,T", [(1, 1), (37, 1), (5, 7), (1, 31), (3, 33), (1, 129), (2, 700), (1, 60001)])
+@pytest.mark.parametrize("D,with_qjl", [(128, True), (32, True), (32, False)])
+def test_dequantize_row_counts(device, B, T, D, with_qjl):
+    """Runs that span several sequences, end inside a pass of a block, and
+    sequences past the range of the 16-bit quotient."""
+    from omnistack_rs.kernels.quantize import dequantize_heads
+    H, g = 2, _data.gen(80 + T)
+    nib = torch.randint(0, 256, (B, H, T, D // 2), generator=g, dtype=torch.uint8)
+    qjl = torch.randint(0, 256, (B, H, T, D // 16), generator=g, dtype=torch.uint8)
+    nrm = torch.rand(B, H, T, generator=g) * 2
+    cb = _data.gaussian_codebook(H) * torch.tensor([[0.9], [1.2]])
+    got = dequantize_heads(nib.to(device), qjl.to(device), nrm.to(device), cb.to(device), user_id=6, with_qjl=with_qjl)
+    want = restate.dequantize_heads(nib, qjl, nrm, cb, user_id=6, with_qjl=with_qjl)
+    assert torch.equal(got.cpu(), want)
+
+
 # ── the wave encoder without a value table (f32 input, D = 32, few rows) ──
 
 _GRID_ROWS = [(1, 1), (15, 1), (1, 17), (5, 3), (1, 64), (3, 65), (7, 37)]
