@@ -253,12 +253,12 @@ int omni_attn(const void *q, int q_dtype,
  * omni_attn with the per-user LoRA update of q applied first:
  *   q_eff[b] = dtype(q[b] + ((x[b] A[idx[b]]^T) B[idx[b]]^T) * lora_alpha)
  * (idx < 0: q unchanged; idx >= n_loras: NaN rows), then attention on q_eff
- * exactly as omni_attn.  LoRA shapes and dtypes as omni_lora_apply.  At
- * head_dim 128 with <= 32 query rows per kv head, a nonzero score scale and
- * a 16-bit adapter of rank 8 or 16, hidden <= 256 and a 16-byte aligned
- * lora_b, the update runs inside the attention kernel's prologue (one
- * launch); otherwise the gather-apply kernel writes
- * q_eff into the workspace tail first.  q_eff is rounded
+ * exactly as omni_attn.  LoRA shapes and dtypes as omni_lora_apply.  Where
+ * the decode kernel runs (head_dim 128 with up to 8 query rows per kv head,
+ * and with 9 to 32 where it is the faster one, at a nonzero score scale) a
+ * 16-bit adapter of rank 8 or 16, hidden <= 256 and a 16-byte aligned lora_b
+ * is applied inside its prologue (one launch); otherwise the gather-apply
+ * kernel writes q_eff into the workspace tail first.  q_eff is rounded
  * exactly as omni_lora_apply rounds it.  `workspace` must hold
  * omni_attn_lora_workspace_size(...) bytes.
  * Replaces omni_attn(..., x, lora_a, lora_b, lora_indices, lora_alpha)
@@ -363,7 +363,8 @@ void omni_attn_plan_destroy(omni_attn_plan *plan);
  * KV cache (MANIFEST.md:211-215; page_size = 16 tokens, config.py:43) but
  * gathers whole sequences instead (scripts/run_criteo_benchmark.py:553-557);
  * this is that gather as page lookups inside the attention kernels (decode
- * for up to 32 query rows per kv head, T * Hq / Hkv; chunked prefill above).
+ * for up to 8 query rows per kv head, T * Hq / Hkv; chunked prefill above 32;
+ * the faster of the two between).
  * Pools (k_nib, k_qjl, k_norms, v_nib) are shaped like a contiguous cache
  * with pages as the batch axis: (n_pages, Hkv, page_size, ...).  Sequence b
  * holds seq_lens[b] tokens; token s sits in page page_table[b * max_pages +

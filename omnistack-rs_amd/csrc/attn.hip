@@ -10,7 +10,8 @@
 //   alpha_s = ||e_s|| sqrt(2/pi) / D,
 // with the encoder's per-head G (seed (user % 1024) ^ h).
 //
-// Work decomposition.  One block streams one (batch, kv head, token split)
+// Work decomposition of the generic kernel (head_dim 32 at a score scale of
+// 0; the kernels below it carry everything else).  One block streams one (batch, kv head, token split)
 // for up to 16 query rows (all GQA heads of the group for one or more query
 // tokens), so every cached byte is read once per group, not once per q head.
 // Each wave takes 16-token tiles round-robin and runs three MFMA chains
@@ -69,6 +70,7 @@ struct AttnArgs {
     int lora_w_dtype, lora_hidden, lora_rank, lora_n;
     float lora_alpha;
     int rows;                  // query rows per block (16: generic kernel, 8: D=128 decode kernel)
+    int tw_shift;              // prefill kernels: log2 of the waves that share a group of rows
     // paged cache (D=128 decode kernel): pool arrays shaped like a contiguous
     // cache with (n_pages, Hkv, page_size); sequence b holds seq_lens[b]
     // tokens in pages page_table[b * max_pages + j] (S = max_pages * page_size)
@@ -466,34 +468,54 @@ __global__ __launch_bounds__(64 * kMaxWaves) void attn_kernel(AttnArgs a) {
     }
 }
 
+// Merge of the splits' (m, l, O): two elements of a row per thread (D / 2
+// threads per row), eight splits' loads in flight: a latency chain of two
+// loads, so it spreads over as many blocks as the rows give.  One block per
+// unit, one split's loads at a time, took 11.2 us for 24 units of 24 rows and
+// 11 splits, this 4.9.
 template <int D>
 __global__ __launch_bounds__(256) void attn_combine_kernel(AttnArgs a) {
+    constexpr int kLanes = D / 2, kRowsPer = 256 / kLanes;
     const int hk = blockIdx.y;
     const int64_t bz = blockIdx.z;
     const int64_t b = bz / a.n_rchunks;
-    const int rc = (int)(bz % a.n_rchunks);
-    const int rows = a.rows;
+    const int rc = (int)(bz - b * a.n_rchunks);
+    const int rr = blockIdx.x * kRowsPer + (int)threadIdx.x / kLanes, d = 2 * ((int)threadIdx.x % kLanes);
+    const int64_t rho = (int64_t)rc * a.rows + rr;
+    if (rr >= a.rows || rho >= a.T * a.G) return;
     const int64_t unit = (b * a.Hkv + hk) * a.n_rchunks + rc;
-    const int64_t nrows_total = a.T * a.G;
-    for (int s = threadIdx.x; s < rows * D; s += blockDim.x) {
-        const int rr = s / D, d = s % D;
-        const int64_t rho = (int64_t)rc * rows + rr;
-        if (rho >= nrows_total) continue;
-        float mx = -INFINITY;
-        for (int sp = 0; sp < a.splits; ++sp)
-            mx = fmaxf(mx, a.ws[((unit * a.splits + sp) * rows + rr) * (D + 2) + D]);
-        const float mu = (mx == -INFINITY) ? 0.0f : mx;
-        float lsum = 0.0f, osum = 0.0f;
-        for (int sp = 0; sp < a.splits; ++sp) {
-            const float *wp = a.ws + ((unit * a.splits + sp) * rows + rr) * (D + 2);
-            const float f = exp2f(wp[D] - mu);
-            lsum = __builtin_fmaf(f, wp[D + 1], lsum);
-            osum = __builtin_fmaf(f, wp[d], osum);
-        }
-        const int64_t t = rho / a.G;
-        const int hq = hk * a.G + (int)(rho % a.G);
-        a.out[((b * a.Hq + hq) * a.T + t) * D + d] = osum / lsum;
+    const int64_t stride = (int64_t)a.rows * (D + 2);
+    const float *wp = a.ws + (unit * a.splits * a.rows + rr) * (D + 2);
+    float mx = -INFINITY;
+    for (int s0 = 0; s0 < a.splits; s0 += 8) {
+        float m[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) m[k] = wp[imin(s0 + k, a.splits - 1) * stride + D];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) mx = fmaxf(mx, m[k]);
     }
+    const float mu = (mx == -INFINITY) ? 0.0f : mx;
+    float lsum = 0.0f, o0 = 0.0f, o1 = 0.0f;
+    for (int s0 = 0; s0 < a.splits; s0 += 8) {
+        float2 ml[8], o[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const float *p = wp + imin(s0 + k, a.splits - 1) * stride;
+            ml[k] = *reinterpret_cast<const float2 *>(p + D);
+            o[k] = *reinterpret_cast<const float2 *>(p + d);
+        }
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+            if (s0 + k < a.splits) {
+                const float f = exp2f(ml[k].x - mu);
+                lsum = __builtin_fmaf(f, ml[k].y, lsum);
+                o0 = __builtin_fmaf(f, o[k].x, o0);
+                o1 = __builtin_fmaf(f, o[k].y, o1);
+            }
+    }
+    const int64_t t = rho / a.G;
+    const int hq = hk * a.G + (int)(rho - t * a.G);
+    *reinterpret_cast<float2 *>(a.out + ((b * a.Hq + hq) * a.T + t) * D + d) = make_float2(o0 / lsum, o1 / lsum);
 }
 
 // ── D = 128 decode kernel ───────────────────────────────────────────────
@@ -569,6 +591,7 @@ constexpr int kDecSlabBytes = kDecWaves * kDecRows * kObStride * 4;
 static_assert(kDecSlabBytes + 2 * kDecWaves * kDecRows * 4 <= kDecQsOff, "epilogue slabs overlap the query rows");
 static_assert(kDecWaves >= kDecRows, "one query row per wave in the prologue");
 
+typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 
 __device__ __forceinline__ half8_t as_half8(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
@@ -742,9 +765,8 @@ __device__ __forceinline__ void paged_half_rows(const AttnArgs &a, const int32_t
 }
 
 __device__ __forceinline__ uint32_t cvt_pk_h2(float x, float y) {
-    typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
     typedef float f2_t __attribute__((ext_vector_type(2)));
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f2_t){x, y}, h2_t));
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f2_t){x, y}, half2_t));
 }
 
 // max over lanes {l, l^16, l^32, l^48} without LDS (v_permlane16/32_swap).
@@ -1762,6 +1784,217 @@ __global__ __launch_bounds__(64 * kDecWaves) void attn_decode128_kernel(AttnArgs
     }
 }
 
+// Merge of the waves that share a group of RW rows (2^tws waves per group):
+// each row's weights exp2(m - max) over its waves, in place of m, and its
+// denominator (with the largest m in the first wave's l slot).
+template <int RW>
+__device__ __forceinline__ void merge_weights(float *ml, float *lt, const float *bad, int tid, int groups, int tws) {
+    if (tid >= RW * groups) return;
+    const int gr = tid / RW, r = tid % RW, w0 = gr << tws, nw = 1 << tws;
+    float mx = -__FLT_MAX__, l = 0.0f, nan = 0.0f;
+    for (int w = w0; w < w0 + nw; ++w) mx = fmaxf(mx, ml[(w * RW + r) * 2]);
+    for (int w = w0; w < w0 + nw; ++w) {
+        float *p = ml + (w * RW + r) * 2;
+        const float f = __builtin_amdgcn_exp2f(p[0] - mx);
+        l = __builtin_fmaf(f, p[1], l);
+        p[0] = f;
+        nan += bad[w];
+    }
+    lt[tid] = nan != 0.0f ? __builtin_nanf("") : l;
+    ml[(w0 * RW + r) * 2 + 1] = mx;
+}
+
+// The merged rows, four elements a thread: out, or the split's partials.
+template <int D, int RW>
+__device__ __forceinline__ void merge_rows(const AttnArgs &a, const float *slabs, const float *ml, const float *lt, int tid,
+                                           int threads, int groups, int tws, int rc, int nrows_total, int64_t b, int hk,
+                                           int64_t unit, int split) {
+    constexpr int kStride = D + 4;
+    for (int e = tid; e < groups * RW * (D / 4); e += threads) {
+        const int rr = e / (D / 4), d = 4 * (e % (D / 4)), gr = rr / RW, r = rr % RW, w0 = gr << tws;
+        const int rho = rc * a.rows + rr;
+        if (rho >= nrows_total) break;                 // rows ascend with e
+        float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 4
+        for (int w = 0; w < (1 << tws); ++w) {
+            const float f = ml[((w0 + w) * RW + r) * 2];
+            const float4 v = *reinterpret_cast<const float4 *>(slabs + ((w0 + w) * RW + r) * kStride + d);
+            o.x = __builtin_fmaf(f, v.x, o.x);
+            o.y = __builtin_fmaf(f, v.y, o.y);
+            o.z = __builtin_fmaf(f, v.z, o.z);
+            o.w = __builtin_fmaf(f, v.w, o.w);
+        }
+        const float l = lt[rr];
+        if (a.splits == 1) {
+            const int t = rho / a.G, hq = hk * a.G + (rho - t * a.G);
+            *reinterpret_cast<float4 *>(a.out + ((b * a.Hq + hq) * a.T + t) * D + d) =
+                make_float4(o.x / l, o.y / l, o.z / l, o.w / l);
+        } else {
+            float *wp = a.ws + ((unit * a.splits + split) * a.rows + rr) * (D + 2);
+            *reinterpret_cast<float2 *>(wp + d) = make_float2(o.x, o.y);
+            *reinterpret_cast<float2 *>(wp + d + 2) = make_float2(o.z, o.w);
+            if (d == 0) { wp[D] = ml[(w0 * RW + r) * 2 + 1]; wp[D + 1] = l; }
+        }
+    }
+}
+
+// Query rows of the prefill kernels, 16 * NS of them per wave: (sign flip,)
+// WHT in the reference's stage order, rounding to q's dtype; then a power of
+// two per row into fp16 range, the score scale's sign (exact, so that every
+// row's score scale is >= 0 and the exponent takes it in an fma), and fp16
+// rows in LDS (QLO: the fp16 remainders of f32 rows `lo_plane` halves on).
+// Lane (n, g) holds 32 values: elements 32 s + 8 g + i of row n (D = 128) or
+// 8 g + i of row 16 s + n (D = 32), so all rows' loads are in flight together
+// and a butterfly stage costs 16 additions per lane.  D = 128: 16-byte chunk c
+// of row r is stored at chunk c ^ (r % 16) (the rows of one read lie 256
+// bytes apart: on the same banks otherwise).  One row per wave at a time, as
+// before, took about 1.2 us a row: a call of 128 rows and 128 tokens, 8 kv
+// heads, 46.9 -> 29.2 us (head_dim 32: 33.4 -> 20.0).
+template <int D, int NS, bool QLO>
+__device__ __forceinline__ void stage_rows(const AttnArgs &a, int64_t b, int hk, int row0, int nrows_total, int lane,
+                                           uint16_t *stage, int lo_plane, float *qsr_l) {
+    static_assert(D == 128 ? NS == 1 : NS <= 4, "one set of 16 rows at D = 128");
+    constexpr int C = D == 128 ? 4 : NS;               // chunks of eight values held
+    const int n = lane & 15, g = lane >> 4;
+    float x[C][8];
+    int rho[NS];
+    const char *base[NS];
+    const int esz = a.q_dtype == OMNI_F32 ? 4 : 2;
+#pragma unroll
+    for (int q = 0; q < NS; ++q) {
+        rho[q] = row0 + 16 * q + n;
+        const int rc = rho[q] < nrows_total ? rho[q] : nrows_total - 1;
+        const int t = rc / a.G, hq = hk * a.G + (rc - t * a.G);
+        base[q] = reinterpret_cast<const char *>(a.q) + ((b * a.Hq + hq) * a.T + t) * (int64_t)(D * esz) + 8 * g * esz;
+    }
+    if (a.q_dtype == OMNI_F32) {
+#pragma unroll
+        for (int s = 0; s < C; ++s) {
+            const float4 *p = reinterpret_cast<const float4 *>(base[D == 128 ? 0 : s] + (D == 128 ? 128 * s : 0));
+            const float4 u = p[0], v = p[1];
+            x[s][0] = u.x; x[s][1] = u.y; x[s][2] = u.z; x[s][3] = u.w;
+            x[s][4] = v.x; x[s][5] = v.y; x[s][6] = v.z; x[s][7] = v.w;
+        }
+    } else {
+        uint4 w[C];
+#pragma unroll
+        for (int s = 0; s < C; ++s)
+            w[s] = *reinterpret_cast<const uint4 *>(base[D == 128 ? 0 : s] + (D == 128 ? 64 * s : 0));
+        const bool bf = a.q_dtype == OMNI_BF16;
+#pragma unroll
+        for (int s = 0; s < C; ++s) {
+            const uint32_t d[4] = {w[s].x, w[s].y, w[s].z, w[s].w};
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const uint16_t u = (uint16_t)((i & 1) ? d[i >> 1] >> 16 : d[i >> 1] & 0xffffu);
+                x[s][i] = bf ? bf16_to_f32(u) : f16_to_f32(u);
+            }
+        }
+    }
+    if (a.rotate_q) {
+        if (a.sign_flip) {
+#pragma unroll
+            for (int s = 0; s < C; ++s) {
+                if (D == 32 && s > 0) break;           // one 32-element pattern for every set
+                const uint2 f = *reinterpret_cast<const uint2 *>(a.sign_flip + (D == 128 ? 32 * s : 0) + 8 * g);
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const uint32_t m = ((i < 4 ? f.x >> (8 * i) : f.y >> (8 * i - 32)) & 0x80u) << 24;
+#pragma unroll
+                    for (int q = 0; q < (D == 128 ? 1 : C); ++q)
+                        x[D == 128 ? s : q][i] = __uint_as_float(__float_as_uint(x[D == 128 ? s : q][i]) ^ m);
+                }
+            }
+        }
+#pragma unroll
+        for (int hh = 1; hh < 8; hh <<= 1)
+#pragma unroll
+            for (int s = 0; s < C; ++s)
+#pragma unroll
+                for (int i = 0; i < 8; ++i)
+                    if (!(i & hh)) {
+                        const float u = x[s][i], l = x[s][i + hh];
+                        x[s][i] = u + l;
+                        x[s][i + hh] = u - l;
+                    }
+#pragma unroll
+        for (int s = 0; s < C; ++s)
+#pragma unroll
+            for (int i = 0; i < 8; i += 2) xlane_pair_butterfly<16>(x[s][i], x[s][i + 1]);
+#pragma unroll
+        for (int s = 0; s < C; ++s)
+#pragma unroll
+            for (int i = 0; i < 8; i += 2) xlane_pair_butterfly<32>(x[s][i], x[s][i + 1]);
+        if constexpr (D == 128) {
+#pragma unroll
+            for (int hs = 1; hs < 4; hs <<= 1)
+#pragma unroll
+                for (int s = 0; s < 4; ++s)
+                    if (!(s & hs))
+#pragma unroll
+                        for (int i = 0; i < 8; ++i) {
+                            const float u = x[s][i], l = x[s + hs][i];
+                            x[s][i] = u + l;
+                            x[s + hs][i] = u - l;
+                        }
+        }
+#pragma unroll
+        for (int s = 0; s < C; ++s)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                float p = x[s][i] * a.wht_scale;
+                asm volatile("" : "+v"(p));            // rounded to fp32 before q's dtype
+                x[s][i] = round_to_dtype(p, a.q_dtype);
+            }
+    }
+    const float ssign = a.qscale < 0.0f ? -1.0f : 1.0f;
+#pragma unroll
+    for (int q = 0; q < NS; ++q) {
+        const bool ok = rho[q] < nrows_total;
+        // row max |q| -> 2^k with max * 2^k in [2^14, 2^15)
+        float m = 0.0f;
+#pragma unroll
+        for (int s = 0; s < C; ++s)
+            if (D == 128 || s == q)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) m = fmaxf(m, fabsf(x[s][i]));
+        m = max_over_groups(m);
+        m = ok ? m : 0.0f;
+        int ex = 0;
+        if (m > 0.0f && m < INFINITY) frexpf(m, &ex);
+        const float sr = ldexpf(1.0f, 15 - imax(ex, -100));      // m * sr in [2^14, 2^15) unless m < 2^-101
+        // a positive factor is kept >= FLT_MIN (one that underflows leaves
+        // every score as good as 0 either way), so a masked score's -inf
+        // stays -inf through the maximum and the exponent; a zero scale (D =
+        // 128) keeps 0 (inf x 0 = NaN, as the reference forms scale x score)
+        // and re-masks the exponents there
+        const float q0 = fabsf(a.qscale) / sr;
+        if (g == 0) qsr_l[16 * q + n] = (q0 < __FLT_MIN__ && (D == 32 || a.qscale != 0.0f)) ? __FLT_MIN__ : q0;
+        const float f = ssign;
+#pragma unroll
+        for (int s = 0; s < C; ++s)
+            if (D == 128 || s == q) {
+                uint32_t hw[4], lw[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    float v[2];
+                    uint16_t h[2], l[2];
+#pragma unroll
+                    for (int k = 0; k < 2; ++k) {
+                        v[k] = ok ? f * x[s][2 * j + k] * sr : 0.0f;
+                        h[k] = f32_to_f16_rne(v[k]);
+                        l[k] = QLO ? f32_to_f16_rne(v[k] - f16_to_f32(h[k])) : (uint16_t)0;
+                    }
+                    hw[j] = (uint32_t)h[0] | ((uint32_t)h[1] << 16);
+                    lw[j] = (uint32_t)l[0] | ((uint32_t)l[1] << 16);
+                }
+                uint16_t *dst = stage + (16 * q + n) * D + 8 * (D == 128 ? (4 * s + g) ^ n : g);
+                *reinterpret_cast<uint4 *>(dst) = make_uint4(hw[0], hw[1], hw[2], hw[3]);
+                if constexpr (QLO) *reinterpret_cast<uint4 *>(dst + lo_plane) = make_uint4(lw[0], lw[1], lw[2], lw[3]);
+            }
+    }
+}
+
 // ── chunked-prefill kernel (many query rows per (batch, kv head)) ────────
 //
 // Same math as the decode kernel, organised for T > 1: each wave owns 16 * NCB
@@ -1776,14 +2009,16 @@ __global__ __launch_bounds__(64 * kDecWaves) void attn_decode128_kernel(AttnArgs
 // (hi, lo) operand.  Rows past T * G, or keys past a row's causal limit,
 // are masked.
 constexpr int kPreWaves = 8;
-constexpr int kPrefillMinRows = 32;                              // T * (Hq / Hkv) above this takes this kernel
+constexpr int kDecMaxRows = 32;                                  // T * (Hq / Hkv) above this takes this kernel (from 9 on: make_plan)
 constexpr int kPreNcb = 2;                                       // column blocks per wave for 16-bit q (f32 q: 1)
 constexpr int kPreCbOff = kSlutOff + kSlutBytes;                 // 16 x (fp16 hi | remainder << 16)
 constexpr int kPreStageOff = kPreCbOff + 64;                     // per wave: q rows fp16, then G q fp32
 constexpr int kPreQsrOff = kPreStageOff + kPreWaves * 32 * 128 * 2;   // per wave: 32 x f32 score scales
-constexpr int kPreLdsBytes = kPreQsrOff + kPreWaves * 32 * 4;
+constexpr int kPreLdsUse = kPreQsrOff + kPreWaves * 32 * 4;
+constexpr int kPreMerge = kPreWaves * (32 * 132 + 3 * 32 + 1) * 4;   // the waves' (m, l, O) of up to 32 rows each
+constexpr int kPreLdsBytes = kPreLdsUse > kPreMerge ? kPreLdsUse : kPreMerge;
 
-template <bool QJL, int NCB, int PF, bool QLO, bool PAGED>
+template <bool QJL, int NCB, int PF, bool QLO, bool PAGED, bool TWS>
 __global__ __launch_bounds__(64 * kPreWaves) void attn_prefill128_kernel(AttnArgs a) {
     constexpr int D = 128, QD = 64, RW = 16 * NCB;      // rows per wave
     static_assert(!QLO || NCB == 1, "the f32 remainder plane shares the 32-row stage area");
@@ -1796,9 +2031,13 @@ __global__ __launch_bounds__(64 * kPreWaves) void attn_prefill128_kernel(AttnArg
     const int64_t b = bz / a.n_rchunks;
     const int rc = (int)(bz % a.n_rchunks);
     const int nrows_total = (int)(a.T * a.G);
-    const int row0 = rc * a.rows + wave * RW;                  // first flat row of this wave
-    unsigned char *stage = smem + kPreStageOff + wave * 32 * 128 * 2;
-    float *qsr_l = reinterpret_cast<float *>(smem + kPreQsrOff) + wave * 32;
+    // TWS: 2^tw_shift waves share one group of RW rows and take its key tiles
+    // in turn (wave tw: tiles tw, tw + 2^tw_shift, ...)
+    const int tws = TWS ? a.tw_shift : 0;
+    const int tw = TWS ? wave & ((1 << tws) - 1) : 0, rg = wave >> tws;
+    const int row0 = rc * a.rows + rg * RW;                    // first flat row of this wave
+    unsigned char *stage = smem + kPreStageOff + (rg << tws) * 32 * 128 * 2;
+    float *qsr_l = reinterpret_cast<float *>(smem + kPreQsrOff) + (rg << tws) * 32;
 
     // ── LUTs (as the decode kernel) ───────────────────────────────────
     {
@@ -1811,53 +2050,12 @@ __global__ __launch_bounds__(64 * kPreWaves) void attn_prefill128_kernel(AttnArg
     }
     sign_table_store(smem, tid);      // 512 threads
 
-    // ── this wave's query rows: (sign flip,) WHT, round; per-row power-of-2
-    //    scale into fp16 range; staged as fp16 ───────────────────────────
-    {
-        const bool use_flip = a.rotate_q && a.sign_flip;
-        const bool flip_lo = use_flip && a.sign_flip[lane] < 0, flip_hi = use_flip && a.sign_flip[64 + lane] < 0;
-        // the score scale's sign goes into the staged rows (exact), so every
-        // row's score scale is >= 0 and the exponent takes it in an fma
-        const float ssign = a.qscale < 0.0f ? -1.0f : 1.0f;
-        for (int rr = 0; rr < RW; ++rr) {
-            const int rho = row0 + rr;
-            const bool ok = rho < nrows_total;
-            const int rc_ = ok ? rho : nrows_total - 1;
-            const int t = rc_ / a.G, hq = hk * a.G + (rc_ - t * a.G);
-            const int64_t base = ((b * a.Hq + hq) * a.T + t) * D;
-            float lo = load_as_f32(a.q, a.q_dtype, base + lane), hi = load_as_f32(a.q, a.q_dtype, base + 64 + lane);
-            lo = flip_lo ? -lo : lo;
-            hi = flip_hi ? -hi : hi;
-            if (a.rotate_q) {
-                wht128_lanes(lo, hi, lane);
-                lo = round_to_dtype(lo * a.wht_scale, a.q_dtype);
-                hi = round_to_dtype(hi * a.wht_scale, a.q_dtype);
-            }
-            if (!ok) lo = hi = 0.0f;
-            // row max |q| -> 2^k with max * 2^k in [2^14, 2^15)
-            float m = fmaxf(fabsf(lo), fabsf(hi));
-            m = wave_max(m);
-            int ex = 0;
-            if (m > 0.0f && m < INFINITY) { frexpf(m, &ex); }
-            const float sr = ldexpf(1.0f, 15 - imax(ex, -100));   // m * sr in [2^14, 2^15) unless m < 2^-101
-            const float los = ssign * lo * sr, his = ssign * hi * sr;
-            const uint16_t l16 = f32_to_f16_rne(los), h16 = f32_to_f16_rne(his);
-            reinterpret_cast<uint16_t *>(stage)[rr * D + lane] = l16;
-            reinterpret_cast<uint16_t *>(stage)[rr * D + 64 + lane] = h16;
-            if constexpr (QLO) {
-                // second plane: fp16 remainder of the scaled f32 row
-                uint16_t *lop = reinterpret_cast<uint16_t *>(stage) + 16 * D;
-                lop[rr * D + lane] = f32_to_f16_rne(los - f16_to_f32(l16));
-                lop[rr * D + 64 + lane] = f32_to_f16_rne(his - f16_to_f32(h16));
-            }
-            // a positive factor is kept >= FLT_MIN (one that underflows
-            // leaves every score as good as 0 either way), so a masked
-            // score's -inf stays -inf through the maximum and the exponent;
-            // a zero scale keeps 0 (inf x 0 = NaN, as the reference forms
-            // scale x score) and re-masks the exponents below
-            const float q0 = fabsf(a.qscale) / sr;
-            if (lane == 0) qsr_l[rr] = (q0 < __FLT_MIN__ && a.qscale != 0.0f) ? __FLT_MIN__ : q0;
-        }
+    // ── the group's query rows (TWS: its sets of 16 among its waves) ─────
+#pragma unroll
+    for (int c = 0; c < NCB; ++c) {
+        if (TWS && (c & ((1 << tws) - 1)) != tw) continue;
+        stage_rows<D, 1, QLO>(a, b, hk, row0 + 16 * c, nrows_total, lane, reinterpret_cast<uint16_t *>(stage) + 16 * c * D,
+                              16 * D, qsr_l + 16 * c);
     }
     __syncthreads();
 
@@ -1885,7 +2083,7 @@ __global__ __launch_bounds__(64 * kPreWaves) void attn_prefill128_kernel(AttnArg
         const uint16_t *qrow = reinterpret_cast<const uint16_t *>(stage) + (16 * c + n) * D;
 #pragma unroll
         for (int s = 0; s < 8; ++s) {
-            const uint2 w = *reinterpret_cast<const uint2 *>(qrow + 32 * g + 4 * s);
+            const uint2 w = *reinterpret_cast<const uint2 *>(qrow + 8 * ((4 * g + (s >> 1)) ^ n) + 4 * (s & 1));
             bk[c][s] = as_half8(w.x, w.x, w.y, w.y);
         }
         qsr[c] = qsr_l[16 * c + n];
@@ -1893,7 +2091,7 @@ __global__ __launch_bounds__(64 * kPreWaves) void attn_prefill128_kernel(AttnArg
             const uint16_t *lrow = reinterpret_cast<const uint16_t *>(stage) + 16 * D + (16 * c + n) * D;
 #pragma unroll
             for (int s = 0; s < 8; ++s) {
-                const uint2 w = *reinterpret_cast<const uint2 *>(lrow + 32 * g + 4 * s);
+                const uint2 w = *reinterpret_cast<const uint2 *>(lrow + 8 * ((4 * g + (s >> 1)) ^ n) + 4 * (s & 1));
                 bkl[c][s] = as_half8(w.x, w.x, w.y, w.y);
             }
         }
@@ -1909,6 +2107,7 @@ __global__ __launch_bounds__(64 * kPreWaves) void attn_prefill128_kernel(AttnArg
         const uint32_t *gh = a.g_bits + (int64_t)hk * QD * 4;
 #pragma unroll
         for (int ob = 0; ob < 4; ++ob) {
+            if (TWS && (ob & ((1 << tws) - 1)) != tw) continue;    // another wave of the group (wave-uniform)
             const uint4 gw = *reinterpret_cast<const uint4 *>(gh + (16 * ob + n) * 4);
             const uint32_t gws[4] = {gw.x, gw.y, gw.z, gw.w};
 #pragma unroll
@@ -1917,13 +2116,13 @@ __global__ __launch_bounds__(64 * kPreWaves) void attn_prefill128_kernel(AttnArg
 #pragma unroll
                 for (int c = 0; c < NCB; ++c) {
                     const uint4 qv = *reinterpret_cast<const uint4 *>(reinterpret_cast<const uint16_t *>(stage) +
-                                                                     (16 * c + n) * D + 32 * s + 8 * g);
+                                                                     (16 * c + n) * D + 8 * ((4 * s + g) ^ n));
                     gacc[c][ob] = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_half8(qv.x, qv.y, qv.z, qv.w), bg,
                                                                         gacc[c][ob], 0, 0, 0);
                     if constexpr (QLO) {
                         // the f32 row's fp16 remainder plane
                         const uint4 lv = *reinterpret_cast<const uint4 *>(reinterpret_cast<const uint16_t *>(stage) +
-                                                                         16 * D + (16 * c + n) * D + 32 * s + 8 * g);
+                                                                         16 * D + (16 * c + n) * D + 8 * ((4 * s + g) ^ n));
                         gacc[c][ob] = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_half8(lv.x, lv.y, lv.z, lv.w), bg,
                                                                             gacc[c][ob], 0, 0, 0);
                     }
@@ -1933,13 +2132,18 @@ __global__ __launch_bounds__(64 * kPreWaves) void attn_prefill128_kernel(AttnArg
     }
     // gacc[c][ob][i] = (staged) G q for row 16 c + 4 g + i, output 16 ob + n:
     // through the stage area (q is no longer needed) into B layout
-    float *gqs = reinterpret_cast<float *>(stage);     // [RW][64]
+    // (TWS: through the next wave's area, q is still being read; each wave
+    // writes the outputs that it formed)
+    float *gqs = reinterpret_cast<float *>(stage + (TWS ? 32 * 128 * 2 : 0));     // [RW][64]
 #pragma unroll
-    for (int c = 0; c < NCB; ++c)
+    for (int ob = 0; ob < 4; ++ob) {
+        if (TWS && (ob & ((1 << tws) - 1)) != tw) continue;
 #pragma unroll
-        for (int ob = 0; ob < 4; ++ob)
+        for (int c = 0; c < NCB; ++c)
 #pragma unroll
             for (int i = 0; i < 4; ++i) gqs[(16 * c + 4 * g + i) * QD + 16 * ob + n] = gacc[c][ob][i];
+    }
+    if constexpr (TWS) __syncthreads();
 #pragma unroll
     for (int c = 0; c < NCB; ++c) {
         // B carries sqrt(2/pi) / D on the staged (2^k-scaled) G q (fp16 hi in
@@ -1969,6 +2173,7 @@ __global__ __launch_bounds__(64 * kPreWaves) void attn_prefill128_kernel(AttnArg
         for (int c = 0; c < NCB; ++c)
 #pragma unroll
             for (int s = 0; s < 2; ++s) {
+                if (TWS && ((c * 2 + s) & ((1 << tws) - 1)) != tw) continue;
                 img[((c * 2 + s) * 2) * 64 + lane] = __builtin_bit_cast(uint4, bgq[c][s]);
                 img[((c * 2 + s) * 2 + 1) * 64 + lane] = __builtin_bit_cast(uint4, bgl[c][s]);
             }
@@ -2039,13 +2244,14 @@ __global__ __launch_bounds__(64 * kPreWaves) void attn_prefill128_kernel(AttnArg
     // are loaded in order, so the next tile's page ids are requested here
     // and waited for only at the next call)
     int32_t pid[2] = {0, 0};
-    if constexpr (PAGED) paged_page_ids(a, pt_row, s_begin, pid);
+    const int stride = kDecTile << tws, s_first = s_begin + tw * kDecTile;
+    if constexpr (PAGED) paged_page_ids(a, pt_row, s_first, pid);
     auto load_tile = [&](TileRaw &R, int t) {
         if constexpr (PAGED) {
             uint32_t rb[2];
             paged_rows(a, pid, hk, t, s_end, page_bad, rb);
             tile_load_paged<QJL>(R, P, OFS, rb);
-            paged_page_ids(a, pt_row, t + kDecTile, pid);
+            paged_page_ids(a, pt_row, t + stride, pid);
         } else {
             tile_load<QJL>(R, P, OFS, t);
         }
@@ -2271,12 +2477,11 @@ __global__ __launch_bounds__(64 * kPreWaves) void attn_prefill128_kernel(AttnArg
         }
     };
 
-    // every key tile, in order, with the decode kernel's unconditional ring
-    constexpr int stride = kDecTile;
+    // this wave's key tiles, in order, with the decode kernel's unconditional ring
     TileRaw ring[PF];
 #pragma unroll
-    for (int p = 0; p < PF - 1; ++p) load_tile(ring[p], s_begin + p * stride);
-    int tt0 = s_begin;
+    for (int p = 0; p < PF - 1; ++p) load_tile(ring[p], s_first + p * stride);
+    int tt0 = s_first;
     for (; tt0 + (PF - 1) * stride < s_end; tt0 += PF * stride) {
 #pragma unroll
         for (int p = 0; p < PF; ++p) {
@@ -2309,6 +2514,38 @@ __global__ __launch_bounds__(64 * kPreWaves) void attn_prefill128_kernel(AttnArg
     int le = lane;
     asm volatile("" : "+v"(le));
     const int ne = le & 15, ge = le >> 4;
+    if constexpr (TWS) {
+        // merge the group's waves: their (m, l, O) through LDS (the tables
+        // are dead), weighted by exp2(m - max) in wave order
+        constexpr int kStride = D + 4, kSlab = RW * kStride;
+        static_assert(kPreWaves * (kSlab + 3 * RW + 1) * 4 <= kPreLdsBytes, "the waves' states fit");
+        float *ob = reinterpret_cast<float *>(smem) + wave * kSlab;
+        float *ml = reinterpret_cast<float *>(smem) + kPreWaves * kSlab;       // [wave][row]: m (then its weight), l
+        float *lt = ml + kPreWaves * 2 * RW;                                     // [group][row]: l
+        float *bad = lt + kPreWaves * RW;                                        // [wave]
+        __syncthreads();
+#pragma unroll
+        for (int c = 0; c < NCB; ++c) {
+            const int r = 16 * c + ne;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int k = 0; k < 8; k += 4)
+                    *reinterpret_cast<float4 *>(ob + r * kStride + 8 * (4 * ge + i) + k) =
+                        make_float4(oacc[c][k][i], oacc[c][k + 1][i], oacc[c][k + 2][i], oacc[c][k + 3][i]);
+            if (ge == 0) {
+                ml[(wave * RW + r) * 2] = m_run[c];
+                ml[(wave * RW + r) * 2 + 1] = lacc[c][0];
+            }
+        }
+        if (le == 0) bad[wave] = (seq_bad || page_bad || len_bad) ? 1.0f : 0.0f;
+        __syncthreads();
+        merge_weights<RW>(ml, lt, bad, tid, kPreWaves >> tws, tws);
+        __syncthreads();
+        merge_rows<D, RW>(a, reinterpret_cast<const float *>(smem), ml, lt, tid, 64 * kPreWaves, kPreWaves >> tws, tws,
+                          rc, nrows_total, b, hk, unit, split);
+        return;
+    }
 #pragma unroll
     for (int c = 0; c < NCB; ++c) {
         const int rho = row0 + 16 * c + ne;
@@ -2350,7 +2587,12 @@ __global__ __launch_bounds__(64 * kPreWaves) void attn_prefill128_kernel(AttnArg
 //           4g .. 4g + 3 and forms pair bytes (two tokens' nibbles at dim 2n
 //           or 2n + 1), whose LUT entries are MFMA-ready (hi, lo) pairs
 // Online softmax in the exp2 domain with P in fp16, summed by an MFMA
-// against ones, as in the other kernels.
+// against ones, as in the other kernels; the token-split variant (few rows:
+// a decode step) adds P's fp16 remainder, 3 MFMAs a tile and 5 % of the time.
+// A decode step (32 sequences of 8192 tokens, 8 kv heads, 4 rows each, 80 MB)
+// took 71.4 us on the generic kernel (16-token tiles, one in flight, byte
+// loads of V per token) and takes 26.9 us here: bound by the issue of LDS
+// reads and VALU work, not by the 11 us that its bytes take.
 #ifndef OMNI_P32_WAVES
 #define OMNI_P32_WAVES 8
 #endif
@@ -2388,22 +2630,12 @@ __device__ __forceinline__ void tile_load32(TileRaw32 &R, const DecBufs &P, int 
         R.v[i] = __builtin_amdgcn_raw_buffer_load_b8(P.vn, (t + 16u * (i / 4) + 4u * g + (i % 4)) * 16u + (uint32_t)n, 0, 0);
 }
 
-// Normalized 32-point WHT of the element (lane % 32) of each half-wave's
-// row (_wht_torch order, fp32; an fma with +-1 rounds as the add/subtract).
-__device__ __forceinline__ float wht32_lane(float x, int lane) {
-    x = __builtin_fmaf((lane & 1) ? -1.0f : 1.0f, x, xor_partner<1>(x, lane));
-    x = __builtin_fmaf((lane & 2) ? -1.0f : 1.0f, x, xor_partner<2>(x, lane));
-    x = __builtin_fmaf((lane & 4) ? -1.0f : 1.0f, x, xor_partner<4>(x, lane));
-    x = __builtin_fmaf((lane & 8) ? -1.0f : 1.0f, x, xor_partner<8>(x, lane));
-    x = __builtin_fmaf((lane & 16) ? -1.0f : 1.0f, x, xor_partner<16>(x, lane));
-    return x;
-}
-
-template <bool QJL, int NCB, bool QLO>
-__global__ __launch_bounds__(64 * kP32Waves) void attn_prefill32_kernel(AttnArgs a) {
+template <bool QJL, int NCB, bool QLO, int NW, bool TWS>
+__global__ __launch_bounds__(64 * NW) void attn_prefill32_kernel(AttnArgs a) {
     constexpr int D = 32, QD = 16, RW = 16 * NCB;       // rows per wave
     static_assert(RW * D * 2 * (QLO ? 2 : 1) <= kP32StageBytes && RW * QD * 4 <= kP32StageBytes,
                   "q rows (and the f32 remainder plane), then G q, fit the wave's stage area");
+    static_assert(NW == kP32Waves || (TWS && NW == 16 && NCB == 1), "sixteen waves share one group of 16 rows");
     __shared__ __attribute__((aligned(16))) unsigned char smem[kP32LdsBytes];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -2413,9 +2645,14 @@ __global__ __launch_bounds__(64 * kP32Waves) void attn_prefill32_kernel(AttnArgs
     const int64_t b = bz / a.n_rchunks;
     const int rc = (int)(bz % a.n_rchunks);
     const int nrows_total = (int)(a.T * a.G);
-    const int row0 = rc * a.rows + wave * RW;
-    uint16_t *stage = reinterpret_cast<uint16_t *>(smem + kP32StageOff + wave * kP32StageBytes);
-    float *qsr_l = reinterpret_cast<float *>(smem + kP32QsrOff) + wave * 64;
+    // TWS: 2^tw_shift waves share one group of RW rows and take its key tiles
+    // in turn, as in the head_dim-128 kernel
+    const int tws = TWS ? (NW == 16 ? 4 : a.tw_shift) : 0;
+    const int tw = TWS ? wave & ((1 << tws) - 1) : 0, rg = wave >> tws;
+    const int row0 = rc * a.rows + rg * RW;
+    unsigned char *stage_b = smem + kP32StageOff + (rg << tws) * kP32StageBytes;
+    uint16_t *stage = reinterpret_cast<uint16_t *>(stage_b);
+    float *qsr_l = reinterpret_cast<float *>(smem + kP32QsrOff) + (rg << tws) * 64;
 
     // ── codebook pairs and the sign table ───────────────────────────────
     {
@@ -2428,48 +2665,15 @@ __global__ __launch_bounds__(64 * kP32Waves) void attn_prefill32_kernel(AttnArgs
     }
     if (tid < 512) sign_table_store(smem, tid);
 
-    // ── this wave's query rows, two per pass (half-waves): (sign flip,)
-    //    WHT, round; per-row power-of-2 scale into fp16 range; fp16 stage.
-    //    The score scale's sign goes into the staged rows (exact), so every
-    //    row's score scale qsr is >= 0 and the exponent takes it in an fma ──
-    {
-        const int e = lane & 31, half = lane >> 5;
-        const bool flip = a.rotate_q && a.sign_flip && a.sign_flip[e] < 0;
-        const float ssign = a.qscale < 0.0f ? -1.0f : 1.0f;
-        for (int rp = 0; rp < RW; rp += 2) {
-            const int rr = rp + half;
-            const int rho = row0 + rr;
-            const bool ok = rho < nrows_total;
-            const int rcl = ok ? rho : nrows_total - 1;
-            const int t = rcl / a.G, hq = hk * a.G + (rcl - t * a.G);
-            float x = load_as_f32(a.q, a.q_dtype, ((b * a.Hq + hq) * a.T + t) * D + e);
-            x = flip ? -x : x;
-            if (a.rotate_q) x = round_to_dtype(wht32_lane(x, lane) * a.wht_scale, a.q_dtype);
-            if (!ok) x = 0.0f;
-            float m = fabsf(x);
-#pragma unroll
-            for (int sh = 16; sh >= 1; sh >>= 1) m = fmaxf(m, __shfl_xor(m, sh));
-            int ex = 0;
-            if (m > 0.0f && m < INFINITY) frexpf(m, &ex);
-            const float sr = ldexpf(1.0f, 15 - imax(ex, -100));
-            const float xs = ssign * x * sr;
-            const uint16_t x16 = f32_to_f16_rne(xs);
-            stage[rr * D + e] = x16;
-            if constexpr (QLO) stage[RW * D + rr * D + e] = f32_to_f16_rne(xs - f16_to_f32(x16));
-            // kept >= FLT_MIN (a positive scale that underflows here leaves
-            // every score as good as 0 either way): the softmax below
-            // relies on -inf x qsr = -inf.  A zero scale runs elsewhere.
-            const float q0 = fabsf(a.qscale) / sr;
-            if (e == 0) qsr_l[rr] = q0 < __FLT_MIN__ ? __FLT_MIN__ : q0;
-        }
-    }
+    // ── the group's query rows (TWS: by one of its waves) ──────────────
+    if (tw == 0) stage_rows<D, NCB, QLO>(a, b, hk, row0, nrows_total, lane, stage, RW * D, qsr_l);
     __syncthreads();
 
     // ── byte LUT (after the codebook pairs are visible): entry e, 16-byte
     //    chunk k (two of its 32 copies) per item ───────────────────────────
     {
         const uint32_t *cbh = reinterpret_cast<const uint32_t *>(smem + kP32CbOff);
-        for (int it = tid; it < 256 * 16; it += 64 * kP32Waves) {
+        for (int it = tid; it < 256 * 16; it += 64 * NW) {
             const int e = it >> 4;
             const uint32_t w0 = cbh[e & 15], w1 = cbh[e >> 4];
             const uint32_t hp = __builtin_amdgcn_perm(w1, w0, 0x05040100u);
@@ -2506,6 +2710,7 @@ __global__ __launch_bounds__(64 * kP32Waves) void attn_prefill32_kernel(AttnArgs
         const half8_t bg = sign_halves(smem, gw, 8u * g, (uint32_t)kSlutOff | ((uint32_t)(lane & 31) * 8u));
 #pragma unroll
         for (int c = 0; c < NCB; ++c) {
+            if (TWS && (c & ((1 << tws) - 1)) != tw) continue;     // another wave of the group (wave-uniform)
             const uint4 qv = *reinterpret_cast<const uint4 *>(stage + (16 * c + n) * D + 8 * g);
             gacc[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_half8(qv.x, qv.y, qv.z, qv.w), bg, gacc[c], 0, 0, 0);
             if constexpr (QLO) {
@@ -2517,11 +2722,15 @@ __global__ __launch_bounds__(64 * kP32Waves) void attn_prefill32_kernel(AttnArgs
     // through the stage area (q is no longer read) into the QJL B layout:
     // column n = row 16 c + n; k-slots 8g .. 8g + 7 = projections 8 (g % 2)
     // .. + 7 as fp16 hi (g < 2) or fp16 remainder (g >= 2)
-    float *gqs = reinterpret_cast<float *>(stage);      // [RW][16]
+    // (TWS: through the next wave's area, q is still being read)
+    float *gqs = reinterpret_cast<float *>(stage_b + (TWS ? kP32StageBytes : 0));      // [RW][16]
 #pragma unroll
-    for (int c = 0; c < NCB; ++c)
+    for (int c = 0; c < NCB; ++c) {
+        if (TWS && (c & ((1 << tws) - 1)) != tw) continue;
 #pragma unroll
         for (int i = 0; i < 4; ++i) gqs[(16 * c + 4 * g + i) * QD + n] = gacc[c][i];
+    }
+    if constexpr (TWS) __syncthreads();
 #pragma unroll
     for (int c = 0; c < NCB; ++c) {
         const float *row = gqs + (16 * c + n) * QD + 8 * (g & 1);
@@ -2737,12 +2946,26 @@ __global__ __launch_bounds__(64 * kP32Waves) void attn_prefill32_kernel(AttnArgs
             float ex[8];
 #pragma unroll
             for (int k = 0; k < 8; ++k) ex[k] = __builtin_fmaf(sc[c][k], qmul[c], nm);
-            uint32_t pw[4];
+            uint32_t pw[4], pr[4];
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
-                pw[j] = cvt_pk_h2(__builtin_amdgcn_exp2f(ex[2 * j]), __builtin_amdgcn_exp2f(ex[2 * j + 1]));
+            for (int j = 0; j < 4; ++j) {
+                const float p0 = __builtin_amdgcn_exp2f(ex[2 * j]), p1 = __builtin_amdgcn_exp2f(ex[2 * j + 1]);
+                pw[j] = cvt_pk_h2(p0, p1);
+                if constexpr (TWS) {
+                    const half2_t ph2 = __builtin_bit_cast(half2_t, pw[j]);
+                    pr[j] = cvt_pk_h2(p0 - (float)ph2.x, p1 - (float)ph2.y);
+                }
+            }
             const half8_t pb = as_half8(pw[0], pw[1], pw[2], pw[3]);
             lacc[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ones, pb, lacc[c], 0, 0, 0);
+            if constexpr (TWS) {
+                // P's fp16 remainder (against the codebook's hi plane), so
+                // that a call of few rows keeps P to 22 bits
+                const half8_t pl8 = as_half8(pr[0], pr[1], pr[2], pr[3]);
+                lacc[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ones, pl8, lacc[c], 0, 0, 0);
+                oacc[c][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahv[0], pl8, oacc[c][0], 0, 0, 0);
+                oacc[c][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahv[1], pl8, oacc[c][1], 0, 0, 0);
+            }
 #pragma unroll
             for (int p = 0; p < 2; ++p) {
                 oacc[c][p] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahv[p], pb, oacc[c][p], 0, 0, 0);
@@ -2751,12 +2974,12 @@ __global__ __launch_bounds__(64 * kP32Waves) void attn_prefill32_kernel(AttnArgs
         }
     };
 
-    // every key tile, in order, with a two-slot ring of unconditional loads
+    // this wave's key tiles, in order, with a two-slot ring of unconditional loads
     // (past the split end they read 0 and touch no memory)
-    constexpr int stride = kDecTile;
+    const int stride = kDecTile << tws, s_first = s_begin + tw * kDecTile;
     TileRaw32 ring[2];
-    tile_load32<QJL>(ring[0], P, n, g, s_begin);
-    int tt0 = s_begin;
+    tile_load32<QJL>(ring[0], P, n, g, s_first);
+    int tt0 = s_first;
     for (; tt0 + stride < s_end; tt0 += 2 * stride) {
         __builtin_amdgcn_sched_barrier(0);
         tile_load32<QJL>(ring[1], P, n, g, tt0 + stride);
@@ -2771,6 +2994,35 @@ __global__ __launch_bounds__(64 * kP32Waves) void attn_prefill32_kernel(AttnArgs
 
     // ── rows out (or split partials): oacc[c][p][i] is dim 8g + 2i + p ────
     const int64_t unit = (b * a.Hkv + hk) * a.n_rchunks + rc;
+    if constexpr (TWS) {
+        // merge the group's waves (see the head_dim-128 kernel)
+        constexpr int kStride = D + 4, kSlab = RW * kStride;
+        static_assert(NW * (kSlab + 3 * RW + 1) * 4 <= kP32LdsBytes, "the waves' states fit");
+        float *ob = reinterpret_cast<float *>(smem) + wave * kSlab;
+        float *ml = reinterpret_cast<float *>(smem) + NW * kSlab;
+        float *lt = ml + NW * 2 * RW;
+        float *bad = lt + NW * RW;
+        __syncthreads();
+#pragma unroll
+        for (int c = 0; c < NCB; ++c) {
+            const int r = 16 * c + n;
+#pragma unroll
+            for (int i = 0; i < 4; i += 2)
+                *reinterpret_cast<float4 *>(ob + r * kStride + 8 * g + 2 * i) =
+                    make_float4(oacc[c][0][i], oacc[c][1][i], oacc[c][0][i + 1], oacc[c][1][i + 1]);
+            if (g == 0) {
+                ml[(wave * RW + r) * 2] = m_run[c];
+                ml[(wave * RW + r) * 2 + 1] = lacc[c][0];
+            }
+        }
+        if (lane == 0) bad[wave] = seq_bad ? 1.0f : 0.0f;
+        __syncthreads();
+        merge_weights<RW>(ml, lt, bad, tid, NW >> tws, tws);
+        __syncthreads();
+        merge_rows<D, RW>(a, reinterpret_cast<const float *>(smem), ml, lt, tid, 64 * NW, NW >> tws, tws, rc, nrows_total,
+                          b, hk, unit, split);
+        return;
+    }
 #pragma unroll
     for (int c = 0; c < NCB; ++c) {
         const int rho = row0 + 16 * c + n;
@@ -2804,7 +3056,8 @@ __global__ __launch_bounds__(64 * kP32Waves) void attn_prefill32_kernel(AttnArgs
 struct Plan {
     bool dec128;       // D == 128: decode kernel with 8 query rows per block
     bool prefill;      // D == 128 with many rows per kv head: prefill kernel
-    bool prefill32;    // D == 32 with many rows per kv head: head_dim-32 prefill kernel
+    bool prefill32;    // D == 32: head_dim-32 prefill kernel
+    int ncb, tws;      // prefill kernels: 16-row column blocks per wave, log2 of the waves sharing them
     int rows, n_rchunks, splits, nw, ncopy;
     int spb;           // decode kernel: sequences sharing a block's 8 row slots
     int64_t split_len;
@@ -2813,75 +3066,162 @@ struct Plan {
 
 static int64_t clamp64(int64_t v, int64_t lo, int64_t hi) { return v < lo ? lo : (v > hi ? hi : v); }
 
+// Static array of omni_attn_noalloc.
+constexpr size_t kScratchBytes = size_t(16) << 20;
+
+// Splits of each unit's `tiles` key tiles, one block per CU at a time, and
+// the call's estimated time in us: rounds of blocks x (a block's fixed part +
+// its tiles) + the combine launch and the partials' way through memory.  The
+// fixed part and the time per tile are measured; the rounds decide: 24 units
+// in 11 splits are 264 blocks on 256 CUs, twice the time of 10 splits (decode
+// of 3 x 20011 tokens, 8 rows: 54.5 us so, 23.6 us in 10 splits with the wider
+// combine).  Candidates: no split, and the most that 1, 2 or 3 full rounds
+// hold with at least kMinSplitTiles tiles each; a split has to promise a
+// tenth (a second, partly filled round runs faster than a full one).
+constexpr int64_t kMinSplitTiles = 4;
+constexpr double kCombineUs = 6.0;
+constexpr double kPartialUsPerByte = 2.0 / 3.5e6;     // written and read, 3.5 TB/s
+
+static double plan_splits(int64_t cus, int64_t units, int64_t tiles, int rows, int D, double fixed, double per_tile, int64_t least,
+                          int64_t &splits) {
+    const int64_t most = tiles / kMinSplitTiles > 1 ? tiles / kMinSplitTiles : 1;
+    if (most == 1 && least <= 1) {            // a short sequence, planned on every small call: no more divisions
+        splits = 1;
+        return (double)((units + cus - 1) / cus) * (fixed + per_tile * (double)tiles);
+    }
+    const size_t unit_bytes = (size_t)rows * (D + 2) * sizeof(float);
+    // as many as one block per CU asks for, of at least 16 tiles, whatever
+    // their partials take; more only while those fit the static array
+    const int64_t plain = clamp64((cus + units - 1) / units, 1, tiles / 16 > 1 ? tiles / 16 : 1);
+    const int64_t fit = (int64_t)(kScratchBytes / (unit_bytes * (size_t)units));
+    const int64_t cap = fit > plain ? fit : plain;
+    double best = 0.0;
+    splits = 0;
+    for (int r = 0; r <= 3; ++r) {
+        int64_t s = r == 0 ? 1 : clamp64(r * cus / units, 1, most < cap ? most : cap);
+        if (s < least) s = least;
+        const double rounds = (double)((units * s + cus - 1) / cus);
+        double t = rounds * (fixed + per_tile * (double)((tiles + s - 1) / s));
+        if (s > 1) t += kCombineUs + (double)(unit_bytes * (size_t)(units * s)) * kPartialUsPerByte;
+        if (splits == 0 || t < (splits == 1 ? 0.9 * best : best)) {
+            best = t;
+            splits = s;
+        }
+    }
+    return best;
+}
+
 // `zero_scale`: a score scale of exactly 0.  The decode and head_dim-32
 // prefill kernels need a positive score factor (a masked key's -inf must
 // stay -inf through it); a zero scale, where an infinite score gives NaN
 // (inf x 0, as the reference forms scale x score), runs the head_dim-128
 // prefill kernel or the generic one instead, which keep the factor 0.
-static Plan make_plan(int64_t B, int Hq, int Hkv, int64_t T, int64_t S, int D, bool q32, bool paged = false,
+//
+// Rows of a prefill block: its waves hold 16 * ncb rows each, and as many of
+// them as the rows leave over share a group of rows and split its key tiles
+// (2^tws waves per group; 1 from 129 rows on, 257 at head_dim 32).
+//
+// D = 128, 9 to 32 rows per kv head: eight per decode block, so that several
+// blocks decode the same cache at the same time, or one prefill block: the
+// smaller estimate.  (Decode holds while its blocks fit the chip at once: 24
+// rows, 8 sequences of 100 tokens 7.7 against 15 us; the prefill kernel where
+// they do not: 32 sequences of 4096 tokens 85 against 54 us.)
+static Plan make_plan(int cus, int64_t B, int Hq, int Hkv, int64_t T, int64_t S, int D, bool q32, bool paged = false,
                       bool zero_scale = false) {
     Plan p;
     const int G = Hq / Hkv;
-    const int cus = device_cus();
-    p.prefill = (D == 128) && (T * G > kPrefillMinRows || zero_scale);
-    p.prefill32 = (D == 32) && T * G > kPrefillMinRows && !zero_scale;
-    p.dec128 = (D == 128) && !p.prefill;
-    p.rows = p.prefill ? kPreWaves * 16 * (q32 ? 1 : kPreNcb)
-                       : (p.prefill32 ? kP32Waves * 16 * (q32 ? 2 : kP32Ncb) : (p.dec128 ? kDecRows : kRows));
-    p.n_rchunks = (int)((T * G + p.rows - 1) / p.rows);
-    // Short decode steps of many sequences (more (sequence, kv head) pairs
-    // than CUs, at most 4 query rows each): two sequences share a block's 8
-    // row slots, halving the blocks (and the per-block prologues) without
-    // idling any slot.
-    p.spb = (p.dec128 && T * G <= kDecRows / 2 && B >= 2 && B * (int64_t)Hkv > cus) ? 2 : 1;
-    const int64_t units = ((B + p.spb - 1) / p.spb) * (int64_t)Hkv * p.n_rchunks;
-    if (p.prefill || p.prefill32) {
-        const int64_t tiles = (S + kDecTile - 1) / kDecTile;
-        int64_t splits = clamp64((cus + units - 1) / (units > 0 ? units : 1), 1, (tiles / 16) > 1 ? tiles / 16 : 1);
-        const int64_t tps = (tiles + splits - 1) / splits;
-        p.splits = (int)splits;
-        p.split_len = tps * kDecTile;
-        p.nw = p.prefill ? kPreWaves : kP32Waves;
-        p.ncopy = 32;
-        p.lds = p.prefill ? kPreLdsBytes : kP32LdsBytes;
-    } else if (p.dec128) {
-        const int64_t tiles = (S + kDecTile - 1) / kDecTile;
-        int64_t splits = clamp64((cus + units - 1) / (units > 0 ? units : 1), 1, (tiles / 16) > 1 ? tiles / 16 : 1);
-        if (p.spb > 1) splits = 1;
-        // paged: splits short enough for every half's pool row to be staged
-        if (paged && p.spb == 1) {
-            const int64_t cap = kDecPtMax / 2;
-            if (tiles > splits * cap) splits = (tiles + cap - 1) / cap;
-        }
-        const int64_t tps = (tiles + splits - 1) / splits;
-        p.splits = (int)splits;
-        p.split_len = tps * kDecTile;
-        p.nw = kDecWaves;
-        p.ncopy = 32;
-        p.lds = kDecLdsBytes;
-    } else {
-        const int64_t tiles = (S + kTile - 1) / kTile;
-        int64_t splits = clamp64((2 * (int64_t)cus + units - 1) / (units > 0 ? units : 1), 1,
-                                 tiles / (2 * kMaxWaves) > 1 ? tiles / (2 * kMaxWaves) : 1);
-        const int64_t tps = (tiles + splits - 1) / splits;
+    const int64_t rows = T * G;
+    const int64_t tiles = (S + kDecTile - 1) / kDecTile;
+    p.prefill = p.prefill32 = p.dec128 = false;
+    p.ncb = 1;
+    p.tws = 0;
+    p.spb = 1;
+    p.ncopy = 32;
+    if (D == 32 && zero_scale) {
+        p.rows = kRows;
+        p.n_rchunks = (int)((rows + p.rows - 1) / p.rows);
+        const int64_t units = B * (int64_t)Hkv * p.n_rchunks;
+        const int64_t t16 = (S + kTile - 1) / kTile;
+        const int64_t splits = clamp64((2 * (int64_t)cus + units - 1) / (units > 0 ? units : 1), 1,
+                                       t16 / (2 * kMaxWaves) > 1 ? t16 / (2 * kMaxWaves) : 1);
+        const int64_t tps = (t16 + splits - 1) / splits;
         p.splits = (int)splits;
         p.split_len = tps * kTile;
         p.nw = (int)clamp64((tps + 1) / 2, 1, kMaxWaves);
         p.ncopy = tps >= 64 ? 16 : (tps >= 8 ? 4 : 1);
-        p.lds = D == 128 ? Lds<128>::total(p.ncopy, p.nw) : Lds<32>::total(p.ncopy, p.nw);
+        p.lds = Lds<32>::total(p.ncopy, p.nw);
+        p.ws_bytes = p.splits > 1 ? (size_t)units * p.splits * p.rows * (D + 2) * sizeof(float) : 0;
+        return p;
     }
+    int64_t splits = 1, units = 0;
+    // the prefill kernel's plan (D = 32: any number of rows)
+    const int nw = D == 128 ? kPreWaves : kP32Waves;
+    const int ncb = D == 128 ? ((q32 || rows <= 16) ? 1 : kPreNcb) : (rows <= 16 ? 1 : ((q32 || rows <= 32) ? 2 : kP32Ncb));
+    const int64_t groups = (rows + 16 * ncb - 1) / (16 * ncb);
+    int rg = 1, tws = 0;
+    while (rg < nw && rg < groups) rg *= 2;
+    while ((rg << tws) < nw) ++tws;
+    const int prows = 16 * ncb * rg;
+    const int64_t punits = B * Hkv * ((rows + prows - 1) / prows);
+    // measured: fixed part, and a tile of one group of rows (of all the
+    // block's groups when its waves share none)
+    const double pfix = D == 128 ? (ncb == 1 ? 11.0 : 14.5) : (ncb == 1 ? 6.0 : 9.0);
+    const double ptile = (D == 128 ? (ncb == 1 ? 1.9 : 2.3) : (ncb == 1 ? 0.6 : (ncb == 2 ? 0.8 : 1.3))) / (1 << tws);
+    const bool dec = D == 128 && rows <= kDecMaxRows && !zero_scale;      // the decode kernel can take it
+    int64_t psplits = 1;
+    double pcost = 0.0;
+    if (!dec || rows > kDecRows) pcost = plan_splits(cus, punits > 0 ? punits : 1, tiles, prows, D, pfix, ptile, 1, psplits);
+    if (dec) {
+        const int n_rchunks = (int)((rows + kDecRows - 1) / kDecRows);
+        // Short decode steps of many sequences (more (sequence, kv head)
+        // pairs than CUs, at most 4 query rows each): two sequences share a
+        // block's 8 row slots, halving the blocks (and the per-block
+        // prologues) without idling any slot.
+        const int spb = (rows <= kDecRows / 2 && B >= 2 && B * (int64_t)Hkv > cus) ? 2 : 1;
+        const int64_t dunits = ((B + spb - 1) / spb) * (int64_t)Hkv * n_rchunks;
+        // paged: splits short enough for every half's pool row to be staged
+        const int64_t cap = kDecPtMax / 2;
+        const int64_t least = (paged && spb == 1 && tiles > cap) ? (tiles + cap - 1) / cap : 1;
+        int64_t dsplits = 1;
+        double dcost = 0.0;
+        if (spb == 1) dcost = plan_splits(cus, dunits > 0 ? dunits : 1, tiles, kDecRows, D, 6.5, 0.19, least, dsplits);
+        if (rows <= kDecRows || dcost <= 1.1 * pcost) {
+            p.dec128 = true;
+            p.rows = kDecRows;
+            p.n_rchunks = n_rchunks;
+            p.spb = spb;
+            p.nw = kDecWaves;
+            p.lds = kDecLdsBytes;
+            splits = dsplits;
+            units = dunits;
+        }
+    }
+    if (!p.dec128) {
+        p.prefill = D == 128;
+        p.prefill32 = D == 32;
+        p.ncb = ncb;
+        p.tws = tws;
+        p.rows = prows;
+        p.n_rchunks = (int)((rows + prows - 1) / prows);
+        p.nw = D == 32 && ncb == 1 ? 16 : nw;
+        p.lds = p.prefill ? kPreLdsBytes : kP32LdsBytes;
+        splits = psplits;
+        units = punits;
+    }
+    const int64_t tps = (tiles + splits - 1) / splits;
+    p.splits = (int)((tiles + tps - 1) / tps);         // none empty
+    p.split_len = tps * kDecTile;
     p.ws_bytes = p.splits > 1 ? (size_t)units * p.splits * p.rows * (D + 2) * sizeof(float) : 0;
     return p;
 }
 
 // Split-K workspace of a contiguous-cache call, whatever its score scale
 // (a zero scale may take another kernel).
-static size_t plan_ws_bytes(int64_t B, int Hq, int Hkv, int64_t T, int64_t S, int D, bool q32) {
-    const size_t a = make_plan(B, Hq, Hkv, T, S, D, q32).ws_bytes;
-    const size_t b = make_plan(B, Hq, Hkv, T, S, D, q32, false, true).ws_bytes;
+static size_t plan_ws_bytes(int cus, int64_t B, int Hq, int Hkv, int64_t T, int64_t S, int D, bool q32) {
+    const size_t a = make_plan(cus, B, Hq, Hkv, T, S, D, q32).ws_bytes;
+    const size_t b = make_plan(cus, B, Hq, Hkv, T, S, D, q32, false, true).ws_bytes;
     return a > b ? a : b;
 }
-
 }  // namespace omni
 
 using namespace omni;
@@ -2889,8 +3229,9 @@ using namespace omni;
 extern "C" size_t omni_attn_workspace_size(int64_t B, int Hq, int Hkv, int64_t T, int64_t S, int head_dim) {
     if (B <= 0 || Hq <= 0 || Hkv <= 0 || T <= 0 || S <= 0 || Hq % Hkv || !head_dim_ok(head_dim)) return 0;
     // the prefill plan differs for f32 queries: size for either
-    const size_t a = plan_ws_bytes(B, Hq, Hkv, T, S, head_dim, false);
-    const size_t b = plan_ws_bytes(B, Hq, Hkv, T, S, head_dim, true);
+    const int cus = device_cus();
+    const size_t a = plan_ws_bytes(cus, B, Hq, Hkv, T, S, head_dim, false);
+    const size_t b = plan_ws_bytes(cus, B, Hq, Hkv, T, S, head_dim, true);
     return a > b ? a : b;
 }
 
@@ -2911,6 +3252,26 @@ static void launch_decode128(bool lora, dim3 grid, dim3 block, hipStream_t s, co
         hipLaunchKernelGGL((attn_decode128_kernel<QJL, kDecPrefetch, SPB, true, PAGED>), grid, block, 0, s, a);
     else
         hipLaunchKernelGGL((attn_decode128_kernel<QJL, kDecPrefetch, SPB, false, PAGED>), grid, block, 0, s, a);
+}
+
+template <bool QJL, bool PAGED>
+static void launch_prefill128(const Plan &p, bool q32, dim3 grid, dim3 block, hipStream_t s, const AttnArgs &a) {
+    if (q32 && p.tws) hipLaunchKernelGGL((attn_prefill128_kernel<QJL, 1, 2, true, PAGED, true>), grid, block, 0, s, a);
+    else if (q32) hipLaunchKernelGGL((attn_prefill128_kernel<QJL, 1, 2, true, PAGED, false>), grid, block, 0, s, a);
+    else if (p.ncb == 1) hipLaunchKernelGGL((attn_prefill128_kernel<QJL, 1, 2, false, PAGED, true>), grid, block, 0, s, a);
+    else if (p.tws) hipLaunchKernelGGL((attn_prefill128_kernel<QJL, kPreNcb, 2, false, PAGED, true>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((attn_prefill128_kernel<QJL, kPreNcb, 2, false, PAGED, false>), grid, block, 0, s, a);
+}
+
+template <bool QJL>
+static void launch_prefill32(const Plan &p, bool q32, dim3 grid, dim3 block, hipStream_t s, const AttnArgs &a) {
+    if (p.ncb == 1 && q32) hipLaunchKernelGGL((attn_prefill32_kernel<QJL, 1, true, 16, true>), grid, block, 0, s, a);
+    else if (p.ncb == 1) hipLaunchKernelGGL((attn_prefill32_kernel<QJL, 1, false, 16, true>), grid, block, 0, s, a);
+    else if (q32 && p.tws) hipLaunchKernelGGL((attn_prefill32_kernel<QJL, 2, true, kP32Waves, true>), grid, block, 0, s, a);
+    else if (q32) hipLaunchKernelGGL((attn_prefill32_kernel<QJL, 2, true, kP32Waves, false>), grid, block, 0, s, a);
+    else if (p.ncb == 2) hipLaunchKernelGGL((attn_prefill32_kernel<QJL, 2, false, kP32Waves, true>), grid, block, 0, s, a);
+    else if (p.tws) hipLaunchKernelGGL((attn_prefill32_kernel<QJL, kP32Ncb, false, kP32Waves, true>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((attn_prefill32_kernel<QJL, kP32Ncb, false, kP32Waves, false>), grid, block, 0, s, a);
 }
 
 // Paged cache of omni_attn_paged.
@@ -2939,7 +3300,7 @@ static int attn_run(const void *q, int q_dtype, const uint8_t *k_nib, const uint
     OMNI_CHECK_ARG(S < (int64_t(1) << 25), "omni_attn: S must be < 2^25 tokens per sequence");
     OMNI_CHECK_ARG(T * (Hq / Hkv) < (int64_t(1) << 31), "omni_attn: T * (n_heads / n_kv_heads) must be < 2^31");
     OMNI_CHECK_ARG(seq_index == nullptr || n_seqs >= 1, "omni_attn: a cache index needs a pool of >= 1 sequences");
-    Plan p = make_plan(B, Hq, Hkv, T, S, head_dim, q_dtype == OMNI_F32, paged != nullptr, scale == 0.0f);
+    Plan p = make_plan(device_cus(), B, Hq, Hkv, T, S, head_dim, q_dtype == OMNI_F32, paged != nullptr, scale == 0.0f);
     OMNI_CHECK_ARG(paged == nullptr || head_dim == 128, "omni_attn_paged: needs head_dim 128");
     OMNI_CHECK_ARG(Hkv <= 65535 && ((B + p.spb - 1) / p.spb) * p.n_rchunks <= 65535 && p.splits <= 2147483647,
                    "omni_attn: grid too large (batch x row chunks must be <= 65535)");
@@ -2975,7 +3336,7 @@ static int attn_run(const void *q, int q_dtype, const uint8_t *k_nib, const uint
     a.ws = reinterpret_cast<float *>(workspace);
     a.T = T; a.S = S; a.split_len = p.split_len; a.causal_offset = causal_offset;
     a.q_dtype = q_dtype; a.per_head = per_head_codebook; a.Hq = Hq; a.Hkv = Hkv; a.G = Hq / Hkv;
-    a.n_rchunks = p.n_rchunks; a.splits = p.splits; a.ncopy = p.ncopy; a.rows = p.rows;
+    a.n_rchunks = p.n_rchunks; a.splits = p.splits; a.ncopy = p.ncopy; a.rows = p.rows; a.tw_shift = p.tws;
     a.with_qjl = with_qjl; a.rotate_q = rotate_q;
     a.g_magic = ((uint64_t)1 << 32) / (uint64_t)a.G + 1;
     a.rch_magic = ((uint64_t)1 << 32) / (uint64_t)p.n_rchunks + 1;
@@ -2995,54 +3356,34 @@ static int attn_run(const void *q, int q_dtype, const uint8_t *k_nib, const uint
     a.page_shift = paged ? paged->page_shift : 0;
     dim3 grid((unsigned)p.splits, (unsigned)Hkv, (unsigned)(((B + p.spb - 1) / p.spb) * p.n_rchunks));
     dim3 block(64 * p.nw);
+    hipStream_t st = as_stream(stream);
     if (p.prefill && paged) {
-        const bool qlo = q_dtype == OMNI_F32;
-        hipStream_t st = as_stream(stream);
-        if (with_qjl) {
-            if (qlo) hipLaunchKernelGGL((attn_prefill128_kernel<true, 1, 2, true, true>), grid, block, 0, st, a);
-            else hipLaunchKernelGGL((attn_prefill128_kernel<true, kPreNcb, 2, false, true>), grid, block, 0, st, a);
-        } else {
-            if (qlo) hipLaunchKernelGGL((attn_prefill128_kernel<false, 1, 2, true, true>), grid, block, 0, st, a);
-            else hipLaunchKernelGGL((attn_prefill128_kernel<false, kPreNcb, 2, false, true>), grid, block, 0, st, a);
-        }
+        if (with_qjl) launch_prefill128<true, true>(p, q_dtype == OMNI_F32, grid, block, st, a);
+        else launch_prefill128<false, true>(p, q_dtype == OMNI_F32, grid, block, st, a);
     } else if (p.prefill) {
-        const bool qlo = q_dtype == OMNI_F32;
-        hipStream_t st = as_stream(stream);
-        if (with_qjl) {
-            if (qlo) hipLaunchKernelGGL((attn_prefill128_kernel<true, 1, 2, true, false>), grid, block, 0, st, a);
-            else hipLaunchKernelGGL((attn_prefill128_kernel<true, kPreNcb, 2, false, false>), grid, block, 0, st, a);
-        } else {
-            if (qlo) hipLaunchKernelGGL((attn_prefill128_kernel<false, 1, 2, true, false>), grid, block, 0, st, a);
-            else hipLaunchKernelGGL((attn_prefill128_kernel<false, kPreNcb, 2, false, false>), grid, block, 0, st, a);
-        }
+        if (with_qjl) launch_prefill128<true, false>(p, q_dtype == OMNI_F32, grid, block, st, a);
+        else launch_prefill128<false, false>(p, q_dtype == OMNI_F32, grid, block, st, a);
     } else if (p.prefill32) {
-        const bool qlo = q_dtype == OMNI_F32;
-        hipStream_t st = as_stream(stream);
-        if (with_qjl) {
-            if (qlo) hipLaunchKernelGGL((attn_prefill32_kernel<true, 2, true>), grid, block, 0, st, a);
-            else hipLaunchKernelGGL((attn_prefill32_kernel<true, kP32Ncb, false>), grid, block, 0, st, a);
-        } else {
-            if (qlo) hipLaunchKernelGGL((attn_prefill32_kernel<false, 2, true>), grid, block, 0, st, a);
-            else hipLaunchKernelGGL((attn_prefill32_kernel<false, kP32Ncb, false>), grid, block, 0, st, a);
-        }
+        if (with_qjl) launch_prefill32<true>(p, q_dtype == OMNI_F32, grid, block, st, a);
+        else launch_prefill32<false>(p, q_dtype == OMNI_F32, grid, block, st, a);
     } else if (p.dec128 && paged) {
-        hipStream_t st = as_stream(stream);
         if (with_qjl && p.spb > 1) launch_decode128<true, 2, true>(lora_fused, grid, block, st, a);
         else if (with_qjl) launch_decode128<true, 1, true>(lora_fused, grid, block, st, a);
         else if (p.spb > 1) launch_decode128<false, 2, true>(lora_fused, grid, block, st, a);
         else launch_decode128<false, 1, true>(lora_fused, grid, block, st, a);
     } else if (p.dec128) {
-        hipStream_t st = as_stream(stream);
         if (with_qjl && p.spb > 1) launch_decode128<true, 2>(lora_fused, grid, block, st, a);
         else if (with_qjl) launch_decode128<true, 1>(lora_fused, grid, block, st, a);
         else if (p.spb > 1) launch_decode128<false, 2>(lora_fused, grid, block, st, a);
         else launch_decode128<false, 1>(lora_fused, grid, block, st, a);
     } else {
-        hipLaunchKernelGGL(attn_kernel<32>, grid, block, p.lds, as_stream(stream), a);
+        hipLaunchKernelGGL(attn_kernel<32>, grid, block, p.lds, st, a);
     }
     OMNI_CHECK_LAUNCH("omni_attn");
     if (p.splits > 1) {
-        dim3 g2(1, (unsigned)Hkv, (unsigned)(B * p.n_rchunks));
+        const int per = 256 / (head_dim / 2);
+        const int64_t rows = T * a.G < p.rows ? T * a.G : p.rows;
+        dim3 g2((unsigned)((rows + per - 1) / per), (unsigned)Hkv, (unsigned)(B * p.n_rchunks));
         if (head_dim == 128)
             hipLaunchKernelGGL(attn_combine_kernel<128>, g2, dim3(256), 0, as_stream(stream), a);
         else
@@ -3067,7 +3408,7 @@ extern "C" size_t omni_attn_lora_workspace_size(int64_t B, int Hq, int Hkv, int6
                                                 int q_dtype) {
     if (B <= 0 || Hq <= 0 || Hkv <= 0 || T <= 0 || S <= 0 || Hq % Hkv || !head_dim_ok(head_dim) || !dtype_ok(q_dtype))
         return 0;
-    const size_t ws = plan_ws_bytes(B, Hq, Hkv, T, S, head_dim, q_dtype == OMNI_F32);
+    const size_t ws = plan_ws_bytes(device_cus(), B, Hq, Hkv, T, S, head_dim, q_dtype == OMNI_F32);
     // room for the gather-apply fallback's q_eff: the adapter's rank and
     // hidden size, which decide between it and the fused path, are not
     // arguments here
@@ -3125,8 +3466,8 @@ extern "C" int omni_attn_serve(const void *q, int q_dtype, const int64_t *cache_
 // pages: nibbles (n_pages, Hkv, page_size, 64), signs (.., 8), norms
 // (n_pages, Hkv, page_size), V (.., 64).  Sequence b holds seq_lens[b] tokens
 // in pages page_table[b * max_pages + j], j < ceil(len / page_size); entries
-// past that are never read for keys.  D = 128; up to 32 query rows per kv
-// head (T * Hq / Hkv) run the decode kernel, more the chunked-prefill kernel.
+// past that are never read for keys.  D = 128; the kernel by the query
+// rows per kv head (T * Hq / Hkv) as for a contiguous cache (make_plan).
 // causal != 0 aligns query token t with key len - T + t.
 
 static bool paged_args_ok(int64_t B, int Hkv, int64_t n_pages, int page_size, int64_t max_pages, int &shift) {
@@ -3159,8 +3500,8 @@ extern "C" size_t omni_attn_paged_workspace_size(int64_t B, int Hq, int Hkv, int
     // either plan (a zero score scale runs another kernel), plus room for
     // the gather-apply LoRA fallback's q_eff
     const int64_t S = max_pages * (int64_t)page_size;
-    const size_t a = make_plan(B, Hq, Hkv, T, S, 128, q_dtype == OMNI_F32, true).ws_bytes;
-    const size_t z = make_plan(B, Hq, Hkv, T, S, 128, q_dtype == OMNI_F32, true, true).ws_bytes;
+    const size_t a = make_plan(device_cus(), B, Hq, Hkv, T, S, 128, q_dtype == OMNI_F32, true).ws_bytes;
+    const size_t z = make_plan(device_cus(), B, Hq, Hkv, T, S, 128, q_dtype == OMNI_F32, true, true).ws_bytes;
     return align256(a > z ? a : z) + (size_t)B * Hq * T * 128 * (q_dtype == OMNI_F32 ? 4 : 2);
 }
 
@@ -3208,7 +3549,6 @@ extern "C" int omni_attn_paged(const void *q, int q_dtype, const uint8_t *k_nib,
 // (each launch writes every partial it reads back).
 namespace omni {
 
-constexpr size_t kScratchBytes = size_t(16) << 20;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
 constexpr int kScratchMaxDevices = 64;

@@ -111,32 +111,6 @@ __global__ __launch_bounds__(256) void code_table_kernel(const float *codebooks,
     table[(int64_t)h * kEncTab + u] = (uint8_t)(code | (code << 4));
 }
 
-// (a, b) <- butterfly with the partner lane across bit 4 (row parity) or 5
-// (half): lanes with the bit clear hold the lower element of each pair.
-// Two swaps and one add/sub pair cover two elements.
-template <int HALF>
-__device__ __forceinline__ void xlane_pair_butterfly(float &a, float &b) {
-    uint32_t t0, t1, u0, u1;
-    if constexpr (HALF == 16) {
-        const auto t = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-        t0 = t[0]; t1 = t[1];
-    } else {
-        const auto t = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-        t0 = t[0]; t1 = t[1];
-    }
-    const float lo = __uint_as_float(t0), hi = __uint_as_float(t1);
-    const float s = lo + hi, d = lo - hi;
-    if constexpr (HALF == 16) {
-        const auto u = __builtin_amdgcn_permlane16_swap(__float_as_uint(s), __float_as_uint(d), false, false);
-        u0 = u[0]; u1 = u[1];
-    } else {
-        const auto u = __builtin_amdgcn_permlane32_swap(__float_as_uint(s), __float_as_uint(d), false, false);
-        u0 = u[0]; u1 = u[1];
-    }
-    a = __uint_as_float(u0);
-    b = __uint_as_float(u1);
-}
-
 // ── omni_wht_rotate ─────────────────────────────────────────────────────
 //
 // Normalized WHT in the reference's butterfly order h = 1, 2, ..., D/2

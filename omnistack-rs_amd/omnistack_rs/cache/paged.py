@@ -14,8 +14,8 @@ the reference's packed layout with the batch axis as pages:
 A sequence is a list of pages (one row of an int32 page table) and a length;
 token s of sequence b sits in page ``page_table[b, s // page_size]`` at slot
 ``s % page_size``.  ``paged_attention`` is one call into libomnistack_amd.so
-(``omni_attn_paged``): the decode kernel (up to 32 query rows per kv head)
-or the chunked-prefill kernel (more rows) reads each 16-token half-tile from
+(``omni_attn_paged``): the decode kernel (few query rows per kv head) or
+the chunked-prefill kernel (many) reads each 16-token half-tile from
 its page in place, with the same arithmetic as the contiguous ``omni_attn``
 (so a sequence gives the same result whichever pages hold it).
 """
@@ -213,9 +213,9 @@ def paged_attention(q: torch.Tensor, cache: PagedKVCache, page_table: torch.Tens
                     validate: bool = True) -> torch.Tensor:
     """``omni_attn`` over a paged cache: query batch entry b attends the
     first ``seq_lens[b]`` tokens of the sequence in row b of ``page_table``.
-    q (B, n_heads, T, 128); up to 32 query rows per kv head
-    (T * n_heads / n_kv_heads) run the decode kernel, more the chunked-prefill
-    kernel.  ``causal`` aligns query token t with key ``seq_lens[b] - T + t``
+    q (B, n_heads, T, 128); up to 8 query rows per kv head
+    (T * n_heads / n_kv_heads) run the decode kernel, more than 32 the
+    chunked-prefill kernel, those between the faster of the two.  ``causal`` aligns query token t with key ``seq_lens[b] - T + t``
     (a row with no visible key is NaN, as in the reference).  Returns float32
     (B, n_heads, T, 128).  With ``validate``, page ids outside the pool and
     lengths beyond the table raise on the host (one device-to-host copy);

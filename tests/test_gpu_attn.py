@@ -614,3 +614,70 @@ def test_prefill_large_and_tiny_query_rows(device):
         want = restate.fused_attn_python(q.float(), kn, kq, kr, vn, cb, uid, scale, True)
         assert torch.isfinite(got).all()
         _assert_close(got, want, f"prefill extreme rows scale {scale:.3g}")
+
+
+def _random_packed(B, Hkv, S, D, seed):
+    """Packed cache of random bytes and a spread, asymmetric codebook per kv head."""
+    g = _data.gen(seed)
+    kn, vn = (torch.randint(0, 256, (B, Hkv, S, D // 2), generator=g, dtype=torch.uint8) for _ in range(2))
+    kq = torch.randint(0, 256, (B, Hkv, S, D // 16), generator=g, dtype=torch.uint8)
+    kr = torch.rand((B, Hkv, S), generator=g)
+    cb = torch.sort(torch.randn(Hkv, 16, generator=g), dim=1).values
+    return kn, kq, kr, vn, cb
+
+
+def _row_calls():
+    for D in (128, 32):
+        for rows in (1, 8, 9, 16, 17, 32, 33, 64, 65, 128, 129, 256, 257):
+            yield D, rows, 77, torch.bfloat16 if rows % 2 else torch.float16
+            yield D, rows, 1000, torch.float32
+        yield D, 24, 20011, torch.bfloat16       # more than eight splits through the combine kernel
+        yield D, 40, 9001, torch.float32
+        yield D, 3, 1, torch.float32             # one key: all waves of a group but one without a tile
+
+
+@pytest.mark.parametrize("D,rows,S,dtype", list(_row_calls()))
+def test_attn_row_counts(device, D, rows, S, dtype):
+    """Row counts at the edges of the kernels and of a wave's rows (waves
+    that share one group of rows take its key tiles in turn), with the causal
+    window that the rows leave, in-kernel rotation, and q one element past an
+    aligned address."""
+    B, Hkv, G, uid = 2, 2, (1 if rows % 3 else 3), 5
+    T, Hq = rows // G, Hkv * G
+    print(f"[rows] D={D} rows={rows} S={S} {dtype}", flush=True)
+    kn, kq, kr, vn, cb = _random_packed(B, Hkv, S, D, seed=700 + rows + S)
+    q = torch.randn(B, Hq, T, D, generator=_data.gen(701 + rows)).to(dtype)
+    sign = _data.sign_flip()[:D].contiguous()
+    off = max(S - T, 0)
+    room = torch.empty(q.numel() + 1, dtype=dtype, device=device)
+    q1 = room[1:].view(q.shape).copy_(q)
+    kw = dict(causal_offset=off, rotate_q=True, sign_flip=sign.to(device))
+    got = _run(device, q, kn, kq, kr, vn, cb, uid, **kw)
+    got1 = _run(device, q1, kn, kq, kr, vn, cb, uid, **kw)
+    if D == 32 or rows > 32:             # (the decode kernel's waves claim tiles as they get to them)
+        same = torch.equal(got, got1)
+        assert same, f"q past an aligned address: {(got - got1).abs().max().item():.3e} off"
+    k = restate.dequantize_heads(kn, kq, kr, cb, user_id=uid)
+    v = restate.dequantize_heads(vn, kq, kr, cb, user_id=uid, with_qjl=False)
+    want = exact.attention(restate.rotate(q, sign).float(), k, v, 1 / math.sqrt(D), mask=_causal_mask(T, S, off))
+    assert torch.isfinite(got).all()
+    _assert_close(got, want, f"rows D{D} {rows} S{S} {dtype}")
+    _assert_close(got1, want, f"rows D{D} {rows} S{S} {dtype}, q past an aligned address")
+
+
+@pytest.mark.parametrize("B,T,S", [(2, 12, 100), (40, 12, 2100), (40, 32, 2100)])
+def test_attn_decode_or_prefill_rows(device, B, T, S):
+    """9 to 32 rows at head_dim 128: a few short sequences (decode blocks of
+    eight rows) and many long ones (prefill blocks), contiguous and paged."""
+    from omnistack_rs.cache import PagedKVCache, paged_attention
+    Hkv, Hq, uid = 8, 8, 6
+    kn, kq, kr, vn, cb = _random_packed(B, Hkv, S, 128, seed=710)
+    q = torch.randn(B, Hq, T, 128, generator=_data.gen(711)).bfloat16()
+    got = _run(device, q, kn, kq, kr, vn, cb, uid)
+    cache, pt, lens = PagedKVCache.from_contiguous(*(t.to(device) for t in (kn, kq, kr, vn)), page_size=16)
+    paged = paged_attention(q.to(device), cache, pt, lens, cb.to(device), user_id=uid)
+    for b in (0, B - 1):
+        sl = slice(b, b + 1)
+        want = restate.fused_attn_python(q[sl].float(), kn[sl], kq[sl], kr[sl], vn[sl], cb, uid, 1 / math.sqrt(128), True)
+        _assert_close(got[sl], want, f"B{B} T{T} S{S} b{b}")
+        _assert_close(paged[sl], want, f"paged B{B} T{T} S{S} b{b}")
