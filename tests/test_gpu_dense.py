@@ -101,3 +101,49 @@ def test_unfused_python_path_matches_oracle(device):
     assert got.dtype == q.dtype
     # both round an fp32 result to q's dtype: at most one ulp apart
     assert bool(((got.cpu().float() - want.float()).abs() <= 2 ** -7 * want.float().abs() + 1e-6).all())
+
+
+@pytest.mark.parametrize("D", [32, 64, 128, 256])
+@pytest.mark.parametrize("T,S", [(4, 1), (5, 31), (17, 32), (16, 33), (300, 65), (1300, 40)])
+def test_dense_attn_row_and_key_edges(device, D, T, S):
+    """Rows and keys at the edges of 16-row waves and 32-key tiles, on both
+    sides of the rule between the launches that split rows and keys (1300
+    queries x 8 kv heads: rows), with a causal mask and its column-major copy
+    (same values: same bits)."""
+    from omnistack_rs.attention import reference_attn
+    B, Hq, Hkv = 1, 16, 8
+    g = _data.gen(540 + T + S)
+    q = torch.randn(B, Hq, T, D, generator=g)
+    k, v = torch.randn(B, Hkv, S, D, generator=g), torch.randn(B, Hkv, S, D, generator=g)
+    mask = torch.full((T, S), float("-inf")).triu(1) if T >= S else torch.zeros(T, S)
+    mask[:, S // 2:] += 0.25
+    dev = [t.to(device) for t in (q, k, v)]
+    want = restate.reference_attn(q, k, v, mask=mask)
+    got = reference_attn(*dev, mask=mask.to(device))
+    _close(got, want, f"T{T} S{S} D{D} mask")
+    same = torch.equal(got, reference_attn(*dev, mask=mask.t().contiguous().to(device).t()))
+    assert same, "column-major mask"
+    _close(reference_attn(*dev), restate.reference_attn(q, k, v), f"T{T} S{S} D{D}")
+
+
+@pytest.mark.parametrize("where,value", [("k", float("nan")), ("k", float("inf")), ("v", float("nan")), ("v", float("-inf")),
+                                         ("k", 3e38), ("q", 3e38), ("v", 3e38)])
+def test_dense_attn_hidden_tiles(device, where, value):
+    """Whole tiles of hidden keys are skipped only where they change nothing:
+    a NaN or infinite key or value there, or scores that overflow, give the
+    reference's NaN (0 x inf, inf - inf)."""
+    from omnistack_rs.attention import reference_attn
+    B, Hq, Hkv, T, S, D = 1, 16, 8, 1100, 160, 32
+    g = _data.gen(560)
+    t = dict(q=torch.randn(B, Hq, T, D, generator=g), k=torch.randn(B, Hkv, S, D, generator=g),
+             v=torch.randn(B, Hkv, S, D, generator=g))
+    mask = torch.zeros(T, S)
+    mask[:, 64:] = float("-inf")               # keys 64 .. 159 hidden from every query
+    if where == "q":
+        t["q"][0, 3, 5, 7] = value
+        t["k"][0, 1, 100:] *= 1e3
+    else:
+        t[where][0, 1, 100, 3] = value
+    want = restate.reference_attn(t["q"], t["k"], t["v"], mask=mask)
+    got = reference_attn(*(x.to(device) for x in (t["q"], t["k"], t["v"])), mask=mask.to(device))
+    _close(got, want, f"hidden {where} {value}")
