@@ -78,6 +78,7 @@ struct AttnArgs {
     const int32_t *seq_lens;
     int64_t max_pages, n_pages;
     int page_size, page_shift;  // page_size = 2^page_shift >= 16
+    int by_len;                // two sequences per block: pair the longest with the shortest
     float qscale;              // scale * log2(e)
     float alpha_c;             // fp32 sqrt(2/pi)/D (the row scale multiplies the whole score)
     float wht_scale;
@@ -570,6 +571,8 @@ __device__ __forceinline__ int dec_chunk(int row, int c) { return c ^ (2 * (row 
 constexpr int kDecCntOff = kDecCscOff + kDecRows * 4;                // next unclaimed tile of the block
 constexpr int kDecLrOff = kDecCntOff + 16;                           // fused LoRA: x A^T of two row groups
 constexpr int kDecLdsBytes = kDecLrOff + 2 * 16 * 4;
+constexpr int kByLenMax = 128;               // sequences that a block ranks by length (AttnArgs::by_len)
+constexpr int kDecTileTokensMax = (1 << 25) - 1;   // tokens of a sequence (host check)
 // Paged cache: the pool row of each 16-token half of the split (half h at
 // kDecPtOff + 4 h, the row of token s_begin + 16 h), staged in the prologue
 // when the split has at most kDecPtMax halves (the paged plan keeps every
@@ -1031,11 +1034,82 @@ __global__ __launch_bounds__(64 * kDecWaves) void attn_decode128_kernel(AttnArgs
     const int bz = blockIdx.z;
     const int bzq = div_small(bz, a.rch_magic);
     const int rc = bz - bzq * a.n_rchunks;
-    const int b32 = bzq * SPB;
+    const int n = lane & 15, g = lane >> 4;
+    // ── prologue loads that need no sequence ──────────────────────────
+    const bool use_flip = a.rotate_q && a.sign_flip;
+    const __amdgpu_buffer_rsrc_t SF = __builtin_amdgcn_make_buffer_rsrc(
+        (void *)(use_flip ? (const void *)a.sign_flip : (const void *)a.codebooks), (short)0, use_flip ? D : 0, kBufWord3);
+    const uint32_t sf_lo = __builtin_amdgcn_raw_buffer_load_b8(SF, (uint32_t)lane, 0, 0);
+    const uint32_t sf_hi = __builtin_amdgcn_raw_buffer_load_b8(SF, (uint32_t)(64 + lane), 0, 0);
+    // codebook entry lane % 16 (threads 0-15 publish it as fp16 hi / remainder)
+    const __amdgpu_buffer_rsrc_t CB = __builtin_amdgcn_make_buffer_rsrc(
+        (void *)(a.codebooks + (a.per_head ? hk * 16 : 0)), (short)0, 16 * 4, kBufWord3);
+    const float cb_mine = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(CB, 4u * (lane & 15), 0, 0));
+    // G rows 16 * wave + n (waves 0-3 compute that 16-column block of G q)
+    const __amdgpu_buffer_rsrc_t GB = __builtin_amdgcn_make_buffer_rsrc(
+        (void *)(a.g_bits + (QJL ? (int64_t)hk * QD * 4 : 0)), (short)0, (QJL && wave < QD / 16) ? QD * 16 : 0, kBufWord3);
+    const u32x4_t gw = __builtin_amdgcn_raw_buffer_load_b128(GB, (uint32_t)(16 * wave + n) * 16u, 0, 0);
+
+    int b32 = bzq * SPB, b32b = b32 + 1;      // the block's sequence; its second one (SPB > 1)
+    int nseq = (SPB > 1 && b32 + 1 < a.B) ? 2 : 1;
+    int32_t L0 = 0, L1 = 0;                   // paged: their lengths
+    if constexpr (PAGED) {
+        if (SPB > 1 && a.by_len) {
+            // The bz-th longest sequence and the bz-th shortest (ties by
+            // index; a length outside [0, capacity] counts as 0): a thread
+            // per sequence counts the greater (length, index) keys.
+            static_assert(kByLenMax == 128 && kDecTileTokensMax < (1 << 25), "two keys per lane, length * 128 + index in 32 bits");
+            // (the sign table while the lengths are on their way)
+            const __amdgpu_buffer_rsrc_t LB = __builtin_amdgcn_make_buffer_rsrc((void *)a.seq_lens, (short)0, (int)a.B * 4, kBufWord3);
+            uint32_t u[2], raw[2];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int i = 64 * h + lane;
+                const uint32_t L = raw[h] = __builtin_amdgcn_raw_buffer_load_b32(LB, 4u * (uint32_t)i, 0, 0);
+                u[h] = i < a.B ? ((int64_t)L > a.S ? 0u : L) * 128u + (uint32_t)(127 - i) : 0u;
+            }
+            if (tid < 512) sign_table_store(smem, tid);
+            // wave w counts over the sequences w, w + 12, ...; the partial
+            // counts meet as bytes in the area of G q (not written before
+            // the next barrier)
+            unsigned char *part = smem + kDecQsOff + kDecRows * D * 4;
+            static_assert(kByLenMax * kDecWaves <= kDecRows * kDecGqStride * 4 && kDecWaves == 12, "three dwords of counts per sequence");
+            uint32_t r0 = 0, r1 = 0;
+#pragma unroll
+            for (int k = 0; k < (kByLenMax + kDecWaves - 1) / kDecWaves; ++k) {
+                const int q = wave + kDecWaves * k;
+                if (q < a.B) {                               // (wave-uniform)
+                    const uint32_t other = (uint32_t)__builtin_amdgcn_readlane(q < 64 ? u[0] : u[1], q & 63);
+                    r0 += other > u[0] ? 1u : 0u;
+                    r1 += other > u[1] ? 1u : 0u;
+                }
+            }
+            part[lane * kDecWaves + wave] = (unsigned char)r0;
+            part[(64 + lane) * kDecWaves + wave] = (unsigned char)r1;
+            __syncthreads();
+            int rank[2];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const uint32_t *c = reinterpret_cast<const uint32_t *>(part + (64 * h + lane) * kDecWaves);
+                const int v = (int)__builtin_amdgcn_sad_u8(c[0], 0u, __builtin_amdgcn_sad_u8(c[1], 0u, __builtin_amdgcn_sad_u8(c[2], 0u, 0u)));
+                rank[h] = 64 * h + lane < a.B ? v : -1;
+            }
+            auto at = [&](int r) {
+                const uint64_t lo = __builtin_amdgcn_ballot_w64(rank[0] == r);
+                return lo ? (int)__builtin_ctzll(lo) : 64 + (int)__builtin_ctzll(__builtin_amdgcn_ballot_w64(rank[1] == r));
+            };
+            b32 = at(bz);
+            b32b = at((int)a.B - 1 - bz);
+            nseq = b32 != b32b ? 2 : 1;
+            L0 = __builtin_amdgcn_readlane(b32 < 64 ? raw[0] : raw[1], b32 & 63);
+            L1 = __builtin_amdgcn_readlane(b32b < 64 ? raw[0] : raw[1], b32b & 63);
+        } else {
+            L0 = a.seq_lens[b32];
+            if (SPB > 1 && nseq > 1) L1 = a.seq_lens[b32b];
+        }
+    }
     const int64_t b = b32;
     const int nrows_total = (int)(a.T * a.G);
-    const int nseq = (SPB > 1 && b32 + 1 < a.B) ? 2 : 1;
-    const int n = lane & 15, g = lane >> 4;
     // row slot r -> (sequence index, flat (t, head) row of that sequence, valid)
     auto row_seq = [&](int r) { return (SPB > 1 && r >= nrows_total) ? 1 : 0; };
     auto row_rho = [&](int r) { return SPB > 1 ? r - row_seq(r) * nrows_total : rc * kDecRows + r; };
@@ -1051,12 +1125,10 @@ __global__ __launch_bounds__(64 * kDecWaves) void attn_decode128_kernel(AttnArgs
     int seq_len = (int)a.S, seq_len1 = (int)a.S;
     bool len_bad = false, len_bad1 = false;
     if constexpr (PAGED) {
-        const int32_t L = a.seq_lens[b32];
-        len_bad = L < 0 || (int64_t)L > a.S;
-        seq_len = len_bad ? 0 : L;
+        len_bad = L0 < 0 || (int64_t)L0 > a.S;
+        seq_len = len_bad ? 0 : L0;
         seq_len1 = seq_len;
         if (SPB > 1 && nseq > 1) {
-            const int32_t L1 = a.seq_lens[b32 + 1];
             len_bad1 = L1 < 0 || (int64_t)L1 > a.S;
             seq_len1 = len_bad1 ? 0 : L1;
         }
@@ -1135,7 +1207,7 @@ __global__ __launch_bounds__(64 * kDecWaves) void attn_decode128_kernel(AttnArgs
     // pool marks this wave's state bad (the sequence's rows come out NaN)
     bool page_bad = false, page_bad1 = false;
     const int32_t *pt_row = PAGED ? a.page_table + b * a.max_pages : nullptr;
-    const int32_t *pt_row1 = PAGED && SPB > 1 && nseq > 1 ? pt_row + a.max_pages : pt_row;
+    const int32_t *pt_row1 = PAGED && SPB > 1 && nseq > 1 ? a.page_table + b32b * a.max_pages : pt_row;
     auto half_rows = [&](int t, int sq, uint32_t (&rb)[2]) {
         if (SPB > 1 && sq) paged_half_rows(a, pt_row1, hk, t, s_end1, page_bad1, rb);
         else paged_half_rows(a, pt_row, hk, t, s_end, page_bad, rb);
@@ -1197,7 +1269,7 @@ __global__ __launch_bounds__(64 * kDecWaves) void attn_decode128_kernel(AttnArgs
     // this wave's query row
     const bool row_ok = row_valid(wave);
     const int rho_c = row_ok ? row_rho(wave) : 0;
-    const int64_t b_q = row_ok ? b + row_seq(wave) : b;
+    const int64_t b_q = row_ok && row_seq(wave) ? b32b : b32;
     const int t_q = div_small(rho_c, a.g_magic);
     const int hq_q = hk * a.G + (rho_c - t_q * a.G);
     const bool q32 = a.q_dtype == OMNI_F32;
@@ -1217,20 +1289,6 @@ __global__ __launch_bounds__(64 * kDecWaves) void attn_decode128_kernel(AttnArgs
             lora_x_load(lora_xw, a, b_q, t_q, lane);
         }
     }
-    const bool use_flip = a.rotate_q && a.sign_flip;
-    const __amdgpu_buffer_rsrc_t SF = __builtin_amdgcn_make_buffer_rsrc(
-        (void *)(use_flip ? (const void *)a.sign_flip : (const void *)a.codebooks), (short)0, use_flip ? D : 0, kBufWord3);
-    const uint32_t sf_lo = __builtin_amdgcn_raw_buffer_load_b8(SF, (uint32_t)lane, 0, 0);
-    const uint32_t sf_hi = __builtin_amdgcn_raw_buffer_load_b8(SF, (uint32_t)(64 + lane), 0, 0);
-    // codebook entry lane % 16 (threads 0-15 publish it as fp16 hi / remainder)
-    const __amdgpu_buffer_rsrc_t CB = __builtin_amdgcn_make_buffer_rsrc(
-        (void *)(a.codebooks + (a.per_head ? hk * 16 : 0)), (short)0, 16 * 4, kBufWord3);
-    const float cb_mine = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(CB, 4u * (lane & 15), 0, 0));
-    // G rows 16 * wave + n (waves 0-3 compute that 16-column block of G q)
-    const __amdgpu_buffer_rsrc_t GB = __builtin_amdgcn_make_buffer_rsrc(
-        (void *)(a.g_bits + (QJL ? (int64_t)hk * QD * 4 : 0)), (short)0, (QJL && wave < QD / 16) ? QD * 16 : 0, kBufWord3);
-    const u32x4_t gw = __builtin_amdgcn_raw_buffer_load_b128(GB, (uint32_t)(16 * wave + n) * 16u, 0, 0);
-
     // ── both ring slots in flight (tiles `wave` and `wave + nw` of the
     //    split) before the prologue's work, so the cache streams while the
     //    prologue runs.  Loads are unconditional (past the split end they
@@ -1257,7 +1315,7 @@ __global__ __launch_bounds__(64 * kDecWaves) void attn_decode128_kernel(AttnArgs
     // tiles 0 .. 2 nw - 1 are taken statically (two per wave, already in flight)
     if (tid == 0) *reinterpret_cast<int *>(smem + kDecCntOff) = 2 * nw;
     // ── sign table (threads 0..511) ───────────────────────────────────
-    if (tid < 512) sign_table_store(smem, tid);
+    if (tid < 512 && !(PAGED && SPB > 1 && a.by_len)) sign_table_store(smem, tid);
     // fused LoRA with G % 4 == 0: row slots 4 k .. 4 k + 3 hold one
     // (sequence, token), so x A^T is shared: each of the four waves sums a
     // quarter of its rank components, the others read them after a barrier
@@ -1469,10 +1527,17 @@ __global__ __launch_bounds__(64 * kDecWaves) void attn_decode128_kernel(AttnArgs
 
     // ── main loop ─────────────────────────────────────────────────────
     const int key_limit = (int)imax64(imin64(key_limit64, (int64_t)0x7fffffff), -1);
-    // tiles ending at or below min(s_end, first masked key of any row) need no masks
-    const int64_t min_limit64 = causal ? coff + div_small(rc * kDecRows, a.g_magic) : INT64_MAX;
-    // two sequences per block: every tile masks the other sequence's columns
-    const int full_end = nseq > 1 ? s_begin : (int)imin64((int64_t)s_end, min_limit64 + 1);
+    // tiles ending at or below min(end, first masked key of any row) of their
+    // sequence need no masks but, with two sequences per block, the other
+    // one's columns (contiguous caches take the masked path for every tile of
+    // two sequences: the second path's registers would spill there)
+    constexpr bool kLight = PAGED && SPB > 1;
+    auto full_of = [&](int end, int len) {
+        const int64_t c = PAGED ? (int64_t)len - a.T : a.causal_offset;
+        return causal ? (int)imin64((int64_t)end, c + div_small(rc * kDecRows, a.g_magic) + 1) : end;
+    };
+    const int full_end = nseq > 1 && !kLight ? s_begin : full_of(s_end, seq_len);
+    const int full_end1 = kLight ? full_of(s_end1, seq_len1) : full_end;
     const uint32_t laneoff = (uint32_t)(lane & 31) * 8u;
     const uint32_t slane = (uint32_t)kSlutOff | laneoff;
     // ones in every slot of A row 0: one MFMA sums the P of all 32 tokens of
@@ -1506,7 +1571,7 @@ __global__ __launch_bounds__(64 * kDecWaves) void attn_decode128_kernel(AttnArgs
 
     // One 32-token tile: scores, online softmax, PV.
     auto tile_step = [&](TileRaw &R, const int tt, const int tseq, auto &&after_k) {
-        const bool full = tt + kDecTile <= full_end;
+        const bool full = tt + kDecTile <= (kLight && tseq ? full_end1 : full_end);
         // wave priority by phase: the K pass 2, masks and maxima 1, the
         // softmax and PV 0 (issue order only: results do not depend on it)
         __builtin_amdgcn_s_setprio(2);
@@ -1552,6 +1617,10 @@ __global__ __launch_bounds__(64 * kDecWaves) void attn_decode128_kernel(AttnArgs
                     const int tn = tt + 16 * u + 4 * g + i;
                     if (tn >= (tseq ? s_end1 : s_end) || tn > key_limit || seq_n != tseq) sc[4 * u + i] = -INFINITY;
                 }
+        } else if (kLight && nseq > 1) {
+            const bool other = seq_n != tseq;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) sc[k] = other ? -INFINITY : sc[k];
         }
 
         // online softmax (exp2 domain), lazy rescale.  The scaled maximum of
@@ -1766,7 +1835,7 @@ __global__ __launch_bounds__(64 * kDecWaves) void attn_decode128_kernel(AttnArgs
         const int rr = s / D, d = s % D;
         if (!row_valid(rr)) continue;
         const int rr_rho = row_rho(rr);
-        const int64_t rr_b = b + row_seq(rr);
+        const int64_t rr_b = row_seq(rr) ? b32b : b32;
         float rmx, lsum, osum;
         if (nw_act == nw) merge(std::integral_constant<int, nw>{}, rr, d, rmx, lsum, osum);
         else merge(nw_act, rr, d, rmx, lsum, osum);
@@ -3348,6 +3417,14 @@ static int attn_run(const void *q, int q_dtype, const uint8_t *k_nib, const uint
     a.seq_index = seq_index;
     a.n_seqs = seq_index ? n_seqs : B;
     a.spb = p.spb;
+    // Paged, two sequences per block: the longest with the shortest, longest
+    // pairs first, where a block's time is its longest pair's: 48 sequences
+    // of 200 to 3000 tokens, 8 kv heads, 40.5 us with neighbours, 31.5 by
+    // length.  Knowing the lengths before anything else costs 0.7 us a block
+    // (equal lengths of 600 tokens 28.8 -> 29.5 us, of 2050 44.0 -> 43.6 with
+    // the masks that the second sequence no longer takes), so capacities
+    // below 1536 tokens and more than 128 sequences pair neighbours.
+    a.by_len = paged != nullptr && p.spb > 1 && S >= 4 * (int64_t)kDecWaves * kDecTile && B <= kByLenMax;
     a.page_table = paged ? paged->page_table : nullptr;
     a.seq_lens = paged ? paged->seq_lens : nullptr;
     a.max_pages = paged ? paged->max_pages : 0;

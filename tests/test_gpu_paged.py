@@ -610,3 +610,43 @@ def test_prepared_paged_attention_refuses_bad_lora_bank(device):
     att = PagedKVAttention(pool, cb, n_heads=8, batch=2, max_pages=4, lora_a=la,
                            lora_b=torch.zeros(4, 8 * 128, 8, dtype=torch.bfloat16, device=device))
     assert att.lora is not None
+
+
+@pytest.mark.parametrize("B", [33, 64, 65, 127, 128, 129])
+def test_paged_pairs_by_length(device, B):
+    """Two sequences per block, paired longest with shortest from a capacity
+    of 1536 tokens and up to 128 sequences: equal, ragged and out-of-range
+    lengths (NaN for that sequence only), the middle one of an odd batch
+    alone, a bad page of one sequence, and a causal query."""
+    from omnistack_rs.cache import PagedKVCache, paged_attention
+    Hq, Hkv, S, uid, ps = 16, 8, 1600, 3, 32
+    g = torch.Generator().manual_seed(B)
+    kn, kq, kr, vn = (t.cpu() for t in _random_cache("cpu", 8, Hkv, S, 600 + B))
+    cb = torch.sort(torch.randn(Hkv, 16, generator=g), dim=1).values
+    q = _data.query((B, Hq, 1, 128), seed=601 + B)
+    # a pool of eight sequences' pages, shared by the batch
+    cache, pt8, _ = PagedKVCache.from_contiguous(*(t.to(device) for t in (kn, kq, kr, vn)), page_size=ps, spare_pages=1)
+    src = torch.arange(B) % 8
+    pt = pt8[src.to(device)].contiguous()
+    for kind in ("ragged", "equal"):
+        lens = torch.randint(1, S + 1, (B,), generator=g) if kind == "ragged" else torch.full((B,), 900)
+        lens[min(B - 1, 5)] = S
+        bad = {}
+        if kind == "ragged":
+            lens[7], lens[B - 2], lens[11] = -3, S + 1, 0
+            bad = {7, B - 2, 11, 20}
+            pt[20, 0] = cache.n_pages
+            lens[20] = 700
+        got = paged_attention(q.to(device), cache, pt, lens.to(torch.int32).to(device), cb.to(device), user_id=uid,
+                              causal=kind == "equal", validate=False).cpu()
+        pt[20] = pt8[4]
+        for b in range(B):
+            if b in bad:
+                assert torch.isnan(got[b]).all(), f"{kind} b{b} should be NaN"
+            else:
+                assert torch.isfinite(got[b]).all(), f"{kind} b{b}"
+        for b in sorted({0, 5, B // 2, B - 1, int(lens.clamp(0, S).argmin())} - set(bad)):
+            L, c = int(lens[b]), int(src[b])
+            want = restate.fused_attn_python(q[b:b + 1].float(), kn[c:c + 1, :, :L], kq[c:c + 1, :, :L], kr[c:c + 1, :, :L],
+                                             vn[c:c + 1, :, :L], cb, uid, 1 / math.sqrt(128), True)
+            _assert_close(got[b:b + 1], want, f"by length {kind} B{B} b{b} len{L}")
