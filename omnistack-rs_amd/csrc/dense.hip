@@ -242,14 +242,15 @@ __global__ __launch_bounds__(64 * kDnWaves, D == 256 ? 1 : (D == 128 ? 3 : 4)) v
     float4 nk[kPer], nv[kPer];
     float mk[2][4] = {};
     auto fetch = [&](int64_t s0) {
-        // the tile's keys below S as buffers: lanes past them read 0
+        // the tile's keys below S as buffers: lanes past them read 0 (the
+        // whole offset is the lane's: the scalar one is not range-checked)
         const int bytes = (int)(s0 + kDnKeys <= a.S ? kDnKeys : a.S - s0) * D * 4;
         const __amdgpu_buffer_rsrc_t K = __builtin_amdgcn_make_buffer_rsrc((void *)(kb0 + s0 * D), (short)0, bytes, kDnBufWord3);
         const __amdgpu_buffer_rsrc_t V = __builtin_amdgcn_make_buffer_rsrc((void *)(vb0 + s0 * D), (short)0, bytes, kDnBufWord3);
 #pragma unroll
         for (int c = 0; c < kPer; ++c) {
-            nk[c] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(K, 16 * tid, c * 1024 * kDnWaves, 0));
-            nv[c] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(V, 16 * tid, c * 1024 * kDnWaves, 0));
+            nk[c] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(K, 16 * tid + c * 1024 * kDnWaves, 0, 0));
+            nv[c] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(V, 16 * tid + c * 1024 * kDnWaves, 0, 0));
         }
     };
     if (a.S > 0) fetch(0);

@@ -147,3 +147,28 @@ def test_dense_attn_hidden_tiles(device, where, value):
     want = restate.reference_attn(t["q"], t["k"], t["v"], mask=mask)
     got = reference_attn(*(x.to(device) for x in (t["q"], t["k"], t["v"])), mask=mask.to(device))
     _close(got, want, f"hidden {where} {value}")
+
+
+@pytest.mark.parametrize("D", [32, 64, 128, 256])
+@pytest.mark.parametrize("S", [33, 40, 63, 97])
+def test_dense_attn_tail_stays_inside(device, D, S):
+    """Keys past S of a last, partly filled tile are not read (row kernel: 24
+    query rows, enough heads for it at every head_dim): K and V are followed
+    by NaN, which P = 0 would not hide (0 x NaN), and which must not decide
+    whether a hidden tile is skipped."""
+    from omnistack_rs.attention import reference_attn
+    B, H, T = 50, 8, 24
+    g = _data.gen(570 + S + D)
+    q = torch.randn(B, H, T, D, generator=g)
+    k, v = torch.randn(B, H, S, D, generator=g), torch.randn(B, H, S, D, generator=g)
+    mask = torch.full((T, S), float("-inf")).triu(S - T + 1)
+    mask[:, 32:] = float("-inf")               # the last tiles hidden from every query
+
+    def before_nan(t):
+        wide = torch.full((t.numel() + 64 * D,), float("nan"), device=device)
+        wide[: t.numel()] = t.to(device).reshape(-1)
+        return wide[: t.numel()].view(t.shape)
+
+    dev = (q.to(device), before_nan(k), before_nan(v))
+    _close(reference_attn(*dev), restate.reference_attn(q, k, v), f"tail S{S} D{D}")
+    _close(reference_attn(*dev, mask=mask.to(device)), restate.reference_attn(q, k, v, mask=mask), f"tail S{S} D{D} mask")
