@@ -230,7 +230,8 @@ int omni_lora_apply(const void *q, int q_dtype, const void *x, const void *A, co
  * WHT(sign_flip * q) to the query inside the kernel (the K/V cache lives in
  * rotated space); 0 reproduces omni_attn, which takes q as given.
  * Output f32 (B, Hq, T, D).  `workspace` must hold
- * omni_attn_workspace_size(...) bytes (may be 0 -> NULL allowed).
+ * omni_attn_workspace_size(...) bytes (may be 0 -> NULL allowed); the size
+ * does not drop as S grows, so the longest cache's serves every shorter one.
  * Domain: codebook centroids within fp16 range (|c| <= 65504; they are held
  * as fp16 hi + fp16 remainder pairs), S < 2^25; query rows of any finite
  * magnitude (each row is scaled by a power of two in-kernel).
@@ -285,9 +286,9 @@ int omni_attn_lora(const void *q, int q_dtype,
  * harnesses that forbid hipMalloc).  No counterpart in the reference.
  * The split-K partials live in a static device array of
  * omni_attn_noalloc_scratch_bytes() bytes (16 MiB) that each device holds
- * until the process ends; a launch needing more
- * (omni_attn_workspace_size(...) > that) returns OMNI_EWORKSPACE without
- * launching.  Calls on one device share the array: calls that overlap on
+ * until the process ends; a launch needing more (never where
+ * omni_attn_workspace_size(...) is within that) returns OMNI_EWORKSPACE
+ * without launching.  Calls on one device share the array: calls that overlap on
  * one device (several streams or threads) race.  The first call on a
  * device looks up the array's address (make it outside graph capture).
  * Results are those of omni_attn with the same arguments.

@@ -3131,6 +3131,7 @@ struct Plan {
     int spb;           // decode kernel: sequences sharing a block's 8 row slots
     int64_t split_len;
     size_t lds, ws_bytes;
+    size_t ws_most;    // the most that a cache of up to S tokens takes: the size queries' answer
 };
 
 static int64_t clamp64(int64_t v, int64_t lo, int64_t hi) { return v < lo ? lo : (v > hi ? hi : v); }
@@ -3147,15 +3148,18 @@ constexpr size_t kScratchBytes = size_t(16) << 20;
 // combine).  Candidates: no split, and the most that 1, 2 or 3 full rounds
 // hold with at least kMinSplitTiles tiles each; a split has to promise a
 // tenth (a second, partly filled round runs faster than a full one).
+// `top`: at least the splits of any shorter sequence, and no fewer for a longer
+// one (rounds and kernels change with the length, so the splits themselves can
+// drop as it grows): a workspace made for the longest cache serves every shorter.
 constexpr int64_t kMinSplitTiles = 4;
 constexpr double kCombineUs = 6.0;
 constexpr double kPartialUsPerByte = 2.0 / 3.5e6;     // written and read, 3.5 TB/s
 
 static double plan_splits(int64_t cus, int64_t units, int64_t tiles, int rows, int D, double fixed, double per_tile, int64_t least,
-                          int64_t &splits) {
+                          int64_t &splits, int64_t &top) {
     const int64_t most = tiles / kMinSplitTiles > 1 ? tiles / kMinSplitTiles : 1;
     if (most == 1 && least <= 1) {            // a short sequence, planned on every small call: no more divisions
-        splits = 1;
+        splits = top = 1;
         return (double)((units + cus - 1) / cus) * (fixed + per_tile * (double)tiles);
     }
     const size_t unit_bytes = (size_t)rows * (D + 2) * sizeof(float);
@@ -3165,10 +3169,11 @@ static double plan_splits(int64_t cus, int64_t units, int64_t tiles, int rows, i
     const int64_t fit = (int64_t)(kScratchBytes / (unit_bytes * (size_t)units));
     const int64_t cap = fit > plain ? fit : plain;
     double best = 0.0;
-    splits = 0;
+    splits = top = 0;
     for (int r = 0; r <= 3; ++r) {
         int64_t s = r == 0 ? 1 : clamp64(r * cus / units, 1, most < cap ? most : cap);
         if (s < least) s = least;
+        if (s > top) top = s;
         const double rounds = (double)((units * s + cus - 1) / cus);
         double t = rounds * (fixed + per_tile * (double)((tiles + s - 1) / s));
         if (s > 1) t += kCombineUs + (double)(unit_bytes * (size_t)(units * s)) * kPartialUsPerByte;
@@ -3220,9 +3225,12 @@ static Plan make_plan(int cus, int64_t B, int Hq, int Hkv, int64_t T, int64_t S,
         p.ncopy = tps >= 64 ? 16 : (tps >= 8 ? 4 : 1);
         p.lds = Lds<32>::total(p.ncopy, p.nw);
         p.ws_bytes = p.splits > 1 ? (size_t)units * p.splits * p.rows * (D + 2) * sizeof(float) : 0;
+        p.ws_most = p.ws_bytes;
         return p;
     }
     int64_t splits = 1, units = 0;
+    const size_t row_bytes = (size_t)(D + 2) * sizeof(float);
+    p.ws_most = 0;
     // the prefill kernel's plan (D = 32: any number of rows)
     const int nw = D == 128 ? kPreWaves : kP32Waves;
     const int ncb = D == 128 ? ((q32 || rows <= 16) ? 1 : kPreNcb) : (rows <= 16 ? 1 : ((q32 || rows <= 32) ? 2 : kP32Ncb));
@@ -3239,7 +3247,11 @@ static Plan make_plan(int cus, int64_t B, int Hq, int Hkv, int64_t T, int64_t S,
     const bool dec = D == 128 && rows <= kDecMaxRows && !zero_scale;      // the decode kernel can take it
     int64_t psplits = 1;
     double pcost = 0.0;
-    if (!dec || rows > kDecRows) pcost = plan_splits(cus, punits > 0 ? punits : 1, tiles, prows, D, pfix, ptile, 1, psplits);
+    if (!dec || rows > kDecRows) {
+        int64_t top;
+        pcost = plan_splits(cus, punits > 0 ? punits : 1, tiles, prows, D, pfix, ptile, 1, psplits, top);
+        if (top > 1) p.ws_most = (size_t)(punits * top) * prows * row_bytes;
+    }
     if (dec) {
         const int n_rchunks = (int)((rows + kDecRows - 1) / kDecRows);
         // Short decode steps of many sequences (more (sequence, kv head)
@@ -3253,7 +3265,12 @@ static Plan make_plan(int cus, int64_t B, int Hq, int Hkv, int64_t T, int64_t S,
         const int64_t least = (paged && spb == 1 && tiles > cap) ? (tiles + cap - 1) / cap : 1;
         int64_t dsplits = 1;
         double dcost = 0.0;
-        if (spb == 1) dcost = plan_splits(cus, dunits > 0 ? dunits : 1, tiles, kDecRows, D, 6.5, 0.19, least, dsplits);
+        if (spb == 1) {
+            int64_t top;
+            dcost = plan_splits(cus, dunits > 0 ? dunits : 1, tiles, kDecRows, D, 6.5, 0.19, least, dsplits, top);
+            const size_t most = top > 1 ? (size_t)(dunits * top) * kDecRows * row_bytes : 0;
+            if (most > p.ws_most) p.ws_most = most;
+        }
         if (rows <= kDecRows || dcost <= 1.1 * pcost) {
             p.dec128 = true;
             p.rows = kDecRows;
@@ -3280,15 +3297,15 @@ static Plan make_plan(int cus, int64_t B, int Hq, int Hkv, int64_t T, int64_t S,
     const int64_t tps = (tiles + splits - 1) / splits;
     p.splits = (int)((tiles + tps - 1) / tps);         // none empty
     p.split_len = tps * kDecTile;
-    p.ws_bytes = p.splits > 1 ? (size_t)units * p.splits * p.rows * (D + 2) * sizeof(float) : 0;
+    p.ws_bytes = p.splits > 1 ? (size_t)units * p.splits * p.rows * row_bytes : 0;
     return p;
 }
 
 // Split-K workspace of a contiguous-cache call, whatever its score scale
 // (a zero scale may take another kernel).
 static size_t plan_ws_bytes(int cus, int64_t B, int Hq, int Hkv, int64_t T, int64_t S, int D, bool q32) {
-    const size_t a = make_plan(cus, B, Hq, Hkv, T, S, D, q32).ws_bytes;
-    const size_t b = make_plan(cus, B, Hq, Hkv, T, S, D, q32, false, true).ws_bytes;
+    const size_t a = make_plan(cus, B, Hq, Hkv, T, S, D, q32).ws_most;
+    const size_t b = make_plan(cus, B, Hq, Hkv, T, S, D, q32, false, true).ws_most;
     return a > b ? a : b;
 }
 }  // namespace omni
@@ -3577,8 +3594,8 @@ extern "C" size_t omni_attn_paged_workspace_size(int64_t B, int Hq, int Hkv, int
     // either plan (a zero score scale runs another kernel), plus room for
     // the gather-apply LoRA fallback's q_eff
     const int64_t S = max_pages * (int64_t)page_size;
-    const size_t a = make_plan(device_cus(), B, Hq, Hkv, T, S, 128, q_dtype == OMNI_F32, true).ws_bytes;
-    const size_t z = make_plan(device_cus(), B, Hq, Hkv, T, S, 128, q_dtype == OMNI_F32, true, true).ws_bytes;
+    const size_t a = make_plan(device_cus(), B, Hq, Hkv, T, S, 128, q_dtype == OMNI_F32, true).ws_most;
+    const size_t z = make_plan(device_cus(), B, Hq, Hkv, T, S, 128, q_dtype == OMNI_F32, true, true).ws_most;
     return align256(a > z ? a : z) + (size_t)B * Hq * T * 128 * (q_dtype == OMNI_F32 ? 4 : 2);
 }
 
@@ -3668,7 +3685,10 @@ extern "C" int omni_attn_noalloc(const void *q, int q_dtype, const uint8_t *k_ni
                                  int64_t T, int64_t S, int head_dim, float scale, int with_qjl,
                                  int64_t causal_offset, int rotate_q, const int8_t *sign_flip, float *out,
                                  void *stream) {
-    const size_t need = omni_attn_workspace_size(B, Hq, Hkv, T, S, head_dim);
+    // (that size covers every shorter cache too; this launch may need less)
+    size_t need = omni_attn_workspace_size(B, Hq, Hkv, T, S, head_dim);
+    if (need > kScratchBytes)
+        need = make_plan(device_cus(), B, Hq, Hkv, T, S, head_dim, q_dtype == OMNI_F32, false, scale == 0.0f).ws_bytes;
     if (need > kScratchBytes) {
         set_error("omni_attn_noalloc: this launch needs %zu bytes of split-K scratch, more than the %zu-byte "
                   "static array; call omni_attn with a workspace instead", need, kScratchBytes);

@@ -280,6 +280,22 @@ def test_workspace_size_host_only(L):
     assert L.omni_attn_workspace_size(1, 3, 2, 1, 10, 128) == 0   # invalid GQA -> 0
 
 
+@pytest.mark.parametrize("D,T", [(128, 1), (128, 3), (128, 8), (128, 512), (32, 1), (32, 40), (32, 512)])
+@pytest.mark.parametrize("Hkv,G", [(8, 1), (8, 4), (8, 8), (1, 8)])
+def test_workspace_of_the_longest_cache_serves_shorter_ones(L, D, T, Hkv, G):
+    """A serving loop allocates once for its longest cache: the sizes never
+    drop as the cache grows (the split plans themselves do: a longer cache
+    can take fewer splits, or the kernel with the smaller partials)."""
+    for B in (1, 2, 5, 13, 64):
+        most = [0, 0, 0]
+        for S in [*range(32, 6000, 32), *range(6000, 60000, 608)]:
+            got = [L.omni_attn_workspace_size(B, Hkv * G, Hkv, T, S, D),
+                   L.omni_attn_lora_workspace_size(B, Hkv * G, Hkv, T, S, D, 2),
+                   L.omni_attn_paged_workspace_size(B, Hkv * G, Hkv, T, S // 16, 16, 2) if D == 128 else 0]
+            assert all(g >= m for g, m in zip(got, most)), (B, S, got, most)
+            most = got
+
+
 def test_host_api_rejects_cpu_tensors():
     from omnistack_rs.kernels.quantize import quantize_heads
     from omnistack_rs.kernels.fused_attention import omni_attn

@@ -110,3 +110,27 @@ def test_noalloc_refuses_oversized_partials(device):
     assert rc == _lib.OMNI_EWORKSPACE and "static array" in _lib.last_error()
     torch.cuda.synchronize()
     assert (out == 7.0).all()
+
+
+def test_noalloc_takes_launches_below_the_size_query(device):
+    """omni_attn_workspace_size covers every shorter cache as well; a launch
+    that itself needs less than the static array is taken."""
+    from omnistack_rs import _lib
+    L = _lib.lib()
+    B, Hq, Hkv, T, S, D = 1, 32, 2, 2000, 1000, 128
+    ws_bytes = L.omni_attn_workspace_size(B, Hq, Hkv, T, S, D)
+    assert ws_bytes > L.omni_attn_noalloc_scratch_bytes()
+    g = _data.gen(79)
+    kn, vn = (torch.randint(0, 256, (B, Hkv, S, 64), generator=g, dtype=torch.uint8) for _ in range(2))
+    kq = torch.randint(0, 256, (B, Hkv, S, 8), generator=g, dtype=torch.uint8)
+    kr = torch.rand(B, Hkv, S, generator=g)
+    cb = torch.linspace(-2, 2, 16).repeat(Hkv, 1)
+    q = _data.query((B, Hq, T, D), seed=80)
+    st = _lib.stream_of(device)
+    head, out_a, keep_a, _ = _args(device, q, kn, kq, kr, vn, cb, 5, -1)
+    _lib.check(L.omni_attn_noalloc(*head, st))
+    headb, out_b, keep_b, _ = _args(device, q, kn, kq, kr, vn, cb, 5, -1)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=device)
+    _lib.check(L.omni_attn(*headb, _lib.ptr(ws), ws_bytes, st))
+    torch.cuda.synchronize()
+    assert torch.isfinite(out_a).all() and torch.equal(out_a, out_b)
