@@ -32,8 +32,9 @@
 // reference's fp32 `mean()` rounds along the way: its last bits can differ,
 // and so can a convergence decision taken at the tolerance.)  Where two
 // distances of one sample can round to a tie with a lower index (centroids
-// closer than 2^-22 of the distances compared) the step goes over the
-// samples one by one instead.  Samples must be finite.
+// closer than 2^-22 of the distances compared) the step codes each bin by its
+// ends, and the samples one by one only of bins where those do not decide.
+// Samples must be finite.
 //
 // Layout: group g's samples are rows of `inner` contiguous elements:
 // element e of group g is x[(e / inner) * outer_stride + g * group_stride +
@@ -59,7 +60,6 @@ constexpr int kLmMaxBins = 32768;           // bins per group at most (their pla
 // 31 + 154 + 28 + 920 at 256 and 26 + 148 + 24 + 927 at 512 (8 x 1.64 M).
 constexpr int kLmFill = 512;
 constexpr int kLmCache = 32;                // samples per lane a boundary bin may hold in registers
-constexpr int kLmSlowSlots = 256;
 
 struct LmArgs {
     const void *x;
@@ -587,13 +587,27 @@ __device__ __forceinline__ void lm_settle_bin(LmBin &B, int lane) {
     }
 }
 
+// First-index argmin of |x - c_k| (c_k NaN: no candidate), and whether the next
+// distance lies far enough above the least one (by 2^-20 of it; rounding moves
+// either by 2^-24) that the real distances decide, not their rounding.
+__device__ __forceinline__ bool lm_code(const float *c, float x, int &code) {
+    float best = fabsf(x - c[0]), second = INFINITY;
+    code = 0;
+#pragma unroll
+    for (int k = 1; k < kLmK; ++k) {
+        const float d = fabsf(x - c[k]);
+        second = d < best ? best : fminf(second, d);
+        code = d < best ? k : code;
+        best = fminf(best, d);
+    }
+    return best < 1e38f && second > best * 1.00000095367431640625f;
+}
+
 // The whole calibration of a group: wave w finds order statistic w and then,
 // each step, boundary w and the mean of cell w.
 template <int DT>
 __global__ __launch_bounds__(kLmThreads) void lm_lloyd_kernel(LmArgs a) {
-    // places of the bins; a step that goes over the samples one by one uses
-    // the space for its sums and loads the places again
-    __shared__ __attribute__((aligned(16))) uint32_t place[kLmMaxBins + 4];
+    __shared__ uint32_t place[kLmMaxBins + 4];         // first places of the bins
     __shared__ double csum[kLmMaxBins / 64];
     __shared__ uint32_t map[kLmOct];
     __shared__ float cent2[2][kLmK], moved[kLmK];
@@ -602,19 +616,16 @@ __global__ __launch_bounds__(kLmThreads) void lm_lloyd_kernel(LmArgs a) {
     __shared__ double bval[kLmK], bright[kLmK];        // the sums of its bin's samples on its left and right,
     __shared__ double bhead[kLmK], btail[kLmK];        // and of the chunk's bins before and after that bin
     __shared__ int slow;
-    double(*const ls)[kLmSlowSlots] = reinterpret_cast<double(*)[kLmSlowSlots]>(place);
-    uint32_t(*const lc)[kLmSlowSlots] = reinterpret_cast<uint32_t(*)[kLmSlowSlots]>(place + 2 * kLmK * kLmSlowSlots);
-    static_assert(3 * kLmK * kLmSlowSlots <= kLmMaxBins, "sums of the slow step fit the places' space");
+    __shared__ float live[kLmK];                       // step by bins: the centroids, equal ones once (else NaN),
+    __shared__ double tsum[kLmThreads / 64][kLmK];                // each wave's sums and counts of the cells
+    __shared__ uint64_t tcnt[kLmThreads / 64][kLmK];
     const int g = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const double *bsum = a.bsum + (size_t)g * a.nb;
     const uint64_t *start = a.start + (size_t)g * (a.nb + 1);
-    auto load_places = [&]() {
-        if (a.wide) return;                            // 64-bit places stay in memory
+    if (!a.wide)                                       // (64-bit places stay in memory)
         for (int b = tid; b <= a.nb; b += kLmThreads) place[b] = (uint32_t)start[b];
-    };
     auto first_of = [&](int b) -> uint64_t { return a.wide ? start[b] : (uint64_t)place[b]; };
-    load_places();
     for (int c = tid; c < a.nch; c += kLmThreads) csum[c] = a.csum[(size_t)g * a.nch + c];
     if (tid < kLmOct) map[tid] = a.map[(size_t)g * kLmOct + tid];
     __syncthreads();
@@ -797,54 +808,81 @@ __global__ __launch_bounds__(kLmThreads) void lm_lloyd_kernel(LmArgs a) {
             // a centroid equal to the one before it gets no sample (first index)
             if (w == 0 || lm_lane(ck, w > 0 ? w - 1 : 0) != ca) cell(n, s);
         } else {
-            // sample by sample, in a fixed order (the places' readers of this
-            // step are past the barrier above)
-            if (tid < kLmSlowSlots) {
-                float c[kLmK];
-#pragma unroll
-                for (int k = 0; k < kLmK; ++k) {
-                    c[k] = cent[k];
-                    ls[k][tid] = 0.0;
-                    lc[k][tid] = 0u;
+            // Bin by bin: both ends coded alike, and neither near a tie, code
+            // the whole bin (between them |x - c_j| - (1 + 2^-22) |x - c_k| is
+            // least at an end); the others' samples are coded one by one.  Sums
+            // inside a bin are exact, bins and waves are added in a fixed order.
+            // 8 groups x 1.64 M samples, one of them 1e8: 28 us a step (3 us
+            // where boundaries decide; one by one in this block 3570 us, in
+            // a pass of 240 blocks over the samples 62 us).
+            if (tid < kLmK) {
+                bool again = false;
+                for (int j = 0; j < tid; ++j) again = again || cent[j] == cent[tid];
+                live[tid] = again ? __builtin_nanf("") : cent[tid];
+            }
+            __syncthreads();
+            const float *buf = a.buf + (size_t)g * a.n;
+            double ts = 0.0;                           // lane k: cell k
+            uint64_t tn = 0;
+            for (int b0 = 64 * w; b0 < a.nb; b0 += kLmThreads) {
+                const uint64_t at = first_of(b0 + lane), c = first_of(b0 + lane + 1) - at;
+                const double sum = bsum[b0 + lane];
+                int code = 0, code1 = 0;
+                bool whole = false;
+                if (c > 0) {
+                    const uint32_t key = lm_key(buf[at]), mask = (1u << (map[key >> 23] & 31u)) - 1u;
+                    const bool sure0 = lm_code(live, lm_value(key & ~mask), code);
+                    const bool sure1 = lm_code(live, lm_value(key | mask), code1);
+                    whole = sure0 && sure1 && code == code1;
                 }
-                int64_t o = a.outer > 1 ? tid / a.inner : 0, i = tid - o * a.inner;
-                const int64_t so = a.outer > 1 ? kLmSlowSlots / a.inner : 0, si = kLmSlowSlots - so * a.inner;
-                for (int64_t e = tid; e < a.n; e += kLmSlowSlots) {
-                    const int64_t idx = o * a.outer_stride + (int64_t)g * a.group_stride + i;
-                    float x;
-                    if constexpr (DT == OMNI_F32) x = reinterpret_cast<const float *>(a.x)[idx];
-                    else x = lm_widen<DT>(reinterpret_cast<const uint16_t *>(a.x)[idx]);
-                    int best = 0;
-                    float bd = fabsf(x - c[0]);
+                for (uint64_t left = __builtin_amdgcn_ballot_w64(whole); left;) {
+                    const int k = __builtin_amdgcn_readlane(code, __builtin_ctzll(left));
+                    const bool mine = whole && code == k;
+                    const double s1 = lm_wave_sum(mine ? sum : 0.0), n1 = lm_wave_sum(mine ? (double)c : 0.0);
+                    ts += lane == k ? s1 : 0.0;
+                    tn += lane == k ? (uint64_t)n1 : 0u;
+                    left &= ~__builtin_amdgcn_ballot_w64(mine);
+                }
+                for (uint64_t left = __builtin_amdgcn_ballot_w64(c > 0 && !whole); left; left &= left - 1u) {
+                    const int l = __builtin_ctzll(left);
+                    const uint64_t first = __shfl((unsigned long long)at, l), nl = __shfl((unsigned long long)c, l);
+                    double bs = 0.0;
+                    for (uint64_t e = 0; e < nl; e += 256u) {
+                        float x[4];
 #pragma unroll
-                    for (int k = 1; k < kLmK; ++k) {
-                        const float d = fabsf(x - c[k]);
-                        if (d < bd) {
-                            bd = d;
-                            best = k;
+                        for (int q = 0; q < 4; ++q) {
+                            const uint64_t i = e + 64u * q + (uint32_t)lane;
+                            x[q] = buf[first + (i < nl ? i : nl - 1u)];
+                        }
+#pragma unroll 1
+                        for (int q = 0; q < 4; ++q) {
+                            const bool in = e + 64u * q + (uint32_t)lane < nl;
+                            int cx;
+                            lm_code(live, x[0], cx);
+                            for (uint64_t some = __builtin_amdgcn_ballot_w64(in); some;) {
+                                const int k = __builtin_amdgcn_readlane(cx, __builtin_ctzll(some));
+                                const bool mine = in && cx == k;
+                                const uint64_t m = __builtin_amdgcn_ballot_w64(mine);
+                                const double s1 = lm_wave_sum(mine ? (double)x[0] : 0.0);
+                                bs += lane == k ? s1 : 0.0;
+                                tn += lane == k ? (uint64_t)__popcll(m) : 0u;
+                                some &= ~m;
+                            }
+                            x[0] = x[1]; x[1] = x[2]; x[2] = x[3];
                         }
                     }
-                    ls[best][tid] += (double)x;
-                    lc[best][tid] += 1u;
-                    o += so;
-                    i += si;
-                    if (i >= a.inner && a.outer > 1) {
-                        i -= a.inner;
-                        ++o;
-                    }
+                    ts += bs;
                 }
             }
-            __syncthreads();
-            double m = 0.0;
-#pragma unroll
-            for (int q = 0; q < kLmSlowSlots / 64; ++q) {
-                s += ls[w][64 * q + lane];
-                m += (double)lc[w][64 * q + lane];
+            if (lane < kLmK) {
+                tsum[w][lane] = ts;
+                tcnt[w][lane] = tn;
             }
-            s = lm_wave_sum(s);
-            n = (uint64_t)lm_wave_sum(m);
             __syncthreads();
-            load_places();                             // used after the next barrier
+            for (int v = 0; v < kLmThreads / 64; ++v) {
+                s += tsum[v][w];
+                n += tcnt[v][w];
+            }
         }
         const float nc = n > 0 ? (float)(s / (double)n) : ca;
         if (lane == 0) {

@@ -152,14 +152,15 @@ def _step(x: torch.Tensor, c: torch.Tensor) -> torch.Tensor:
 
 
 @pytest.mark.parametrize("kind", ["n16", "n17", "one_run", "run_plus_1", "odd_rows", "full_bins", "zeros", "outliers",
-                                  "close_levels", "tiny", "bf16_large", "f16"])
+                                  "close_levels", "tiny", "bf16_large", "f16", "one_outlier", "cluster", "bf16_close"])
 def test_steps_match_their_definition(device, kind):
     """Steps 1, 2 and 3 from the library's own initial centroids, at the edges
     of the binned passes: the smallest groups, a block's run of 32768 samples
     and one more, rows that are no multiple of four, bins with more samples
     than a wave keeps in registers, values so far out or levels so close that
-    distances to several centroids round to a tie (samples one by one),
-    denormals, 16-bit types (one value per bin)."""
+    distances to several centroids round to a tie (steps by bins: one sample
+    with a centroid of its own, half the samples within 1e-6 of each other,
+    levels an ulp apart), denormals, 16-bit types (one value per bin)."""
     g = _data.gen(450)
     n = {"n16": 16, "n17": 17, "one_run": 32768, "run_plus_1": 32769, "odd_rows": 3 * 4099}.get(kind, 50000)
     x = torch.randn(n, generator=g)
@@ -172,6 +173,13 @@ def test_steps_match_their_definition(device, kind):
         x[:4000] *= 1e30
     elif kind == "close_levels":
         x = 1.0 + torch.randint(0, 20, (n,), generator=g) * 2.0 ** -23
+    elif kind == "one_outlier":
+        x[1234] = 1e8
+    elif kind == "cluster":
+        x = torch.where(torch.rand(n, generator=g) < 0.9, 1e-6 * torch.rand(n, generator=g), 100 * torch.rand(n, generator=g))
+    elif kind == "bf16_close":
+        x = (1.0 + torch.randint(0, 24, (n,), generator=g) * 2.0 ** -7).to(torch.bfloat16)
+        x[77] = 3e30
     elif kind == "tiny":
         x *= 1e-39
     elif kind == "bf16_large":
@@ -192,3 +200,31 @@ def test_steps_match_their_definition(device, kind):
         c = _step(x.float(), c)
         assert int(done[-1]) == it
         assert torch.equal(got[-1].cpu(), c.sort().values), f"{kind} step {it}"
+
+
+def test_an_outlier_does_not_slow_the_steps(device):
+    """One sample per head so far out that it keeps a centroid to itself puts
+    every distance up to it beyond the other centroids' gaps: each step then
+    codes bins, not 1.6 M samples one by one (which took thousands of times a
+    plain step)."""
+    from omnistack_rs.quantization.codebook import _lloyd_max_hip
+    n, steps = 1638400, 24
+    x = torch.randn(8, n, generator=torch.Generator(device=device).manual_seed(470), device=device)
+
+    def seconds(x):
+        times = []
+        for _ in range(4):
+            e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+            e[0].record()
+            _, done = _lloyd_max_hip(x, 8, 1, n, 0, n, steps, 0.0)
+            e[1].record()
+            torch.cuda.synchronize()
+            assert done.tolist() == [steps] * 8
+            times.append(e[0].elapsed_time(e[1]))
+        return min(times)
+
+    plain = seconds(x)
+    x[:, 5] = 1e8
+    far = seconds(x)
+    print(f"[calib] {steps} steps: {plain:.3f} ms, with an outlier a head {far:.3f} ms", flush=True)
+    assert far < 8 * plain
