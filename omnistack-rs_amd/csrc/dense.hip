@@ -218,8 +218,9 @@ __global__ __launch_bounds__(64 * kDnWaves, D == 256 ? 1 : (D == 128 ? 3 : 4)) v
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int n = lane & 15, g = lane >> 4;
     // the last rows first: under a causal mask they are the longest
-    const int64_t bh = (int64_t)a.Hkv * a.B, id = blockIdx.x;
+    const int64_t bh = (int64_t)a.Hkv * a.B, id = (int64_t)blockIdx.y * gridDim.x + blockIdx.x;
     const int64_t chunk = (a.rows + kDnRows - 1) / kDnRows - 1 - id / bh, b = id % bh / a.Hkv;
+    if (chunk < 0) return;                        // past the last block
     const int hk = (int)(id % bh % a.Hkv);
     const int64_t row0 = chunk * kDnRows + 16 * wave;
 
@@ -536,8 +537,11 @@ extern "C" int omni_dense_attn(const float *q, const float *k, const float *v, c
         OMNI_CHECK_LAUNCH("omni_dense_attn");
         return OMNI_OK;
     }
-    OMNI_CHECK_ARG(blocks <= 2147483647, "omni_dense_attn: grid too large");
-    const dim3 grid((unsigned)blocks), block(64 * kDnWaves);
+    // a launch takes fewer than 2^32 threads in a dimension (more are cut off
+    // without an error): 2^22 blocks in x, the rest in y
+    const int64_t gx = blocks < (int64_t(1) << 22) ? blocks : int64_t(1) << 22, gy = (blocks + gx - 1) / gx;
+    OMNI_CHECK_ARG(gy <= 65535, "omni_dense_attn: grid too large");
+    const dim3 grid((unsigned)gx, (unsigned)gy), block(64 * kDnWaves);
     switch (head_dim) {
         case 32: launch_rows<32>(grid, block, st, a); break;
         case 64: launch_rows<64>(grid, block, st, a); break;

@@ -172,3 +172,21 @@ def test_dense_attn_tail_stays_inside(device, D, S):
     dev = (q.to(device), before_nan(k), before_nan(v))
     _close(reference_attn(*dev), restate.reference_attn(q, k, v), f"tail S{S} D{D}")
     _close(reference_attn(*dev, mask=mask.to(device)), restate.reference_attn(q, k, v, mask=mask), f"tail S{S} D{D} mask")
+
+
+def test_dense_attn_many_blocks(device):
+    """More blocks than one grid dimension of 256-thread blocks holds (2^24; a
+    launch of more is cut off without an error): sequences of one key, so
+    every query row is that key's value.  79 GB."""
+    from omnistack_rs.attention import reference_attn
+    torch.cuda.empty_cache()
+    B, H, T, D = 4096, 4097, 17, 32
+    v = torch.randn(B, H, 1, D, generator=torch.Generator(device=device).manual_seed(580), device=device)
+    q = torch.zeros(B, H, T, D, device=device)
+    out = reference_attn(q, v, v)
+    del q
+    for b in range(0, B, 512):
+        same = torch.equal(out[b:b + 512], v[b:b + 512].expand(-1, -1, T, -1))
+        assert same, f"batch {b}"
+    del out, v
+    torch.cuda.empty_cache()
