@@ -122,13 +122,15 @@ __global__ __launch_bounds__(256) void code_table_kernel(const float *codebooks,
 //   f32     element 32 s + 16 (i / 4) + 4 g + i % 4
 // 102,400 f32 rows of 128: 85 us with a lane per row before, 19 us (5.5 TB/s)
 // now; 2^20 bf16 rows 1360 -> 104 us.
+constexpr int64_t kWhtGridX = 65536;
+
 template <int XDT, int D>
 __global__ __launch_bounds__(256) void wht_kernel(const void *x, int64_t rows, const int8_t *sign_flip, void *out,
                                                   float scale) {
     constexpr int kSets = D == 128 ? 1 : 4;
     constexpr bool F32 = XDT == OMNI_F32;
     const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
-    const int64_t v0 = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * (16 * kSets);
+    const int64_t v0 = (((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * 4 + (threadIdx.x >> 6)) * (16 * kSets);
     if (v0 >= rows) return;
     auto at = [&](int s, int i) {                      // element offset of x[s][i] (i a multiple of 4 or 8)
         const int64_t r = v0 + n + (D == 128 ? 0 : 16 * s);
@@ -1290,7 +1292,9 @@ extern "C" int omni_wht_rotate(const void *x, int dtype, int64_t rows, int head_
     OMNI_CHECK_ARG(rows == 0 || (x && out), "omni_wht_rotate: NULL pointer");
     if (rows == 0) return OMNI_OK;
     const int per_block = 4 * (head_dim == 128 ? 16 : 64);
-    const dim3 grid((unsigned)((rows + per_block - 1) / per_block)), block(256);
+    // (two dimensions: a launch of 2^32 threads or more in one is cut off)
+    const int64_t blocks = (rows + per_block - 1) / per_block, gx = blocks < kWhtGridX ? blocks : kWhtGridX;
+    const dim3 grid((unsigned)gx, (unsigned)((blocks + gx - 1) / gx)), block(256);
     const float s = inv_sqrt_dim_f32(head_dim);
     hipStream_t st = as_stream(stream);
     if (head_dim == 128) {

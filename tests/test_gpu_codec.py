@@ -487,3 +487,17 @@ def test_qjl_module_other_dims_on_device(device):
     assert (signs.cpu() != ((err @ G.T) >= 0)).sum().item() <= 1
     with pytest.raises(RuntimeError, match="HIP devices only"):
         qjl.encode(err, 2, user_id=9)
+
+
+def test_wht_rows_past_one_grid_dimension(device):
+    """65536 blocks of 64 rows fill the launch's first dimension; the rows
+    behind them (second dimension) are rotated too, in place as well."""
+    from omnistack_rs import _lib
+    n, D = 65536 * 64 + 70, 128
+    x = torch.randn(n, D, generator=torch.Generator(device=device).manual_seed(350), device=device).to(torch.bfloat16)
+    parts = [slice(0, 64), slice(65536 * 64 - 70, n)]
+    want = [restate.rotate(x[p].cpu(), None) for p in parts]
+    _lib.check(_lib.lib().omni_wht_rotate(_lib.ptr(x), _lib.dtype_code(x.dtype), n, D, None, _lib.ptr(x),
+                                          _lib.stream_of(device)))
+    for p, w in zip(parts, want):
+        assert torch.equal(x[p].cpu().view(torch.int16), w.view(torch.int16))
