@@ -191,12 +191,18 @@ int omni_dense_attn(const float *q, const float *k, const float *v, const float 
  * finite, n >= 16.  Means are taken from fp64 sums in a fixed order
  * (deterministic); the reference's fp32 mean() can differ in the last bits.
  * iters_out (device int32 per group, nullable) receives the steps run.
- * workspace: omni_lloyd_max_workspace_size(...) bytes.
+ * workspace: omni_lloyd_max_workspace_size(...) bytes: about 4 per sample,
+ * the samples are stored once by bins of their value (8 groups x 1.64 M
+ * samples, 300 steps 1.3 ms).  A smaller one, down to
+ * omni_lloyd_max_workspace_least(...) bytes (0.1 MB a group at most), gives
+ * the same recipe with a pass over the samples in place per step (17.7 ms;
+ * the sums' order, so the last bits of a mean, can differ).
  * Replaces LloydMaxCalibrator.fit / calibrate_codebook / calibrate_per_group
  * (omnistack_rs/quantization/codebook.py:64-108, :129-172) as the bake calls
  * them (scripts/run_criteo_benchmark.py:357-362).
  */
 size_t omni_lloyd_max_workspace_size(int n_groups, int64_t outer, int64_t inner);
+size_t omni_lloyd_max_workspace_least(int n_groups, int64_t outer, int64_t inner);
 
 int omni_lloyd_max(const void *x, int x_dtype, int n_groups, int64_t outer, int64_t inner,
                    int64_t outer_stride, int64_t group_stride, int max_iters, float tol,

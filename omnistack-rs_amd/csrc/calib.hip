@@ -15,7 +15,8 @@
 // A Lloyd step needs no pass over the samples.  They are counted and stored
 // once by bins of their order-preserving key: a bin is one exponent (of one
 // sign) or a power-of-two part of it, as fine as its share of the samples
-// asks for (up to 512 a bin on average).  One exponent per bin makes the fp64 sum of up
+// asks for (up to 512 a bin on average).  (calib_inplace.hip calibrates where
+// there is no room for that copy.)  One exponent per bin makes the fp64 sum of up
 // to 2^29 of its samples exact in any order.  Under sorted centroids the
 // codes ascend with x, so cell k is a run of whole bins between two boundary
 // bins plus a part of each: per boundary the largest fp32 value that still
@@ -44,11 +45,10 @@
 #include <float.h>
 #include <math.h>
 
-#include "omni_common.h"
+#include "calib.h"
 
 namespace omni {
 
-constexpr int kLmK = 16;                    // centroids
 constexpr int kLmThreads = 1024;
 constexpr int kLmPer = 32;                  // samples per thread of the counting and storing passes
 constexpr int kLmBlock = kLmThreads * kLmPer;
@@ -82,14 +82,6 @@ struct LmArgs {
     float *out;             // [g][16]
     int32_t *iters;         // [g], nullable
 };
-
-__device__ __forceinline__ uint32_t lm_key(float f) {
-    const uint32_t u = __float_as_uint(f);
-    return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
-}
-__device__ __forceinline__ float lm_value(uint32_t k) {
-    return __uint_as_float((k & 0x80000000u) ? (k & 0x7fffffffu) : ~k);
-}
 
 template <int DT>
 __device__ __forceinline__ float lm_widen(uint16_t h) {
@@ -914,8 +906,6 @@ __global__ __launch_bounds__(kLmThreads) void lm_lloyd_kernel(LmArgs a) {
     }
 }
 
-static size_t align256c(size_t x) { return (x + 255) & ~(size_t)255; }
-
 // Bins by the samples per group: kLmFill samples a bin, or as many as keep
 // 2 n / fill + 512 within kLmMaxBins.
 static void lm_shape(int x_dtype, int64_t n, LmArgs &a) {
@@ -933,7 +923,7 @@ static size_t lm_layout(int groups, int64_t n, char *base, LmArgs &a) {
     size_t off = 0;
     auto take = [&](size_t bytes) {
         char *p = base ? base + off : nullptr;
-        off = align256c(off + bytes);
+        off = lm_align256(off + bytes);
         return p;
     };
     const size_t gr = (size_t)groups;
@@ -975,6 +965,13 @@ extern "C" size_t omni_lloyd_max_workspace_size(int n_groups, int64_t outer, int
     return lm_layout(n_groups, outer * inner, nullptr, a);
 }
 
+extern "C" size_t omni_lloyd_max_workspace_least(int n_groups, int64_t outer, int64_t inner) {
+    if (n_groups <= 0 || outer <= 0 || inner <= 0 || outer > INT64_MAX / inner) return 0;
+    const size_t all = omni_lloyd_max_workspace_size(n_groups, outer, inner);
+    const size_t least = lm_inplace_bytes(n_groups, outer * inner);
+    return least < all ? least : all;
+}
+
 extern "C" int omni_lloyd_max(const void *x, int x_dtype, int n_groups, int64_t outer, int64_t inner,
                               int64_t outer_stride, int64_t group_stride, int max_iters, float tol,
                               float *codebooks, int32_t *iters_out, void *workspace, size_t workspace_bytes,
@@ -988,6 +985,18 @@ extern "C" int omni_lloyd_max(const void *x, int x_dtype, int n_groups, int64_t 
     OMNI_CHECK_ARG(n >= kLmK, "omni_lloyd_max: need at least 16 samples per group, got %lld", (long long)n);
     OMNI_CHECK_ARG(max_iters >= 0 && max_iters <= 100000, "omni_lloyd_max: max_iters must be in [0, 100000]");
     OMNI_CHECK_ARG(x && codebooks, "omni_lloyd_max: NULL pointer");
+    const size_t least = omni_lloyd_max_workspace_least(n_groups, outer, inner);
+    if (workspace == nullptr || workspace_bytes < least) {
+        set_error("omni_lloyd_max: workspace of %zu bytes required, %zu given", least, workspace_bytes);
+        return OMNI_EWORKSPACE;
+    }
+    hipStream_t st = as_stream(stream);
+    if (workspace_bytes < omni_lloyd_max_workspace_size(n_groups, outer, inner)) {
+        lm_inplace_run({x, x_dtype, n_groups, outer, inner, outer_stride, group_stride, max_iters, tol, codebooks, iters_out},
+                       workspace, st);
+        OMNI_CHECK_LAUNCH("omni_lloyd_max");
+        return OMNI_OK;
+    }
     LmArgs a;
     a.x = x;
     a.outer = outer; a.inner = inner; a.outer_stride = outer_stride; a.group_stride = group_stride;
@@ -1001,13 +1010,7 @@ extern "C" int omni_lloyd_max(const void *x, int x_dtype, int n_groups, int64_t 
     // 4-element loads: every run of four lies in one row and is aligned
     a.vec = (inner % 4 == 0 && outer_stride % 4 == 0 && group_stride % 4 == 0 &&
              (uintptr_t)x % (4 * dtype_size(x_dtype)) == 0) ? 1 : 0;
-    const size_t need = omni_lloyd_max_workspace_size(n_groups, outer, inner);
-    if (workspace == nullptr || workspace_bytes < need) {
-        set_error("omni_lloyd_max: workspace of %zu bytes required, %zu given", need, workspace_bytes);
-        return OMNI_EWORKSPACE;
-    }
     lm_layout(n_groups, n, reinterpret_cast<char *>(workspace), a);
-    hipStream_t st = as_stream(stream);
     if (x_dtype == OMNI_F32) lm_launch<OMNI_F32>(a, n_groups, st);
     else if (x_dtype == OMNI_BF16) lm_launch<OMNI_BF16>(a, n_groups, st);
     else lm_launch<OMNI_F16>(a, n_groups, st);

@@ -10,7 +10,8 @@ the result is sorted ascending.
 
 Samples on a HIP device run ``omni_lloyd_max`` (csrc/calib.hip: samples
 stored by bins of their value once, every Lloyd step from the bins, fp64 cell
-sums in a fixed order);
+sums in a fixed order; where the device has no room for that copy of them,
+csrc/calib_inplace.hip: a pass over the samples per step);
 ``calibrate_heads`` calibrates every head of a (B, H, T, D) cache in one
 call without copying the per-head samples.  CPU samples run the same recipe
 with torch on the CPU, as the reference does.  Either way cell means are not
@@ -48,7 +49,11 @@ def _lloyd_max_hip(x: torch.Tensor, groups: int, outer: int, inner: int, outer_s
     dev = x.device
     L = _lib.lib()
     ws_bytes = L.omni_lloyd_max_workspace_size(groups, outer, inner)
-    ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
+    try:
+        ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
+    except torch.OutOfMemoryError:
+        ws_bytes = L.omni_lloyd_max_workspace_least(groups, outer, inner)
+        ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
     out = torch.empty(groups, N_CENTROIDS, dtype=torch.float32, device=dev)
     iters = torch.empty(groups, dtype=torch.int32, device=dev)
     _lib.check(L.omni_lloyd_max(_lib.ptr(x), _lib.dtype_code(x.dtype), groups, outer, inner, outer_stride,

@@ -202,6 +202,36 @@ def test_steps_match_their_definition(device, kind):
         assert torch.equal(got[-1].cpu(), c.sort().values), f"{kind} step {it}"
 
 
+@pytest.mark.parametrize("kind,dtype", [("normal", torch.float32), ("ties", torch.float32), ("ties", torch.bfloat16),
+                                        ("tiny_n", torch.float16)])
+def test_calibration_without_room_for_a_copy(device, kind, dtype, monkeypatch):
+    """Where the device cannot hold the stored samples the call runs with the
+    least workspace, in place: the same initial centroids and steps (means
+    from fp64 sums of another order: one ulp), refused below that size."""
+    from omnistack_rs import _lib
+    from omnistack_rs.quantization.codebook import _lloyd_max_hip
+    L = _lib.lib()
+    n = 17 if kind == "tiny_n" else 60001
+    x = torch.randn(2, n, generator=_data.gen(480))
+    if kind == "ties":
+        x = torch.round(x * 4) / 4 + 0.125
+    x = x.to(dtype).to(device)
+    args = (x, 2, 1, n, 0, n)
+    want = [_lloyd_max_hip(*args, it, 0.0) for it in (0, 1, 40)]
+    least = L.omni_lloyd_max_workspace_least(2, 1, n)
+    assert 0 < least <= L.omni_lloyd_max_workspace_size(2, 1, n) and least < 1 << 18
+    monkeypatch.setattr(L, "omni_lloyd_max_workspace_size", lambda *a: 1 << 50)      # more than any device has
+    got = [_lloyd_max_hip(*args, it, 0.0) for it in (0, 1, 40)]
+    for (c0, i0), (c1, i1), steps in zip(want, got, (0, 1, 40)):
+        assert i0.tolist() == i1.tolist() == [steps] * 2
+        assert torch.allclose(c0, c1, rtol=2.0 ** -23 if steps < 2 else 1e-6, atol=1e-9 if steps < 2 else 1e-6)
+    out = torch.empty(2, 16, device=device)
+    ws = torch.empty(least, dtype=torch.uint8, device=device)
+    rc = L.omni_lloyd_max(_lib.ptr(x), _lib.dtype_code(dtype), 2, 1, n, 0, n, 1, 0.0, _lib.ptr(out), None, _lib.ptr(ws),
+                          least - 1, _lib.stream_of(device))
+    assert rc == _lib.OMNI_EWORKSPACE
+
+
 def test_an_outlier_does_not_slow_the_steps(device):
     """One sample per head so far out that it keeps a centroid to itself puts
     every distance up to it beyond the other centroids' gaps: each step then
