@@ -681,3 +681,15 @@ def test_attn_decode_or_prefill_rows(device, B, T, S):
         want = restate.fused_attn_python(q[sl].float(), kn[sl], kq[sl], kr[sl], vn[sl], cb, uid, 1 / math.sqrt(128), True)
         _assert_close(got[sl], want, f"B{B} T{T} S{S} b{b}")
         _assert_close(paged[sl], want, f"paged B{B} T{T} S{S} b{b}")
+
+
+@pytest.mark.parametrize("D,rows", [(128, 40), (32, 5), (32, 70)])
+def test_attn_sign_flip_past_an_aligned_address(device, D, rows):
+    """The prefill kernels read the sign flip eight bytes at a time, from any address."""
+    B, Hkv, S, uid = 1, 2, 200, 5
+    kn, kq, kr, vn, cb = _random_packed(B, Hkv, S, D, seed=720)
+    q = torch.randn(B, Hkv, rows, D, generator=_data.gen(721)).bfloat16()
+    sign = _data.sign_flip(D).to(device)
+    past = torch.cat([sign[:3], sign])[3:]
+    got = [_run(device, q, kn, kq, kr, vn, cb, uid, rotate_q=True, sign_flip=s) for s in (sign, past)]
+    assert past.data_ptr() % 8 and torch.equal(*got)

@@ -501,3 +501,56 @@ def test_wht_rows_past_one_grid_dimension(device):
                                           _lib.stream_of(device)))
     for p, w in zip(parts, want):
         assert torch.equal(x[p].cpu().view(torch.int16), w.view(torch.int16))
+
+
+@pytest.mark.parametrize("B,T,D,dtype", [(100, 37, 128, torch.float32), (4, 2500, 128, torch.float32),
+                                          (1, 63, 128, torch.bfloat16), (350, 37, 32, torch.bfloat16),
+                                          (26000, 1, 32, torch.float16), (5, 5200, 32, torch.float32)])
+def test_encode_grid_runs_of_rows(device, B, T, D, dtype):
+    """Enough rows per head that a wave of encode_grid_kernel takes a second
+    and third group (3072 rows of 128, 12288 of 32 for K and V of 8 heads
+    fill one per wave): groups that wrap over batch entries, one-token
+    entries, ragged ends.  K against the oracle, V bit-equal to its own call
+    (another split of the rows)."""
+    from omnistack_rs.kernels.quantize import PackedKVEncoder, encode_kv
+    H, uid = 8, 9
+    print(f"[encode] grid B={B} T={T} D={D} {dtype}", flush=True)
+    k, v = (_data.kv((B, H, T, D), seed=360 + i, dtype=dtype) for i in range(2))
+    s = _data.sign_flip(D)
+    cb = _data.gaussian_codebook(H) * torch.linspace(0.8, 1.3, H).reshape(H, 1)
+    enc = PackedKVEncoder(cb.to(device), H, user_id=uid, sign_flip=s.to(device), dtype=dtype, head_dim=D)
+    got_k, got_v = enc.encode(k.to(device), v.to(device))
+    _check_encode(restate.rotate(k, s), cb, uid, *got_k, tag=f"grid {B}x{T} D{D}")
+    alone = encode_kv(v.to(device), cb.to(device), user_id=uid, sign_flip=s.to(device))
+    assert all(torch.equal(g, w) for g, w in zip(got_v, alone))
+
+
+@pytest.mark.parametrize("D", [128, 32])
+def test_codec_past_aligned_addresses(device, D):
+    """Inputs and outputs one element past an aligned address give the same
+    bits (the kernels' wide accesses need the elements' alignment only)."""
+    from omnistack_rs import _lib
+    L, st = _lib.lib(), _lib.stream_of(device)
+    H, T, uid = 2, 83, 4
+    keep = []
+
+    def off(t):
+        keep.append(torch.cat([t.reshape(-1)[:1], t.reshape(-1)]).to(device)[1:])
+        return _lib.ptr(keep[-1])
+
+    room = lambda n, dt: torch.zeros(n + 1, dtype=dt, device=device)[1:]
+    cb = (_data.gaussian_codebook(H) * torch.linspace(0.8, 1.3, H).reshape(H, 1)).to(device)
+    gb = _lib.g_bits(_lib.head_seeds(uid, H), D, device)
+    s = _data.sign_flip(D)
+    for dtype in (torch.bfloat16, torch.float32):
+        x = _data.kv((1, H, T, D), seed=370, dtype=dtype)
+        y = room(x.numel(), dtype)
+        _lib.check(L.omni_wht_rotate(off(x), _lib.dtype_code(dtype), H * T, D, off(s), _lib.ptr(y), st))
+        assert torch.equal(y.view(x.shape).cpu(), restate.rotate(x, s))
+    nib, qjl = (torch.randint(0, 256, (1, H, T, D // n), generator=_data.gen(371), dtype=torch.uint8) for n in (2, 16))
+    nrm = torch.rand(1, H, T, generator=_data.gen(372))
+    out = room(H * T * D, torch.float32)
+    _lib.check(L.omni_dequantize(off(nib), off(qjl), off(nrm), _lib.ptr(cb), 1, _lib.ptr(gb),
+                                 1, H, T, D, 1, _lib.ptr(out), st))
+    want = restate.dequantize_heads(nib, qjl, nrm, cb.cpu(), user_id=uid)
+    assert torch.equal(out.view(want.shape).cpu(), want)

@@ -650,3 +650,76 @@ def test_paged_pairs_by_length(device, B):
             want = restate.fused_attn_python(q[b:b + 1].float(), kn[c:c + 1, :, :L], kq[c:c + 1, :, :L], kr[c:c + 1, :, :L],
                                              vn[c:c + 1, :, :L], cb, uid, 1 / math.sqrt(128), True)
             _assert_close(got[b:b + 1], want, f"by length {kind} B{B} b{b} len{L}")
+
+
+@pytest.mark.parametrize("T,with_qjl,lora", [(1, True, True), (1, False, True), (2, True, True), (2, False, False)])
+def test_paged_pairs_by_length_variants(device, T, with_qjl, lora):
+    """Pairs by length with the fused adapter prologue (a user's adapter goes
+    with its sequence, not with its place in the pair), without QJL, and with
+    two causal tokens per sequence (four query rows either way)."""
+    from omnistack_rs.cache import PagedKVCache, paged_attention
+    B, Hkv, S, uid, ps, NL, HID = 65, 8, 1600, 3, 16, 7, 128
+    Hq = Hkv * 4 // T
+    g = torch.Generator().manual_seed(640 + T)
+    kn, kq, kr, vn = (t.cpu() for t in _random_cache("cpu", 8, Hkv, S, 641))
+    cb = torch.sort(torch.randn(Hkv, 16, generator=g), dim=1).values
+    q = _data.query((B, Hq, T, 128), seed=642)
+    cache, pt8, _ = PagedKVCache.from_contiguous(*(t.to(device) for t in (kn, kq, kr, vn)), page_size=ps)
+    src = torch.arange(B) % 8
+    lens = torch.randint(T, S + 1, (B,), generator=g)
+    la, lb = (t.to(torch.bfloat16) for t in _data.lora_bank(NL, 8, HID, Hq * 128, seed=643))
+    ids = torch.randint(-1, NL, (B,), generator=g, dtype=torch.int32)
+    x = _data.query((B, T, HID), seed=644)
+    kw = dict(x=x.to(device), lora_a=la.to(device), lora_b=lb.to(device), lora_indices=ids.to(device), lora_alpha=8.0) if lora else {}
+    got = paged_attention(q.to(device), cache, pt8[src.to(device)].contiguous(), lens.to(torch.int32).to(device), cb.to(device),
+                          user_id=uid, with_qjl=with_qjl, causal=True, **kw).cpu()
+    qe = restate.apply_lora_to_q(q, x, la, lb, ids, 8.0) if lora else q
+    assert not lora or (qe.float() - q.float()).abs().mean() > 0.05       # the adapters matter
+    order = lens.argsort()
+    for b in sorted({0, 1, B // 2, B - 1, *order[:3].tolist(), *order[-3:].tolist(), int(order[B // 2])}):
+        L, c = int(lens[b]), int(src[b])
+        want = restate.fused_attn_python(qe[b:b + 1].float(), kn[c:c + 1, :, :L], kq[c:c + 1, :, :L], kr[c:c + 1, :, :L],
+                                         vn[c:c + 1, :, :L], cb, uid, 1 / math.sqrt(128), with_qjl,
+                                         mask=_causal_mask(T, L, L - T))
+        _assert_close(got[b:b + 1], want, f"by length T{T} qjl{with_qjl} lora{lora} b{b} len{L}")
+
+
+@pytest.mark.parametrize("B,Hq,T,S", [(40, 8, 32, 2100), (3, 64, 3, 20011), (2, 8, 12, 100)])
+def test_rows_between_kernels_with_adapters(device, B, Hq, T, S):
+    """9 to 32 query rows with adapters: where the prefill kernel is planned
+    (the first two shapes, the second in several splits) the update runs
+    ahead of it into the workspace behind the split partials, and the result
+    is that of the updated queries bit for bit; a decode block (the third)
+    updates in its prologue.  Contiguous, pool-indexed and paged; ids of -1
+    and past the bank."""
+    from omnistack_rs.cache import PagedKVAttention
+    from omnistack_rs.kernels.fused_attention import PackedKVAttention, _apply_lora_to_q
+    Hkv, uid, NL, HID = 8, 6, 5, 128
+    kn, kq, kr, vn = _random_cache(device, B, Hkv, S, 650)
+    cb = torch.sort(torch.randn(Hkv, 16, generator=_data.gen(651)), dim=1).values.to(device)
+    q = _data.query((B, Hq, T, 128), seed=652).to(device)
+    la, lb = (t.to(torch.bfloat16).to(device) for t in _data.lora_bank(NL, 8, HID, Hq * 128, seed=653))
+    ids = (torch.arange(B, dtype=torch.int32) % (NL + 2) - 1).to(device)      # -1, 0 .. NL - 1, NL (past the bank)
+    x = _data.query((B, T, HID), seed=654).to(device)
+    qe = _apply_lora_to_q(q, x, la, lb, ids, 8.0, validate=False)
+    order = torch.randperm(B, generator=_data.gen(655)).to(device)
+    cache, pt, lens = _paged(device, kn, kq, kr, vn, 16, seed=43)
+    kw, bank = dict(user_id=uid, q_tokens=T), dict(lora_a=la, lora_b=lb, lora_alpha=8.0)
+    runs = {"contiguous": lambda **b: PackedKVAttention(kn, kq, kr, vn, cb, Hq, **kw, **b),
+            "pool": lambda **b: PackedKVAttention(kn, kq, kr, vn, cb, Hq, batch=B, **kw, **b),
+            "paged": lambda **b: PagedKVAttention(cache, cb, n_heads=Hq, batch=B, max_pages=pt.shape[1], **kw, **b)}
+    for name, make in runs.items():
+        more = dict(cache_index=order) if name == "pool" else {}
+        pages = (pt, lens) if name == "paged" else ()
+        got, want = make(**bank).run(q, *pages, x, ids, **more), make().run(qe, *pages, **more)
+        nan = torch.isnan(want)
+        print(f"[rows+lora] {name} B{B} T{T} S{S}: {nan.float().mean().item():.3f} NaN, "
+              f"{(got - want)[~nan].abs().max().item():.2e} off", flush=True)
+        assert torch.equal(torch.isnan(got), nan)
+        if B == 2:
+            _assert_close(got[~nan].cpu(), want[~nan].cpu(), name)
+        else:
+            same = torch.equal(got[~nan], want[~nan])
+            assert same, name
+    bad = ids == NL
+    assert torch.equal(nan, bad.view(B, 1, 1, 1).expand_as(nan))
