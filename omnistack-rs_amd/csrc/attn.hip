@@ -3151,6 +3151,9 @@ constexpr size_t kScratchBytes = size_t(16) << 20;
 // `top`: at least the splits of any shorter sequence, and no fewer for a longer
 // one (rounds and kernels change with the length, so the splits themselves can
 // drop as it grows): a workspace made for the longest cache serves every shorter.
+// More rounds count for it only where they give more splits a round: otherwise
+// they never win (what rounding up a split's tiles can gain is less than a
+// round's fixed part).
 constexpr int64_t kMinSplitTiles = 4;
 constexpr double kCombineUs = 6.0;
 constexpr double kPartialUsPerByte = 2.0 / 3.5e6;     // written and read, 3.5 TB/s
@@ -3169,11 +3172,18 @@ static double plan_splits(int64_t cus, int64_t units, int64_t tiles, int rows, i
     const int64_t fit = (int64_t)(kScratchBytes / (unit_bytes * (size_t)units));
     const int64_t cap = fit > plain ? fit : plain;
     double best = 0.0;
-    splits = top = 0;
+    splits = 0;
+    top = least > 1 ? least : 1;
+    int64_t top_full = 1, top_rounds = (units + cus - 1) / cus;
     for (int r = 0; r <= 3; ++r) {
-        int64_t s = r == 0 ? 1 : clamp64(r * cus / units, 1, most < cap ? most : cap);
+        const int64_t full = r * cus / units > 1 ? r * cus / units : 1, full_rounds = (units * full + cus - 1) / cus;
+        int64_t s = clamp64(full, 1, most < cap ? most : cap);
         if (s < least) s = least;
-        if (s > top) top = s;
+        if (full * top_rounds > top_full * full_rounds) {
+            top_full = full;
+            top_rounds = full_rounds;
+            if (s > top) top = s;
+        }
         const double rounds = (double)((units * s + cus - 1) / cus);
         double t = rounds * (fixed + per_tile * (double)((tiles + s - 1) / s));
         if (s > 1) t += kCombineUs + (double)(unit_bytes * (size_t)(units * s)) * kPartialUsPerByte;

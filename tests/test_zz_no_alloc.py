@@ -117,7 +117,7 @@ def test_noalloc_takes_launches_below_the_size_query(device):
     that itself needs less than the static array is taken."""
     from omnistack_rs import _lib
     L = _lib.lib()
-    B, Hq, Hkv, T, S, D = 1, 32, 2, 2000, 1000, 128
+    B, Hq, Hkv, T, S, D = 3, 32, 8, 512, 1000, 128
     ws_bytes = L.omni_attn_workspace_size(B, Hq, Hkv, T, S, D)
     assert ws_bytes > L.omni_attn_noalloc_scratch_bytes()
     g = _data.gen(79)
