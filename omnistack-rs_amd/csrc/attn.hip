@@ -3161,9 +3161,12 @@ constexpr double kPartialUsPerByte = 2.0 / 3.5e6;     // written and read, 3.5 T
 static double plan_splits(int64_t cus, int64_t units, int64_t tiles, int rows, int D, double fixed, double per_tile, int64_t least,
                           int64_t &splits, int64_t &top) {
     const int64_t most = tiles / kMinSplitTiles > 1 ? tiles / kMinSplitTiles : 1;
-    if (most == 1 && least <= 1) {            // a short sequence, planned on every small call: no more divisions
+    const double whole = (double)((units + cus - 1) / cus) * (fixed + per_tile * (double)tiles);
+    // a short sequence, planned on every small call: too few tiles, or no time
+    // for a split block and the combine launch within nine tenths of `whole`
+    if (least <= 1 && (most == 1 || 0.9 * whole <= fixed + kCombineUs)) {
         splits = top = 1;
-        return (double)((units + cus - 1) / cus) * (fixed + per_tile * (double)tiles);
+        return whole;
     }
     const size_t unit_bytes = (size_t)rows * (D + 2) * sizeof(float);
     // as many as one block per CU asks for, of at least 16 tiles, whatever
