@@ -78,7 +78,7 @@ struct AttnArgs {
     const int32_t *seq_lens;
     int64_t max_pages, n_pages;
     int page_size, page_shift;  // page_size = 2^page_shift >= 16
-    int by_len;                // two sequences per block: pair the longest with the shortest
+    int by_len;                // two sequences per block: pair the longest with the shortest where neighbours differ
     float qscale;              // scale * log2(e)
     float alpha_c;             // fp32 sqrt(2/pi)/D (the row scale multiplies the whole score)
     float wht_scale;
@@ -1052,63 +1052,6 @@ __global__ __launch_bounds__(64 * kDecWaves) void attn_decode128_kernel(AttnArgs
 
     int b32 = bzq * SPB, b32b = b32 + 1;      // the block's sequence; its second one (SPB > 1)
     int nseq = (SPB > 1 && b32 + 1 < a.B) ? 2 : 1;
-    int32_t L0 = 0, L1 = 0;                   // paged: their lengths
-    if constexpr (PAGED) {
-        if (SPB > 1 && a.by_len) {
-            // The bz-th longest sequence and the bz-th shortest (ties by
-            // index; a length outside [0, capacity] counts as 0): a thread
-            // per sequence counts the greater (length, index) keys.
-            static_assert(kByLenMax == 128 && kDecTileTokensMax < (1 << 25), "two keys per lane, length * 128 + index in 32 bits");
-            // (the sign table while the lengths are on their way)
-            const __amdgpu_buffer_rsrc_t LB = __builtin_amdgcn_make_buffer_rsrc((void *)a.seq_lens, (short)0, (int)a.B * 4, kBufWord3);
-            uint32_t u[2], raw[2];
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const int i = 64 * h + lane;
-                const uint32_t L = raw[h] = __builtin_amdgcn_raw_buffer_load_b32(LB, 4u * (uint32_t)i, 0, 0);
-                u[h] = i < a.B ? ((int64_t)L > a.S ? 0u : L) * 128u + (uint32_t)(127 - i) : 0u;
-            }
-            if (tid < 512) sign_table_store(smem, tid);
-            // wave w counts over the sequences w, w + 12, ...; the partial
-            // counts meet as bytes in the area of G q (not written before
-            // the next barrier)
-            unsigned char *part = smem + kDecQsOff + kDecRows * D * 4;
-            static_assert(kByLenMax * kDecWaves <= kDecRows * kDecGqStride * 4 && kDecWaves == 12, "three dwords of counts per sequence");
-            uint32_t r0 = 0, r1 = 0;
-#pragma unroll
-            for (int k = 0; k < (kByLenMax + kDecWaves - 1) / kDecWaves; ++k) {
-                const int q = wave + kDecWaves * k;
-                if (q < a.B) {                               // (wave-uniform)
-                    const uint32_t other = (uint32_t)__builtin_amdgcn_readlane(q < 64 ? u[0] : u[1], q & 63);
-                    r0 += other > u[0] ? 1u : 0u;
-                    r1 += other > u[1] ? 1u : 0u;
-                }
-            }
-            part[lane * kDecWaves + wave] = (unsigned char)r0;
-            part[(64 + lane) * kDecWaves + wave] = (unsigned char)r1;
-            __syncthreads();
-            int rank[2];
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const uint32_t *c = reinterpret_cast<const uint32_t *>(part + (64 * h + lane) * kDecWaves);
-                const int v = (int)__builtin_amdgcn_sad_u8(c[0], 0u, __builtin_amdgcn_sad_u8(c[1], 0u, __builtin_amdgcn_sad_u8(c[2], 0u, 0u)));
-                rank[h] = 64 * h + lane < a.B ? v : -1;
-            }
-            auto at = [&](int r) {
-                const uint64_t lo = __builtin_amdgcn_ballot_w64(rank[0] == r);
-                return lo ? (int)__builtin_ctzll(lo) : 64 + (int)__builtin_ctzll(__builtin_amdgcn_ballot_w64(rank[1] == r));
-            };
-            b32 = at(bz);
-            b32b = at((int)a.B - 1 - bz);
-            nseq = b32 != b32b ? 2 : 1;
-            L0 = __builtin_amdgcn_readlane(b32 < 64 ? raw[0] : raw[1], b32 & 63);
-            L1 = __builtin_amdgcn_readlane(b32b < 64 ? raw[0] : raw[1], b32b & 63);
-        } else {
-            L0 = a.seq_lens[b32];
-            if (SPB > 1 && nseq > 1) L1 = a.seq_lens[b32b];
-        }
-    }
-    const int64_t b = b32;
     const int nrows_total = (int)(a.T * a.G);
     // row slot r -> (sequence index, flat (t, head) row of that sequence, valid)
     auto row_seq = [&](int r) { return (SPB > 1 && r >= nrows_total) ? 1 : 0; };
@@ -1116,6 +1059,118 @@ __global__ __launch_bounds__(64 * kDecWaves) void attn_decode128_kernel(AttnArgs
     auto row_valid = [&](int r) {
         return SPB > 1 ? (r < 2 * nrows_total && row_seq(r) < nseq) : (rc * kDecRows + r < nrows_total);
     };
+    // this wave's query row (and its adapter and x): branch-free buffer loads
+    // (an absent input gets a zero-size descriptor and reads 0)
+    const bool q32 = a.q_dtype == OMNI_F32;
+    uint32_t q32_lo, q32_hi, q16_lo, q16_hi;
+    int32_t lora_id = -1;
+    uint32_t lora_xw[4] = {0u, 0u, 0u, 0u};
+    auto load_row = [&]() {
+        const bool ok = row_valid(wave);
+        const int rho = ok ? row_rho(wave) : 0;
+        const int64_t b_q = ok && row_seq(wave) ? b32b : b32;
+        const int t_q = div_small(rho, a.g_magic);
+        const int hq_q = hk * a.G + (rho - t_q * a.G);
+        const int esz = q32 ? 4 : 2;
+        const __amdgpu_buffer_rsrc_t QR = __builtin_amdgcn_make_buffer_rsrc(
+            (void *)(reinterpret_cast<const char *>(a.q) + ((b_q * a.Hq + hq_q) * a.T + t_q) * (int64_t)(D * esz)),
+            (short)0, D * esz, kBufWord3);
+        q32_lo = __builtin_amdgcn_raw_buffer_load_b32(QR, 4u * lane, 0, 0);
+        q32_hi = __builtin_amdgcn_raw_buffer_load_b32(QR, 4u * (64 + lane), 0, 0);
+        q16_lo = __builtin_amdgcn_raw_buffer_load_b16(QR, 2u * lane, 0, 0);
+        q16_hi = __builtin_amdgcn_raw_buffer_load_b16(QR, 2u * (64 + lane), 0, 0);
+        if constexpr (LORA) {
+            lora_id = -1;
+            if (ok && wave < kDecRows) {
+                lora_id = a.lora_idx[b_q];
+                lora_x_load(lora_xw, a, b_q, t_q, lane);
+            }
+        }
+    };
+    constexpr bool kPairs = PAGED && SPB > 1;  // the pair may be one by length
+    int32_t L0 = 0, L1 = 0;                   // paged: their lengths
+    if constexpr (kPairs) {
+        if (a.by_len) {
+            // Every length, then the neighbours' rows and the sign table
+            // while those are on their way.
+            static_assert(kByLenMax == 128, "two lengths per lane");
+            const __amdgpu_buffer_rsrc_t LB = __builtin_amdgcn_make_buffer_rsrc((void *)a.seq_lens, (short)0, (int)a.B * 4, kBufWord3);
+            uint32_t L[2];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) L[h] = __builtin_amdgcn_raw_buffer_load_b32(LB, 256u * h + 4u * lane, 0, 0);
+            load_row();
+            if (tid < 512) sign_table_store(smem, tid);
+            auto len_of = [&](int i) { return (int32_t)__builtin_amdgcn_readlane(i < 64 ? L[0] : L[1], i & 63); };
+            // Neighbours stay a pair where every two neighbours are within the
+            // tiles that the waves take at once, or all their sums are within
+            // four tiles of the first's: ranking costs a block as much as
+            // three tiles of its pair.
+            int p[2];
+            bool far = false, even = true;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int t = (int64_t)L[h] > a.S ? 0 : (int)(L[h] + kDecTile - 1) / kDecTile;       // (past B: 0)
+                p[h] = t + (int)__float_as_uint(dpp_mov<0xB1>(__uint_as_float((uint32_t)t)));          // + lane ^ 1
+                const int d = p[h] - __builtin_amdgcn_readfirstlane(p[0]);
+                far = far || p[h] > 2 * nw;
+                even = even && ((d < 4 && d > -4) || 64 * h + lane >= (int)(a.B & ~1ll));
+            }
+            const bool ranked = __builtin_amdgcn_ballot_w64(far) != 0ull && __builtin_amdgcn_ballot_w64(!even) != 0ull;
+            if (ranked) {
+                // The bz-th longest sequence and the bz-th shortest (ties by
+                // index; a length outside [0, capacity] counts as 0): wave w
+                // counts the greater (length, index) keys among the sequences
+                // w, w + 12, ...; the partial counts meet as bytes in the area
+                // of G q (not written before the next barrier)
+                static_assert(kDecTileTokensMax < (1 << 25), "length * 128 + index in 32 bits");
+                unsigned char *part = smem + kDecQsOff + kDecRows * D * 4;
+                static_assert(kByLenMax * kDecWaves <= kDecRows * kDecGqStride * 4 && kDecWaves == 12, "three dwords of counts per sequence");
+                uint32_t u[2];
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const int i = 64 * h + lane;
+                    u[h] = i < a.B ? ((int64_t)L[h] > a.S ? 0u : L[h]) * 128u + (uint32_t)(127 - i) : 0u;
+                }
+                uint32_t r0 = 0, r1 = 0;
+#pragma unroll
+                for (int k = 0; k < (kByLenMax + kDecWaves - 1) / kDecWaves; ++k) {
+                    const int q = wave + kDecWaves * k;
+                    if (q < a.B) {                               // (wave-uniform)
+                        const uint32_t other = (uint32_t)__builtin_amdgcn_readlane(q < 64 ? u[0] : u[1], q & 63);
+                        r0 += other > u[0] ? 1u : 0u;
+                        r1 += other > u[1] ? 1u : 0u;
+                    }
+                }
+                part[lane * kDecWaves + wave] = (unsigned char)r0;
+                part[(64 + lane) * kDecWaves + wave] = (unsigned char)r1;
+                __syncthreads();
+                int rank[2];
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const uint32_t *c = reinterpret_cast<const uint32_t *>(part + (64 * h + lane) * kDecWaves);
+                    const int v = (int)__builtin_amdgcn_sad_u8(c[0], 0u, __builtin_amdgcn_sad_u8(c[1], 0u, __builtin_amdgcn_sad_u8(c[2], 0u, 0u)));
+                    rank[h] = 64 * h + lane < a.B ? v : -1;
+                }
+                auto at = [&](int r) {
+                    const uint64_t lo = __builtin_amdgcn_ballot_w64(rank[0] == r);
+                    return lo ? (int)__builtin_ctzll(lo) : 64 + (int)__builtin_ctzll(__builtin_amdgcn_ballot_w64(rank[1] == r));
+                };
+                b32 = at(bz);
+                b32b = at((int)a.B - 1 - bz);
+                nseq = b32 != b32b ? 2 : 1;
+                load_row();
+            }
+            L0 = len_of(b32);
+            if (nseq > 1) L1 = len_of(b32b);
+        } else {
+            L0 = a.seq_lens[b32];
+            if (nseq > 1) L1 = a.seq_lens[b32b];
+            load_row();
+        }
+    } else if constexpr (PAGED) {
+        L0 = a.seq_lens[b32];
+    }
+    const int64_t b = b32;
 
     // ── cache stream descriptors ──────────────────────────────────────
     const int s_begin = split * (int)a.split_len;
@@ -1263,32 +1318,12 @@ __global__ __launch_bounds__(64 * kDecWaves) void attn_decode128_kernel(AttnArgs
         rb[1] = __builtin_amdgcn_readfirstlane(q.r.y);
     };
 
-    // ── prologue loads: branch-free buffer loads (an absent input gets a
-    //    zero-size descriptor and reads 0), issued before the cache
-    //    prefetch so that waiting for them does not wait for the cache ──
-    // this wave's query row
+    // ── this wave's query row, requested before the cache prefetch so that
+    //    waiting for it does not wait for the cache ───────────────────────
+    if constexpr (!kPairs) load_row();
     const bool row_ok = row_valid(wave);
     const int rho_c = row_ok ? row_rho(wave) : 0;
-    const int64_t b_q = row_ok && row_seq(wave) ? b32b : b32;
-    const int t_q = div_small(rho_c, a.g_magic);
-    const int hq_q = hk * a.G + (rho_c - t_q * a.G);
-    const bool q32 = a.q_dtype == OMNI_F32;
-    const int esz = q32 ? 4 : 2;
-    const __amdgpu_buffer_rsrc_t QR = __builtin_amdgcn_make_buffer_rsrc(
-        (void *)(reinterpret_cast<const char *>(a.q) + ((b_q * a.Hq + hq_q) * a.T + t_q) * (int64_t)(D * esz)),
-        (short)0, D * esz, kBufWord3);
-    const uint32_t q32_lo = __builtin_amdgcn_raw_buffer_load_b32(QR, 4u * lane, 0, 0);
-    const uint32_t q32_hi = __builtin_amdgcn_raw_buffer_load_b32(QR, 4u * (64 + lane), 0, 0);
-    const uint32_t q16_lo = __builtin_amdgcn_raw_buffer_load_b16(QR, 2u * lane, 0, 0);
-    const uint32_t q16_hi = __builtin_amdgcn_raw_buffer_load_b16(QR, 2u * (64 + lane), 0, 0);
-    int32_t lora_id = -1;
-    uint32_t lora_xw[4] = {0u, 0u, 0u, 0u};
-    if constexpr (LORA) {
-        if (row_ok && wave < kDecRows) {
-            lora_id = a.lora_idx[b_q];
-            lora_x_load(lora_xw, a, b_q, t_q, lane);
-        }
-    }
+    const int hq_q = hk * a.G + (rho_c - div_small(rho_c, a.g_magic) * a.G);
     // ── both ring slots in flight (tiles `wave` and `wave + nw` of the
     //    split) before the prologue's work, so the cache streams while the
     //    prologue runs.  Loads are unconditional (past the split end they
@@ -1315,7 +1350,7 @@ __global__ __launch_bounds__(64 * kDecWaves) void attn_decode128_kernel(AttnArgs
     // tiles 0 .. 2 nw - 1 are taken statically (two per wave, already in flight)
     if (tid == 0) *reinterpret_cast<int *>(smem + kDecCntOff) = 2 * nw;
     // ── sign table (threads 0..511) ───────────────────────────────────
-    if (tid < 512 && !(PAGED && SPB > 1 && a.by_len)) sign_table_store(smem, tid);
+    if (tid < 512 && !(kPairs && a.by_len)) sign_table_store(smem, tid);
     // fused LoRA with G % 4 == 0: row slots 4 k .. 4 k + 3 hold one
     // (sequence, token), so x A^T is shared: each of the four waves sums a
     // quarter of its rank components, the others read them after a barrier
@@ -3399,7 +3434,8 @@ static int attn_run(const void *q, int q_dtype, const uint8_t *k_nib, const uint
     OMNI_CHECK_ARG(S < (int64_t(1) << 25), "omni_attn: S must be < 2^25 tokens per sequence");
     OMNI_CHECK_ARG(T * (Hq / Hkv) < (int64_t(1) << 31), "omni_attn: T * (n_heads / n_kv_heads) must be < 2^31");
     OMNI_CHECK_ARG(seq_index == nullptr || n_seqs >= 1, "omni_attn: a cache index needs a pool of >= 1 sequences");
-    Plan p = make_plan(device_cus(), B, Hq, Hkv, T, S, head_dim, q_dtype == OMNI_F32, paged != nullptr, scale == 0.0f);
+    const int cus = device_cus();
+    Plan p = make_plan(cus, B, Hq, Hkv, T, S, head_dim, q_dtype == OMNI_F32, paged != nullptr, scale == 0.0f);
     OMNI_CHECK_ARG(paged == nullptr || head_dim == 128, "omni_attn_paged: needs head_dim 128");
     OMNI_CHECK_ARG(Hkv <= 65535 && ((B + p.spb - 1) / p.spb) * p.n_rchunks <= 65535 && p.splits <= 2147483647,
                    "omni_attn: grid too large (batch x row chunks must be <= 65535)");
@@ -3447,14 +3483,18 @@ static int attn_run(const void *q, int q_dtype, const uint8_t *k_nib, const uint
     a.seq_index = seq_index;
     a.n_seqs = seq_index ? n_seqs : B;
     a.spb = p.spb;
-    // Paged, two sequences per block: the longest with the shortest, longest
-    // pairs first, where a block's time is its longest pair's: 48 sequences
-    // of 200 to 3000 tokens, 8 kv heads, 40.5 us with neighbours, 31.5 by
-    // length.  Knowing the lengths before anything else costs 0.7 us a block
-    // (equal lengths of 600 tokens 28.8 -> 29.5 us, of 2050 44.0 -> 43.6 with
-    // the masks that the second sequence no longer takes), so capacities
-    // below 1536 tokens and more than 128 sequences pair neighbours.
-    a.by_len = paged != nullptr && p.spb > 1 && S >= 4 * (int64_t)kDecWaves * kDecTile && B <= kByLenMax;
+    // Paged, two sequences per block: by length where neighbours differ (the
+    // kernel reads the lengths), as a block's time is its pair's: 48 sequences
+    // of 20 to 2000 tokens, 8 kv heads, 27.5 us with neighbours, 21.7 by
+    // length.  Blocks of one length leave a partly filled last round idle, where
+    // blocks of neighbours' lengths fill in: 72 of them (288 blocks on 256 CUs)
+    // 35.8 against 37.6 us, 112 (448 blocks) 43.6 against 38.6; so by length
+    // from three quarters of a last round on.  Reading every length first costs
+    // 0.1 us (20 or 100 tokens each), so not below a capacity of 1536 tokens;
+    // more than 128 sequences pair neighbours.
+    const int64_t dec_blocks = (B + 1) / 2 * Hkv;
+    a.by_len = paged != nullptr && p.spb > 1 && S >= 4 * (int64_t)kDecWaves * kDecTile && B <= kByLenMax &&
+               (dec_blocks <= cus || 4 * ((dec_blocks - 1) % cus + 1) >= 3 * cus);
     a.page_table = paged ? paged->page_table : nullptr;
     a.seq_lens = paged ? paged->seq_lens : nullptr;
     a.max_pages = paged ? paged->max_pages : 0;

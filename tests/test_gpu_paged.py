@@ -658,7 +658,7 @@ def test_paged_pairs_by_length_variants(device, T, with_qjl, lora):
     with its sequence, not with its place in the pair), without QJL, and with
     two causal tokens per sequence (four query rows either way)."""
     from omnistack_rs.cache import PagedKVCache, paged_attention
-    B, Hkv, S, uid, ps, NL, HID = 65, 8, 1600, 3, 16, 7, 128
+    B, Hkv, S, uid, ps, NL, HID = 63, 8, 1600, 3, 16, 7, 128
     Hq = Hkv * 4 // T
     g = torch.Generator().manual_seed(640 + T)
     kn, kq, kr, vn = (t.cpu() for t in _random_cache("cpu", 8, Hkv, S, 641))
@@ -723,3 +723,85 @@ def test_rows_between_kernels_with_adapters(device, B, Hq, T, S):
             assert same, name
     bad = ids == NL
     assert torch.equal(nan, bad.view(B, 1, 1, 1).expand_as(nan))
+
+
+@pytest.mark.parametrize("B", [34, 63, 128])
+@pytest.mark.parametrize("kind", ["short", "equal", "even_pairs", "one_long", "bad"])
+def test_paged_pairs_stay_neighbours(device, B, kind):
+    """Batches whose neighbours stay pairs although the capacity allows pairs
+    by length (short sequences, equal ones, neighbours of even sums), the last
+    of an odd batch alone; one long sequence, which ranks them; lengths
+    outside the capacity beside short ones."""
+    from omnistack_rs.cache import PagedKVCache, paged_attention
+    Hq, Hkv, S, uid, ps = 16, 8, 1600, 3, 32
+    g = torch.Generator().manual_seed(660 + B)
+    kn, kq, kr, vn = (t.cpu() for t in _random_cache("cpu", 8, Hkv, S, 661))
+    cb = torch.sort(torch.randn(Hkv, 16, generator=g), dim=1).values
+    q = _data.query((B, Hq, 1, 128), seed=662)
+    cache, pt8, _ = PagedKVCache.from_contiguous(*(t.to(device) for t in (kn, kq, kr, vn)), page_size=ps)
+    src = torch.arange(B) % 8
+    lens = torch.randint(1, 380, (B,), generator=g)
+    bad = []
+    if kind == "equal":
+        lens[:] = 900
+    elif kind == "even_pairs":
+        lens[0::2] = torch.randint(1, 1500, (lens[0::2].numel(),), generator=g)
+        lens[1::2] = 1510 - lens[0::2][: lens[1::2].numel()]
+    elif kind == "one_long":
+        lens[B - 1] = S
+    elif kind == "bad":
+        bad = [0, 9, B - 1]
+        lens[0], lens[9], lens[B - 1] = -1, 0, S + 1
+    got = paged_attention(q.to(device), cache, pt8[src.to(device)].contiguous(), lens.to(torch.int32).to(device), cb.to(device),
+                          user_id=uid, validate=False).cpu()
+    assert torch.equal(torch.isnan(got).flatten(1).any(dim=1).nonzero().flatten(), torch.tensor(bad, dtype=torch.int64))
+    for b in sorted({0, 1, 8, B // 2, B - 2, B - 1, int(lens.argmin()), int(lens.argmax())} - set(bad)):
+        L, c = int(lens[b]), int(src[b])
+        want = restate.fused_attn_python(q[b:b + 1].float(), kn[c:c + 1, :, :L], kq[c:c + 1, :, :L], kr[c:c + 1, :, :L],
+                                         vn[c:c + 1, :, :L], cb, uid, 1 / math.sqrt(128), True)
+        _assert_close(got[b:b + 1], want, f"neighbours {kind} B{B} b{b} len{L}")
+
+
+@pytest.mark.parametrize("B,lo,hi", [(128, 20, 20), (64, 600, 600), (65, 20, 1000)])
+def test_paged_capacity_does_not_slow_a_step(device, B, lo, hi):
+    """A page table with room for 2048 tokens a sequence takes no longer than
+    one for 1024 over the same tokens: short or equal sequences, and more
+    pairs than CUs (where blocks of one length would leave the last round
+    nearly idle).  Pairs by length without these rules: 13, 4 and 31 % more."""
+    from omnistack_rs.cache import PagedKVAttention, PagedKVCache
+    Hkv, Hq, ps = 8, 32, 16
+    g = torch.Generator().manual_seed(670)
+    lens = torch.randint(lo, hi + 1, (B,), generator=g)
+    pages = (lens + ps - 1) // ps
+    pool = PagedKVCache(int(pages.sum()), Hkv, ps, device=device)
+    pool.k_nibbles.random_(0, 256), pool.v_nibbles.random_(0, 256), pool.k_qjl.random_(0, 256), pool.k_norms.uniform_(0, 2)
+    order = torch.randperm(int(pages.sum()), generator=g).to(torch.int32)
+    cb = torch.sort(torch.randn(Hkv, 16, generator=g), dim=1).values.to(device)
+    q = _data.query((B, Hq, 1, 128), seed=671).to(device)
+    ld = lens.to(torch.int32).to(device)
+    graphs, keep = [], []
+    for cap in (1024, 2048):
+        pt = torch.zeros(B, cap // ps, dtype=torch.int32)
+        for b, at in enumerate((pages.cumsum(0) - pages).tolist()):
+            pt[b, : int(pages[b])] = order[at: at + int(pages[b])]
+        att = PagedKVAttention(pool, cb, n_heads=Hq, batch=B, max_pages=cap // ps, user_id=3, rotate_q=True)
+        pt = pt.to(device)
+        att.run(q, pt, ld)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            for _ in range(200):
+                att.run(q, pt, ld)
+        graphs.append(graph)
+        keep.append((att, pt))
+    best = [1e9, 1e9]
+    for _ in range(8):
+        for i, graph in enumerate(graphs):
+            e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+            e[0].record()
+            graph.replay()
+            e[1].record()
+            torch.cuda.synchronize()
+            best[i] = min(best[i], e[0].elapsed_time(e[1]) * 5)
+    print(f"[paged] B{B} {lo}-{hi} tokens: {best[0]:.2f} us at 1024, {best[1]:.2f} us at 2048", flush=True)
+    assert best[1] < 1.05 * best[0]
