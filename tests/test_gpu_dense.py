@@ -190,3 +190,32 @@ def test_dense_attn_many_blocks(device):
         assert same, f"batch {b}"
     del out, v
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("D,rows,more,S", [(128, 1024, 1040, 16), (128, 1024, 1040, 64), (64, 1360, 1552, 16)])
+def test_dense_attn_few_keys_take_no_longer_than_more_rows(device, D, rows, more, S):
+    """Few keys and many rows: the launch that splits the keys (which leaves
+    most of its waves idle there) is not taken, so a call takes no longer than
+    one with a few rows more, past its rule (31, 23 and 20 % longer with it)."""
+    from omnistack_rs.attention import reference_attn
+    graphs, keep = [], []
+    for n in (rows, more):
+        q, k, v = (torch.randn(1, 8, m, D, generator=_data.gen(590)).to(device) for m in (n, S, S))
+        reference_attn(q, k, v)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            outs = [reference_attn(q, k, v) for _ in range(100)]
+        graphs.append(graph)
+        keep.append((q, k, v, outs))
+    best = [1e9, 1e9]
+    for _ in range(8):
+        for i, graph in enumerate(graphs):
+            e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+            e[0].record()
+            graph.replay()
+            e[1].record()
+            torch.cuda.synchronize()
+            best[i] = min(best[i], e[0].elapsed_time(e[1]) * 10)
+    print(f"[dense] D{D} S{S}: {rows} rows {best[0]:.2f} us, {more} rows {best[1]:.2f} us", flush=True)
+    assert best[0] < 1.1 * best[1]
