@@ -10,8 +10,9 @@
 //   alpha_s = ||e_s|| sqrt(2/pi) / D,
 // with the encoder's per-head G (seed (user % 1024) ^ h).
 //
-// Work decomposition of the generic kernel (head_dim 32 at a score scale of
-// 0; the kernels below it carry everything else).  One block streams one (batch, kv head, token split)
+// Work decomposition of the generic kernel (head_dim 32: a score scale of 0, and
+// short caches of many sequences; the kernels below it carry everything else).
+// One block streams one (batch, kv head, token split)
 // for up to 16 query rows (all GQA heads of the group for one or more query
 // tokens), so every cached byte is read once per group, not once per q head.
 // Each wave takes 16-token tiles round-robin and runs three MFMA chains
@@ -373,18 +374,20 @@ __global__ __launch_bounds__(64 * kMaxWaves) void attn_kernel(AttnArgs a) {
         const float m_new = fmaxf(m_run, mt);
         const float m_use = (m_new == -INFINITY) ? 0.0f : m_new;
         const float resc = exp2f(m_run - m_use);
-        uint32_t ph[2];
+        // P as fp16 hi + remainder (against the codebook's hi plane), as the
+        // head_dim-32 prefill kernel's token-split variant
+        float pf[4], pl[4];
         float psum = 0.0f;
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const uint16_t p0 = f32_to_f16_rne(exp2f(sc[2 * i] - m_use));
-            const uint16_t p1 = f32_to_f16_rne(exp2f(sc[2 * i + 1] - m_use));
-            psum += f16_to_f32(p0) + f16_to_f32(p1);
-            ph[i] = (uint32_t)p0 | ((uint32_t)p1 << 16);
+        for (int i = 0; i < 4; ++i) {
+            pf[i] = exp2f(sc[i] - m_use);
+            pl[i] = pf[i] - f16_to_f32(f32_to_f16_rne(pf[i]));
+            psum += f16_to_f32(f32_to_f16_rne(pf[i])) + f16_to_f32(f32_to_f16_rne(pl[i]));
         }
         l_run = __builtin_fmaf(l_run, resc, psum);
         m_run = m_new;
-        const half4_t pb = as_half4(ph[0], ph[1]);
+        const half4_t pb = as_half4(pack_h2(pf[0], pf[1]), pack_h2(pf[2], pf[3]));
+        const half4_t pbl = as_half4(pack_h2(pl[0], pl[1]), pack_h2(pl[2], pl[3]));
 #pragma unroll
         for (int k = 0; k < NBLK; ++k) o_acc[k] *= resc;
 
@@ -411,6 +414,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void attn_kernel(AttnArgs a) {
                                             __builtin_amdgcn_perm(vl[3][bb].y, vl[2][bb].y, sel));
                 o_acc[2 * bb + n] = __builtin_amdgcn_mfma_f32_16x16x16f16(ah, pb, o_acc[2 * bb + n], 0, 0, 0);
                 o_acc[2 * bb + n] = __builtin_amdgcn_mfma_f32_16x16x16f16(al, pb, o_acc[2 * bb + n], 0, 0, 0);
+                o_acc[2 * bb + n] = __builtin_amdgcn_mfma_f32_16x16x16f16(ah, pbl, o_acc[2 * bb + n], 0, 0, 0);
             }
         }
     }
@@ -3160,7 +3164,7 @@ __global__ __launch_bounds__(64 * NW) void attn_prefill32_kernel(AttnArgs a) {
 struct Plan {
     bool dec128;       // D == 128: decode kernel with 8 query rows per block
     bool prefill;      // D == 128 with many rows per kv head: prefill kernel
-    bool prefill32;    // D == 32: head_dim-32 prefill kernel
+    bool prefill32;    // D == 32: head_dim-32 prefill kernel (none of the three: the generic one)
     int ncb, tws;      // prefill kernels: 16-row column blocks per wave, log2 of the waves sharing them
     int rows, n_rchunks, splits, nw, ncopy;
     int spb;           // decode kernel: sequences sharing a block's 8 row slots
@@ -3259,7 +3263,8 @@ static Plan make_plan(int cus, int64_t B, int Hq, int Hkv, int64_t T, int64_t S,
     p.tws = 0;
     p.spb = 1;
     p.ncopy = 32;
-    if (D == 32 && zero_scale) {
+    // the generic kernel's plan
+    auto generic = [&]() {
         p.rows = kRows;
         p.n_rchunks = (int)((rows + p.rows - 1) / p.rows);
         const int64_t units = B * (int64_t)Hkv * p.n_rchunks;
@@ -3275,7 +3280,8 @@ static Plan make_plan(int cus, int64_t B, int Hq, int Hkv, int64_t T, int64_t S,
         p.ws_bytes = p.splits > 1 ? (size_t)units * p.splits * p.rows * (D + 2) * sizeof(float) : 0;
         p.ws_most = p.ws_bytes;
         return p;
-    }
+    };
+    if (D == 32 && zero_scale) return generic();
     int64_t splits = 1, units = 0;
     const size_t row_bytes = (size_t)(D + 2) * sizeof(float);
     p.ws_most = 0;
@@ -3299,6 +3305,19 @@ static Plan make_plan(int cus, int64_t B, int Hq, int Hkv, int64_t T, int64_t S,
         int64_t top;
         pcost = plan_splits(cus, punits > 0 ? punits : 1, tiles, prows, D, pfix, ptile, 1, psplits, top);
         if (top > 1) p.ws_most = (size_t)(punits * top) * prows * row_bytes;
+    }
+    // D = 32, short caches: the prefill kernel fills a CU with one block (a
+    // 64 KB table of codes for each), the generic one runs eight of a few
+    // waves, up to four with a 2 KB table.  4 rows, 2048 (sequence, kv head)
+    // pairs of 50 tokens 47.7 us against 18.0, 128 tokens 47.2 / 28.5, 160
+    // tokens 49.1 / 46.1, 176 49.8 / 52.3; 600 pairs of 160 tokens 19.1 / 15.8;
+    // 512 of 50 13.0 / 11.9, with 16 rows 13.0 / 14.1, with 32 17.3 / 14.9; 32
+    // rows, 1024 pairs of 128 tokens 33.3 / 32.3, 129 tokens 34.7 / 49.1.
+    if (D == 32 && rows <= 2 * kRows && S <= (rows <= kRows ? 10 : 8) * kTile && B * ((rows + kRows - 1) / kRows) <= 65535) {
+        const double gunits = (double)(B * (int64_t)Hkv * ((rows + kRows - 1) / kRows));
+        const double gcost = 3.0 + gunits * (0.0045 + 0.00009 * (double)S);
+        const double least = (rows <= kRows / 2 ? 11.0 : 13.5) + (S > 8 * kTile ? 2.0 : 0.0);
+        if ((gcost > least ? gcost : least) < pcost) return generic();
     }
     if (dec) {
         const int n_rchunks = (int)((rows + kDecRows - 1) / kDecRows);

@@ -693,3 +693,58 @@ def test_attn_sign_flip_past_an_aligned_address(device, D, rows):
     past = torch.cat([sign[:3], sign])[3:]
     got = [_run(device, q, kn, kq, kr, vn, cb, uid, rotate_q=True, sign_flip=s) for s in (sign, past)]
     assert past.data_ptr() % 8 and torch.equal(*got)
+
+
+@pytest.mark.parametrize("rows,S,dtype,with_qjl", [(1, 50, torch.bfloat16, True), (4, 1, torch.float16, True),
+                                                   (4, 112, torch.float32, True), (16, 17, torch.bfloat16, False),
+                                                   (17, 128, torch.bfloat16, True), (32, 64, torch.float32, True), (7, 160, torch.bfloat16, True)])
+def test_attn_head_dim_32_short_caches(device, rows, S, dtype, with_qjl):
+    """More (sequence, kv head) pairs than four blocks a CU and short caches:
+    the generic kernel, with the causal window that the rows leave and
+    in-kernel rotation, against 64 bits.  P keeps its fp16 remainder and every
+    product its operands' (22 bits), as on the kernel for longer caches."""
+    B, Hkv, uid, D = 150, 8, 5, 32
+    kn, kq, kr, vn, cb = _random_packed(B, Hkv, S, D, seed=730 + S)
+    q = torch.randn(B, Hkv, rows, D, generator=_data.gen(731)).to(dtype)
+    sign = _data.sign_flip(D)
+    off = max(S - rows, 0)
+    got = _run(device, q, kn, kq, kr, vn, cb, uid, with_qjl, causal_offset=off, rotate_q=True, sign_flip=sign.to(device)).cpu()
+    assert torch.isfinite(got).all()
+    sl = slice(0, B, 37)
+    k = restate.dequantize_heads(kn[sl], kq[sl], kr[sl], cb, user_id=uid, with_qjl=with_qjl)
+    v = restate.dequantize_heads(vn[sl], kq[sl], kr[sl], cb, user_id=uid, with_qjl=False)
+    want = exact.attention(restate.rotate(q[sl], sign).float(), k, v, 1 / math.sqrt(D), mask=_causal_mask(rows, S, off))
+    err = (got[sl].double() - want).norm() / want.norm()
+    print(f"[attn] short head_dim 32, {rows} rows, {S} tokens: relative error {err:.2e}", flush=True)
+    assert err <= 4e-6                        # 22-bit operands, fp32 sums over at most 160 keys and 32 elements
+
+
+def test_attn_head_dim_32_short_caches_take_a_fraction(device):
+    """256 sequences of 50 tokens, 8 kv heads, head_dim 32: a third of the time
+    of 300 tokens (nine tenths where each pair takes a CU with the prefill
+    kernel's tables)."""
+    from omnistack_rs.kernels.fused_attention import PackedKVAttention
+    B, Hkv, G, D = 256, 8, 4, 32
+    graphs, keep, best = [], [], [1e9, 1e9]
+    for S in (50, 300):
+        kn, kq, kr, vn, cb = (t.to(device) for t in _random_packed(B, Hkv, S, D, seed=740))
+        att = PackedKVAttention(kn, kq, kr, vn, cb, n_heads=Hkv * G, user_id=3)
+        q = _data.query((B, Hkv * G, 1, D), seed=741).to(device)
+        att.run(q)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            for _ in range(50):
+                att.run(q)
+        graphs.append(graph)
+        keep.append((att, q))
+    for _ in range(5):
+        for i, graph in enumerate(graphs):
+            e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+            e[0].record()
+            graph.replay()
+            e[1].record()
+            torch.cuda.synchronize()
+            best[i] = min(best[i], e[0].elapsed_time(e[1]) * 20)
+    print(f"[attn] head_dim 32, 2048 pairs: 50 tokens {best[0]:.1f} us, 300 tokens {best[1]:.1f} us", flush=True)
+    assert best[0] < 0.6 * best[1]
