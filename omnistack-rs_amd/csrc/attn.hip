@@ -3180,13 +3180,21 @@ constexpr size_t kScratchBytes = size_t(16) << 20;
 
 // Splits of each unit's `tiles` key tiles, one block per CU at a time, and
 // the call's estimated time in us: rounds of blocks x (a block's fixed part +
-// its tiles) + the combine launch and the partials' way through memory.  The
-// fixed part and the time per tile are measured; the rounds decide: 24 units
+// its tiles) + the combine launch, which reads its splits eight at a time, and
+// the partials' way through memory.  The fixed part and the time per tile are
+// measured; a contiguous decode tile takes `alone` of its time on an idle chip
+// (0.11 us of 0.19) and all of it with a block on every CU.  The rounds decide: 24 units
 // in 11 splits are 264 blocks on 256 CUs, twice the time of 10 splits (decode
-// of 3 x 20011 tokens, 8 rows: 54.5 us so, 23.6 us in 10 splits with the wider
-// combine).  Candidates: no split, and the most that 1, 2 or 3 full rounds
-// hold with at least kMinSplitTiles tiles each; a split has to promise a
-// tenth (a second, partly filled round runs faster than a full one).
+// of 3 x 20011 tokens, 8 rows: 54.5 us so, 23.6 us in 10 splits).  Candidates:
+// no split, the most that 1, 2 or 3 full rounds hold with at least
+// kMinSplitTiles tiles each, and a half, quarter and eighth of one round's: a
+// decode of 20000 tokens by one pair took 19.7 us in 8 splits, 16.6 in 16, 16.9
+// in 32, 21.9 in 64 and 32.6 in 128.  A split has to promise a tenth (a second,
+// partly filled round runs faster than a full one).
+// Paged sequences end anywhere in their capacity, and splits past their end
+// have nothing to do: there the merge counts as kSplitGainUs at least (capacity
+// 2048, 66 pairs of 24 to 48 tokens: 7.8 us unsplit, 11.2 in three splits), and
+// `quarter` is the time with tables a quarter full.
 // `top`: at least the splits of any shorter sequence, and no fewer for a longer
 // one (rounds and kernels change with the length, so the splits themselves can
 // drop as it grows): a workspace made for the longest cache serves every shorter.
@@ -3194,17 +3202,19 @@ constexpr size_t kScratchBytes = size_t(16) << 20;
 // they never win (what rounding up a split's tiles can gain is less than a
 // round's fixed part).
 constexpr int64_t kMinSplitTiles = 4;
-constexpr double kCombineUs = 6.0;
+constexpr double kSplitGainUs = 6.0;                  // a call this much above a block's fixed part may gain from a split
+constexpr double kCombineUs = 1.6, kCombineSplitUs = 0.165;
 constexpr double kPartialUsPerByte = 2.0 / 3.5e6;     // written and read, 3.5 TB/s
 
-static double plan_splits(int64_t cus, int64_t units, int64_t tiles, int rows, int D, double fixed, double per_tile, int64_t least,
-                          int64_t &splits, int64_t &top) {
+static double plan_splits(int64_t cus, int64_t units, int64_t tiles, int rows, int D, double fixed, double per_tile, double alone,
+                          bool paged, int64_t least, int64_t &splits, int64_t &top, double &quarter) {
     const int64_t most = tiles / kMinSplitTiles > 1 ? tiles / kMinSplitTiles : 1;
     const double whole = (double)((units + cus - 1) / cus) * (fixed + per_tile * (double)tiles);
-    // a short sequence, planned on every small call: too few tiles, or no time
-    // for a split block and the combine launch within nine tenths of `whole`
-    if (least <= 1 && (most == 1 || 0.9 * whole <= fixed + kCombineUs)) {
+    // a short sequence, planned on every small call: too few tiles, or too
+    // little time to gain from a split
+    if (least <= 1 && (most == 1 || 0.9 * whole <= fixed + kSplitGainUs)) {
         splits = top = 1;
+        quarter = (double)((units + cus - 1) / cus) * (fixed + per_tile * 0.25 * (double)tiles);
         return whole;
     }
     const size_t unit_bytes = (size_t)rows * (D + 2) * sizeof(float);
@@ -3215,24 +3225,37 @@ static double plan_splits(int64_t cus, int64_t units, int64_t tiles, int rows, i
     const int64_t cap = fit > plain ? fit : plain;
     double best = 0.0;
     splits = 0;
-    top = least > 1 ? least : 1;
-    int64_t top_full = 1, top_rounds = (units + cus - 1) / cus;
-    for (int r = 0; r <= 3; ++r) {
-        const int64_t full = r * cus / units > 1 ? r * cus / units : 1, full_rounds = (units * full + cus - 1) / cus;
-        int64_t s = clamp64(full, 1, most < cap ? most : cap);
+    auto consider = [&](int64_t s) {
         if (s < least) s = least;
+        const int64_t blocks = units * s;
+        const double load = blocks < cus ? (double)blocks / (double)cus : 1.0;
+        const double rounds = (double)((blocks + cus - 1) / cus), tile = per_tile * (alone + (1.0 - alone) * load);
+        double t = rounds * (fixed + tile * (double)((tiles + s - 1) / s)), merge = 0.0;
+        if (s > 1) {
+            merge = kCombineUs + kCombineSplitUs * (double)s;
+            if (paged && merge < kSplitGainUs) merge = kSplitGainUs;
+            merge += (double)(unit_bytes * (size_t)blocks) * kPartialUsPerByte;
+            t += merge;
+        }
+        if (splits == 0 || t < (splits == 1 ? 0.9 * best : best)) {
+            best = t;
+            splits = s;
+            quarter = rounds * (fixed + tile * (double)(s > 4 ? (tiles + s - 1) / s : (tiles + 3) / 4)) + merge;
+        }
+        return s;
+    };
+    top = consider(1);
+    int64_t top_full = 1, top_rounds = (units + cus - 1) / cus;
+    for (int r = 1; r <= 3; ++r) {
+        const int64_t full = r * cus / units > 1 ? r * cus / units : 1, full_rounds = (units * full + cus - 1) / cus;
+        const int64_t s = consider(clamp64(full, 1, most < cap ? most : cap));
         if (full * top_rounds > top_full * full_rounds) {
             top_full = full;
             top_rounds = full_rounds;
             if (s > top) top = s;
         }
-        const double rounds = (double)((units * s + cus - 1) / cus);
-        double t = rounds * (fixed + per_tile * (double)((tiles + s - 1) / s));
-        if (s > 1) t += kCombineUs + (double)(unit_bytes * (size_t)(units * s)) * kPartialUsPerByte;
-        if (splits == 0 || t < (splits == 1 ? 0.9 * best : best)) {
-            best = t;
-            splits = s;
-        }
+        if (r == 1)
+            for (int64_t k = s / 2; k >= 2 && k >= s / 8; k /= 2) consider(k);
     }
     return best;
 }
@@ -3251,7 +3274,10 @@ static double plan_splits(int64_t cus, int64_t units, int64_t tiles, int rows, i
 // blocks decode the same cache at the same time, or one prefill block: the
 // smaller estimate.  (Decode holds while its blocks fit the chip at once: 24
 // rows, 8 sequences of 100 tokens 7.7 against 15 us; the prefill kernel where
-// they do not: 32 sequences of 4096 tokens 85 against 54 us.)
+// they do not: 32 sequences of 4096 tokens 85 against 54 us.)  Paged: by the
+// geometric mean of full tables and tables a quarter full (8 sequences of 32
+// rows, capacity 8192: decode 18.8 us at 2000 tokens and 47.5 at 8192, the
+// prefill kernel, one of whose four splits holds the 2000, 36.2 and 37.6).
 static Plan make_plan(int cus, int64_t B, int Hq, int Hkv, int64_t T, int64_t S, int D, bool q32, bool paged = false,
                       bool zero_scale = false) {
     Plan p;
@@ -3300,10 +3326,10 @@ static Plan make_plan(int cus, int64_t B, int Hq, int Hkv, int64_t T, int64_t S,
     const double ptile = (D == 128 ? (ncb == 1 ? 1.9 : 2.3) : (ncb == 1 ? 0.6 : (ncb == 2 ? 0.8 : 1.3))) / (1 << tws);
     const bool dec = D == 128 && rows <= kDecMaxRows && !zero_scale;      // the decode kernel can take it
     int64_t psplits = 1;
-    double pcost = 0.0;
+    double pcost = 0.0, pquarter = 0.0;
     if (!dec || rows > kDecRows) {
         int64_t top;
-        pcost = plan_splits(cus, punits > 0 ? punits : 1, tiles, prows, D, pfix, ptile, 1, psplits, top);
+        pcost = plan_splits(cus, punits > 0 ? punits : 1, tiles, prows, D, pfix, ptile, 1.0, paged, 1, psplits, top, pquarter);
         if (top > 1) p.ws_most = (size_t)(punits * top) * prows * row_bytes;
     }
     // D = 32, short caches: the prefill kernel fills a CU with one block (a
@@ -3331,14 +3357,14 @@ static Plan make_plan(int cus, int64_t B, int Hq, int Hkv, int64_t T, int64_t S,
         const int64_t cap = kDecPtMax / 2;
         const int64_t least = (paged && spb == 1 && tiles > cap) ? (tiles + cap - 1) / cap : 1;
         int64_t dsplits = 1;
-        double dcost = 0.0;
+        double dcost = 0.0, dquarter = 0.0;
         if (spb == 1) {
             int64_t top;
-            dcost = plan_splits(cus, dunits > 0 ? dunits : 1, tiles, kDecRows, D, 6.5, 0.19, least, dsplits, top);
+            dcost = plan_splits(cus, dunits > 0 ? dunits : 1, tiles, kDecRows, D, 6.5, 0.19, paged ? 1.0 : 0.6, paged, least, dsplits, top, dquarter);
             const size_t most = top > 1 ? (size_t)(dunits * top) * kDecRows * row_bytes : 0;
             if (most > p.ws_most) p.ws_most = most;
         }
-        if (rows <= kDecRows || dcost <= 1.1 * pcost) {
+        if (rows <= kDecRows || (paged ? dcost * dquarter <= 1.21 * pcost * pquarter : dcost <= 1.1 * pcost)) {
             p.dec128 = true;
             p.rows = kDecRows;
             p.n_rchunks = n_rchunks;

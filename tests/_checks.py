@@ -53,3 +53,27 @@ def check_encode(x_rot_cpu, cb_cpu, user_id, nib, qjl, nrm, tag=""):
         slack = exact.ulp_distance_f32(r_h, en32[fin]) + 1
         assert (exact.ulp_distance_f32(gn[fin], r_h) <= slack).all(), f"{tag}: norm vs oracle"
     return n_mis_oracle
+
+
+def graph_times(calls, n, reps=6):
+    """Time in us of each call (least of `reps` replays of a graph of `n` of
+    it, the calls' replays in turn); GPU side."""
+    graphs = []
+    for call in calls:
+        call()
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            for _ in range(n):
+                call()
+        graphs.append(graph)
+    best = [float("inf")] * len(graphs)
+    for _ in range(reps):
+        for i, graph in enumerate(graphs):
+            e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+            e[0].record()
+            graph.replay()
+            e[1].record()
+            torch.cuda.synchronize()
+            best[i] = min(best[i], e[0].elapsed_time(e[1]) * 1e3 / n)
+    return best

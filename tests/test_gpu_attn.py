@@ -17,6 +17,7 @@ import torch
 
 from oracle import exact, restate
 from tests import _data
+from tests._checks import graph_times
 
 pytestmark = pytest.mark.gpu
 
@@ -725,26 +726,22 @@ def test_attn_head_dim_32_short_caches_take_a_fraction(device):
     kernel's tables)."""
     from omnistack_rs.kernels.fused_attention import PackedKVAttention
     B, Hkv, G, D = 256, 8, 4, 32
-    graphs, keep, best = [], [], [1e9, 1e9]
-    for S in (50, 300):
-        kn, kq, kr, vn, cb = (t.to(device) for t in _random_packed(B, Hkv, S, D, seed=740))
-        att = PackedKVAttention(kn, kq, kr, vn, cb, n_heads=Hkv * G, user_id=3)
-        q = _data.query((B, Hkv * G, 1, D), seed=741).to(device)
-        att.run(q)
-        torch.cuda.synchronize()
-        graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(graph):
-            for _ in range(50):
-                att.run(q)
-        graphs.append(graph)
-        keep.append((att, q))
-    for _ in range(5):
-        for i, graph in enumerate(graphs):
-            e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
-            e[0].record()
-            graph.replay()
-            e[1].record()
-            torch.cuda.synchronize()
-            best[i] = min(best[i], e[0].elapsed_time(e[1]) * 20)
+    q = _data.query((B, Hkv * G, 1, D), seed=741).to(device)
+    atts = [PackedKVAttention(*(t.to(device) for t in _random_packed(B, Hkv, S, D, seed=740)), n_heads=Hkv * G, user_id=3)
+            for S in (50, 300)]
+    best = graph_times([lambda a=a: a.run(q) for a in atts], 50)
     print(f"[attn] head_dim 32, 2048 pairs: 50 tokens {best[0]:.1f} us, 300 tokens {best[1]:.1f} us", flush=True)
     assert best[0] < 0.6 * best[1]
+
+
+@pytest.mark.parametrize("Hkv", [1, 2, 8])
+def test_attn_long_cache_of_few_pairs(device, Hkv):
+    """One sequence: 20000 tokens take less than 1.7 times as long as 5000 (a
+    split per free CU took 2.1 times, most of it in the merge of 128 splits)."""
+    from omnistack_rs.kernels.fused_attention import PackedKVAttention
+    q = _data.query((1, Hkv, 1, 128), seed=751).to(device)
+    atts = [PackedKVAttention(*(t.to(device) for t in _random_packed(1, Hkv, S, 128, seed=750)), n_heads=Hkv, user_id=3)
+            for S in (5000, 20000)]
+    best = graph_times([lambda a=a: a.run(q) for a in atts], 100)
+    print(f"[attn] {Hkv} pairs: 5000 tokens {best[0]:.1f} us, 20000 tokens {best[1]:.1f} us", flush=True)
+    assert best[1] < 1.7 * best[0]

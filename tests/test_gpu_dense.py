@@ -15,6 +15,7 @@ import torch
 
 from oracle import restate
 from tests import _data
+from tests._checks import graph_times
 
 pytestmark = pytest.mark.gpu
 
@@ -198,24 +199,7 @@ def test_dense_attn_few_keys_take_no_longer_than_more_rows(device, D, rows, more
     most of its waves idle there) is not taken, so a call takes no longer than
     one with a few rows more, past its rule (31, 23 and 20 % longer with it)."""
     from omnistack_rs.attention import reference_attn
-    graphs, keep = [], []
-    for n in (rows, more):
-        q, k, v = (torch.randn(1, 8, m, D, generator=_data.gen(590)).to(device) for m in (n, S, S))
-        reference_attn(q, k, v)
-        torch.cuda.synchronize()
-        graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(graph):
-            outs = [reference_attn(q, k, v) for _ in range(100)]
-        graphs.append(graph)
-        keep.append((q, k, v, outs))
-    best = [1e9, 1e9]
-    for _ in range(8):
-        for i, graph in enumerate(graphs):
-            e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
-            e[0].record()
-            graph.replay()
-            e[1].record()
-            torch.cuda.synchronize()
-            best[i] = min(best[i], e[0].elapsed_time(e[1]) * 10)
+    ts = [[torch.randn(1, 8, m, D, generator=_data.gen(590)).to(device) for m in (n, S, S)] for n in (rows, more)]
+    best = graph_times([lambda t=t: reference_attn(*t) for t in ts], 100)
     print(f"[dense] D{D} S{S}: {rows} rows {best[0]:.2f} us, {more} rows {best[1]:.2f} us", flush=True)
     assert best[0] < 1.1 * best[1]
