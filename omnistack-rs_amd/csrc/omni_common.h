@@ -84,16 +84,6 @@ __device__ __forceinline__ float round_to_dtype(float v, int dtype) {
     return v;
 }
 
-__device__ __forceinline__ void store_from_f32(void *p, int dtype, int64_t i, float v) {
-    if (dtype == OMNI_F32) {
-        reinterpret_cast<float *>(p)[i] = v;
-    } else if (dtype == OMNI_BF16) {
-        reinterpret_cast<uint16_t *>(p)[i] = f32_to_bf16_rne(v);
-    } else {
-        reinterpret_cast<uint16_t *>(p)[i] = f32_to_f16_rne(v);
-    }
-}
-
 // (a, b) <- butterfly with the partner lane across bit 4 (row parity) or 5
 // (half): lanes with the bit clear hold the lower element of each pair.
 // Two swaps and one add/sub pair cover two elements.

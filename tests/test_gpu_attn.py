@@ -1,6 +1,6 @@
 """GPU parity of compressed-KV attention (omni_attn) against the CPU oracle.
 
-Bar (north star): max-abs <= 2e-3 and mean-abs <= 2e-4 against the
+Bar: max-abs <= 2e-3 and mean-abs <= 2e-4 against the
 reference's own CPU path (_fused_attn_python restated in oracle.restate),
 on identical packed inputs.  The reference's CPU path returns q's dtype
 (reference_attn casts its fp32 result back, attention/reference.py:177)

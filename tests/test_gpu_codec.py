@@ -135,7 +135,7 @@ def test_encode_c4_full_size(device):
 def test_prepared_encoder_pair_equals_encode_kv(device, B, T, dtype, D):
     """PackedKVEncoder: K and V in one launch with code tables built once give
     exactly what two encode_kv calls give (the wave kernel for 16-bit inputs
-    at D = 128 and B * T >= 64, the lane-per-row kernel otherwise), and
+    at D = 128 and B * T >= 64, encode_grid_kernel otherwise), and
     writing into preallocated outputs changes nothing; rotate=False equals
     quantize_heads."""
     from omnistack_rs.kernels.quantize import PackedKVEncoder, encode_kv, quantize_heads
@@ -431,7 +431,7 @@ def test_fast_encoder_rows_straddle_sequences(device, dtype):
 
 
 def test_fast_encoder_matches_row_kernel(device):
-    """The wave encoder and the lane-per-row encoder agree bit for bit on the
+    """encode128_kernel and encode_grid_kernel agree bit for bit on the
     same rows (a head with >= 64 rows vs the same rows fed one head at a time)."""
     from omnistack_rs.kernels.quantize import quantize_heads
     x = restate.wht(_data.kv((1, 1, 64, 128), seed=34, dtype=torch.float32)).to(torch.bfloat16)
