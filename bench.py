@@ -309,6 +309,26 @@ def cpu_model() -> str:
     return f"{name} ({fam}{os.cpu_count()} logical CPUs visible)"
 
 
+def without_gc(f):
+    """`f` with Python's cyclic collector off: a full collection walks every
+    object of torch (30-50 ms), and one inside a window of ten calls of 170 us
+    is read as 3-5 ms a call."""
+    import functools
+    import gc
+
+    @functools.wraps(f)
+    def run(*args, **kw):
+        was = gc.isenabled()
+        gc.disable()
+        try:
+            return f(*args, **kw)
+        finally:
+            if was:
+                gc.enable()
+    return run
+
+
+@without_gc
 def timed_region(fn, steps, warmup, stream):
     """`warmup` untimed calls, then exactly `steps` back-to-back calls between
     two synchronizations, bracketed by HIP events on the launch stream.
@@ -328,6 +348,7 @@ def timed_region(fn, steps, warmup, stream):
     return wall / steps, e0.elapsed_time(e1) * 1e-3 / steps
 
 
+@without_gc
 def sustained_blocks(fn, calls, block, stream):
     """`calls` back-to-back calls with a HIP event on the launch stream every
     `block` calls; returns the mean duration per call of each block (s)."""
@@ -344,6 +365,7 @@ def sustained_blocks(fn, calls, block, stream):
     return [evs[i].elapsed_time(evs[i + 1]) * 1e-3 / block for i in range(nb)]
 
 
+@without_gc
 def per_call_events(fn, steps, warmup, stream):
     """Eager calls, each bracketed by HIP events on the launch stream; returns
     the per-call device durations (s)."""
@@ -360,6 +382,7 @@ def per_call_events(fn, steps, warmup, stream):
     return [s.elapsed_time(e) * 1e-3 for s, e in evs]
 
 
+@without_gc
 def wall_eager(fn, steps, warmup):
     """Wall time per call over `steps` back-to-back eager calls (synchronized
     on both sides, no per-call events)."""
@@ -374,6 +397,7 @@ def wall_eager(fn, steps, warmup):
     return (time.perf_counter() - t0) / steps
 
 
+@without_gc
 def wall_graph(fn, steps, warmup):
     """The `steps` calls captured once as a HIP graph (every call reads inputs
     already in HBM and enqueues its kernels; no allocation or memset inside),
