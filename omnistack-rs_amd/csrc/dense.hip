@@ -204,7 +204,7 @@ __device__ __forceinline__ uint32_t dn_abs_max(uint32_t m, float4 v) {
 
 // Bound by the fp32 matrix rate: 2 x 1000 queries, 32 heads over 8, 1000 keys,
 // head_dim 128, 293 us without a mask (112 of the 154 TFLOP/s that a large
-// product reaches) and 224 us causal, where half of the tiles are hidden and
+// product reaches) and 220 us causal, where half of the tiles are hidden and
 // skipped; with row-major scores, whose maxima and sums were 16-lane
 // shuffles, and P through LDS 485 and 537 us.  Registers for three waves per
 // SIMD: two of them 369 us.
@@ -244,14 +244,15 @@ __global__ __launch_bounds__(64 * kDnWaves, D == 256 ? 1 : (D == 128 ? 3 : 4)) v
     float mk[2][4] = {};
     auto fetch = [&](int64_t s0) {
         // the tile's keys below S as buffers: lanes past them read 0 (the
-        // whole offset is the lane's: the scalar one is not range-checked)
+        // whole offset is the lane's and the instruction's: the scalar one is
+        // not range-checked); a wave's loads are consecutive KB
         const int bytes = (int)(s0 + kDnKeys <= a.S ? kDnKeys : a.S - s0) * D * 4;
         const __amdgpu_buffer_rsrc_t K = __builtin_amdgcn_make_buffer_rsrc((void *)(kb0 + s0 * D), (short)0, bytes, kDnBufWord3);
         const __amdgpu_buffer_rsrc_t V = __builtin_amdgcn_make_buffer_rsrc((void *)(vb0 + s0 * D), (short)0, bytes, kDnBufWord3);
 #pragma unroll
         for (int c = 0; c < kPer; ++c) {
-            nk[c] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(K, 16 * tid + c * 1024 * kDnWaves, 0, 0));
-            nv[c] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(V, 16 * tid + c * 1024 * kDnWaves, 0, 0));
+            nk[c] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(K, 16 * lane + 1024 * (kPer * wave + c), 0, 0));
+            nv[c] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(V, 16 * lane + 1024 * (kPer * wave + c), 0, 0));
         }
     };
     if (a.S > 0) fetch(0);
@@ -265,7 +266,7 @@ __global__ __launch_bounds__(64 * kDnWaves, D == 256 ? 1 : (D == 128 ? 3 : 4)) v
         uint32_t km = 0, vm = 0;
 #pragma unroll
         for (int c = 0; c < kPer; ++c) {
-            const int e = 4 * (tid + c * 64 * kDnWaves);
+            const int e = 4 * (lane + 64 * (kPer * wave + c));
             const int key = e / D, d = e - key * D;
             *reinterpret_cast<float4 *>(ks + key * DP + d) = nk[c];
             *reinterpret_cast<float4 *>(vs + key * DP + d) = nv[c];
