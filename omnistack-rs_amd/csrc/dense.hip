@@ -525,13 +525,14 @@ extern "C" int omni_dense_attn(const float *q, const float *k, const float *v, c
     // for a chip full; while its 64-row blocks leave CUs idle, blocks of 16
     // rows whose waves split the keys are faster.  Up to two of those per CU
     // (head_dim 128: one runs at a time), three at smaller head_dims, and one
-    // less where few keys leave most of their waves idle.  32 heads over 8, 700 keys,
-    // causal, row kernel against key kernel: head_dim 128, 120 queries 71.5 /
-    // 30.7 us, 200 71.9 / 57.3, 350 75.9 / 82.9; head_dim 64, 200 47.2 / 31.1,
-    // 350 50.9 / 45.6, 700 x 2 69.6 / 161.  Head_dim 128, 512 groups of 16
-    // rows: 16 keys 12.5 / 16.4, 64 keys 18.0 / 22.2; head_dim 64, 680 groups, 16
-    // keys 9.0 / 10.8.
-    const int64_t per_cu = head_dim == 128 ? (S > 64 ? 2 : 1) : (S > 32 ? 3 : 2);
+    // less where few keys leave most of their waves idle.  32 heads over 8, 700
+    // keys, causal, row kernel against key kernel: head_dim 128, 120 queries
+    // 71.5 / 30.7 us, 200 71.9 / 57.3, 350 75.9 / 82.9; head_dim 64, 200 47.2 /
+    // 31.1, 700 x 2 69.6 / 161.  Few keys: head_dim 128, 512 groups of 16 rows,
+    // 16 keys 12.5 / 16.4, 64 18.0 / 22.2; head_dim 64, 680 groups, causal, 128
+    // keys 12.3 / 24.1, 600 42.5 / 44.5, 700 49.5 / 45.9; head_dim 32, 200 keys
+    // 14.7 / 16.2, 300 18.5 / 16.0.
+    const int64_t per_cu = head_dim == 128 ? (S > 64 ? 2 : 1) : (S > (head_dim == 64 ? 600 : 200) ? 3 : 2);
     if ((rows <= 16 || groups <= per_cu * device_cus()) && head_dim <= 128 &&
         S < (int64_t(1) << 27)) {
         // few rows: the waves split the keys instead of the rows
