@@ -203,7 +203,7 @@ __device__ __forceinline__ uint32_t dn_abs_max(uint32_t m, float4 v) {
 }
 
 // Bound by the fp32 matrix rate: 2 x 1000 queries, 32 heads over 8, 1000 keys,
-// head_dim 128, 293 us without a mask (112 of the 154 TFLOP/s that a large
+// head_dim 128, 294 us without a mask (111 of the 154 TFLOP/s that a large
 // product reaches) and 220 us causal, where half of the tiles are hidden and
 // skipped; with row-major scores, whose maxima and sums were 16-lane
 // shuffles, and P through LDS 485 and 537 us.  Registers for three waves per
